@@ -28,10 +28,14 @@ constexpr int kTraceBlock = 128;
 // The occupancy knob's "no limit" (the registers then allow what they allow).
 constexpr int kTraceMaxWavesPerSimd = 8;
 constexpr int kStack = 128;
-// Stack entries below this depth live in LDS (12 bytes each: 9 KB per
-// workgroup, so the registers, not LDS, limit the waves per CU); deeper ones
-// in the private array.
-constexpr int kStackLds = 6;
+// Stack entries kept in LDS (12 bytes each; a power of two, a ring): 12 KB
+// per workgroup.  2,073,600 primary / 148,743 bounce rays on the clustered 1M
+// scene with rings of 4, 8 and 16 entries: 525 / 447, 518 / 420 and 675 / 417
+// us (16 leave three waves per SIMD).
+constexpr int kStackLds = 8;
+// s_waitcnt operand: no vector memory operation outstanding (vmcnt 0, other
+// counters at their maximum).
+constexpr int kWaitVmem0 = 0x0F70;
 
 struct Ray
 {
@@ -71,9 +75,27 @@ struct Tri
   float p0[3], e0[3], e1[3], nrm[3];
 };
 
-// triangle_intersector (lbvh.h:2055-2075): two-sided, not watertight.
+// The closest hit so far.
+struct Hit
+{
+  uint32_t prim = 0xffffffffu;
+  float t = INFINITY, u = 0.0f, v = 0.0f;
+};
+
+// Whether a hit at distance t of primitive id replaces the closest so far.
+template<int MODE>
 __device__ __forceinline__ bool
-isect_reference(const Tri& tr, const Ray& r, float& t_out, float& u_out, float& v_out)
+better(float t, uint32_t id, const Hit& h)
+{
+  if (MODE == 0)
+    return t < h.t;
+  return (t < h.t) || (t == h.t && id < h.prim && t != INFINITY);
+}
+
+// triangle_intersector (lbvh.h:2055-2075): two-sided, not watertight.
+template<int MODE>
+__device__ __forceinline__ void
+isect_reference(const Tri& tr, uint32_t id, const Ray& r, Hit& h)
 {
   float c[3] = { tr.p0[0] - r.o[0], tr.p0[1] - r.o[1], tr.p0[2] - r.o[2] };
   float rr[3];
@@ -84,20 +106,20 @@ isect_reference(const Tri& tr, const Ray& r, float& t_out, float& u_out, float& 
   float w = (1.0f - u) - v;
   if ((u >= 0.0f) && (v >= 0.0f) && (w >= 0.0f)) {
     float t = dot3(tr.nrm, c) * inv_det;
-    if ((t >= r.tmin) && (t <= r.tmax)) {
-      t_out = t;
-      u_out = u;
-      v_out = v;
-      return true;
+    if ((t >= r.tmin) && (t <= r.tmax) && better<MODE>(t, id, h)) {
+      h.prim = id;
+      h.t = t;
+      h.u = u;
+      h.v = v;
     }
   }
-  return false;
 }
 
 // Watertight test (Woop, Benthin, Wald, JCGT 2(1) 2013) on A = p0,
 // B = p0 - e0, C = p0 + e1; u, v are the weights of B and C.
-__device__ __forceinline__ bool
-isect_watertight(const Tri& tr, const Ray& r, float& t_out, float& u_out, float& v_out)
+template<int MODE>
+__device__ __forceinline__ void
+isect_watertight(const Tri& tr, uint32_t id, const Ray& r, Hit& h)
 {
   float ax = fabsf(r.d[0]), ay = fabsf(r.d[1]), az = fabsf(r.d[2]);
   int kz = (ax > ay) ? ((ax > az) ? 0 : 2) : ((ay > az) ? 1 : 2);
@@ -140,32 +162,23 @@ isect_watertight(const Tri& tr, const Ray& r, float& t_out, float& u_out, float&
   float bay = Bx * Ay, bya = By * Ax;
   float W = bay - bya;
   if ((U < 0.0f || V < 0.0f || W < 0.0f) && (U > 0.0f || V > 0.0f || W > 0.0f))
-    return false;
+    return;
   float det = U + V;
   det = det + W;
   if (det == 0.0f)
-    return false;
+    return;
   float Az = Sz * az_, Bz = Sz * bz_, Cz = Sz * cz_;
   float ua = U * Az, vb2 = V * Bz, wc = W * Cz;
   float T = ua + vb2;
   T = T + wc;
   float rcp = 1.0f / det;
   float t = T * rcp;
-  if (!(t >= r.tmin && t <= r.tmax))
-    return false;
-  t_out = t;
-  u_out = V * rcp;
-  v_out = W * rcp;
-  return true;
-}
-
-template<int MODE>
-__device__ __forceinline__ bool
-better(float t, uint32_t id, float best_t, uint32_t best_id)
-{
-  if (MODE == 0)
-    return t < best_t;
-  return (t < best_t) || (t == best_t && id < best_id && t != INFINITY);
+  if (!(t >= r.tmin && t <= r.tmax && better<MODE>(t, id, h)))
+    return;
+  h.prim = id;
+  h.t = t;
+  h.u = V * rcp;
+  h.v = W * rcp;
 }
 
 // Ray layouts: kLayoutSingle, one tree; kLayoutBatch, a scene batch (ray i
@@ -195,6 +208,15 @@ job_of(const TraceJob* __restrict__ jobs, uint32_t njobs, uint64_t i)
 // order (single layout only, may be null): ray k of the launch is ray
 // order[k] of the input, and its hit is written there; a permutation that
 // puts rays which visit the same nodes into the same wave.
+//
+// Bound by instruction issue (a vector instruction takes a SIMD four cycles
+// for its 64 rays) and by the dependent fetch of each visit.  So a visit has
+// no branch around loads, box tests or addresses (157 instead of 250 vector
+// instructions), and a ray drops its pruned entries in a loop of its own
+// instead of one per visit of its wave.  Clustered 1M scene, 2,073,600
+// primary / 148,743 bounce rays: 621 / 546 us with branches per child, a trip
+// per pruned entry and an LDS stack of the 6 entries nearest the root, 518 /
+// 420 us so.
 template<int MODE, int LAYOUT>
 __global__ __launch_bounds__(kTraceBlock) void
 k_trace(const Node* __restrict__ nodes, const float* __restrict__ tris, uint32_t nprims,
@@ -298,121 +320,102 @@ k_trace(const Node* __restrict__ nodes, const float* __restrict__ tris, uint32_t
   // reference's.  An entry stands for a pushed node and holds what its own
   // node record gave when its box was tested: its two children and the box's
   // entry distance (the reference's tmin), so popping it needs no further
-  // load.  Entries 0 .. sp - 2 are in LDS (the first kStackLds, one column
-  // per thread and field) and a private array (the rest, the only thing in
-  // private memory); the top one is kept in registers: a pop hands it over at
-  // once and leaves the register stale (stale: the top is still entry
-  // sp - 1).  The reload is issued after the children's fetches, so the
-  // latencies overlap; a push onto a stale top needs no reload at all.
+  // load.  The top entry is kept in registers: a pop hands it over at once
+  // and leaves the register stale (stale: the top is still entry sp - 1); its
+  // reload is issued after the children's fetches, so the latencies overlap,
+  // and a push onto a stale top needs no reload at all.  Of the entries below
+  // it, the kStackLds nearest the top are in an LDS ring (one column per
+  // thread and field) and the first `low` in a private array: a ray at any
+  // depth works in the ring, and goes to private memory only when it has
+  // climbed or sunk by kStackLds entries.
   __shared__ uint32_t s_stk[3 * kStackLds * kTraceBlock];
-  uint3 spill[kStack - kStackLds];
-  auto stk_store = [&](uint32_t e, uint3 v) {
-    if (e < uint32_t(kStackLds)) {
-      uint32_t* q = &s_stk[e * kTraceBlock + threadIdx.x];
-      q[0] = v.x;
-      q[kStackLds * kTraceBlock] = v.y;
-      q[2 * kStackLds * kTraceBlock] = v.z;
-    } else {
-      spill[e - kStackLds] = v;
-    }
-  };
-  auto stk_load = [&](uint32_t e) -> uint3 {
-    if (e < uint32_t(kStackLds)) {
-      const uint32_t* q = &s_stk[e * kTraceBlock + threadIdx.x];
-      return make_uint3(q[0], q[kStackLds * kTraceBlock], q[2 * kStackLds * kTraceBlock]);
-    }
-    return spill[e - kStackLds];
+  uint3 spill[kStack];
+  uint32_t low = 0;
+  auto ring = [&](uint32_t e) { return &s_stk[(e & (kStackLds - 1)) * kTraceBlock + threadIdx.x]; };
+  auto ring_load = [&](uint32_t e) {
+    const uint32_t* q = ring(e);
+    return make_uint3(q[0], q[kStackLds * kTraceBlock], q[2 * kStackLds * kTraceBlock]);
   };
   uint3 top = make_uint3(0u, 0u, 0u);
   uint32_t sp = 0;
   bool stale = false;
-  auto push = [&](uint32_t l, uint32_t rr, float tn) {
-    if (sp >= kStack)
-      return;
-    if (sp > 0 && !stale)
-      stk_store(sp - 1, top);
+  auto push = [&](uint3 v) {
+    if (sp > 0 && !stale) {
+      const uint32_t e = sp - 1;
+      if (e - low == uint32_t(kStackLds)) {
+        spill[low] = ring_load(low);
+        low++;
+      }
+      uint32_t* q = ring(e);
+      q[0] = top.x;
+      q[kStackLds * kTraceBlock] = top.y;
+      q[2 * kStackLds * kTraceBlock] = top.z;
+    }
     stale = false;
-    top = make_uint3(l, rr, __float_as_uint(tn));
+    top = v;
     sp++;
   };
-  auto pop = [&]() {
-    if (stale)
-      top = stk_load(sp - 1);
-    const uint3 e = top;
-    sp--;
-    stale = sp > 0;
-    return e;
+  auto reload = [&]() { // a stale top (sp > 0)
+    const uint32_t e = sp - 1;
+    if (e < low) {
+      top = spill[e];
+      low = e;
+      // waited for here: left pending, it would make every later wait for a
+      // child's data wait for more than that data
+      __builtin_amdgcn_s_waitcnt(kWaitVmem0);
+    } else {
+      top = ring_load(e);
+    }
+    stale = false;
   };
 
-  uint32_t best = 0xffffffffu;
-  float best_t = INFINITY, best_u = 0.0f, best_v = 0.0f;
+  Hit best;
 
   // The reference pushes the root and pops it at once: its record gives the
   // first two children.  A node it would push and pop again straight away
   // (the near child, or a single hit child) is taken directly here, but only
   // when that push would have found room, so the visit order and the
   // drop-when-full rule are unchanged.
-  const float* nodes_f = reinterpret_cast<const float*>(nodes);
-  uint32_t cl = 0u, cr = 0u;
-  bool have = false;
   if (nprims >= 2u) {
-    const float4 q1 = reinterpret_cast<const float4*>(nodes_f)[1];
-    cl = __float_as_uint(q1.z);
-    cr = __float_as_uint(q1.w);
-    have = true;
-  }
-  for (;;) {
-    // A pruned entry goes back to the loop head by the same path as a node
-    // whose children both miss: with a separate path, the compiler's
-    // structurizer nests loops and duplicates the child tests (measured 12%
-    // slower on the clustered 1M scene).
-    bool visit = true;
-    if (!have) {
-      if (sp == 0)
-        break;
-      const uint3 e = pop();
-      visit = !(best_t < __uint_as_float(e.z));
-      cl = e.x;
-      cr = e.y;
-    }
-    have = false;
-    if (!visit)
-      continue;
-    // Both children's data at once: a leaf's triangle, an internal node's
-    // record (its box and children).  A child out of range (only possible
-    // for a corrupt node array) is skipped.
-    const uint32_t ch[2] = { cl, cr };
-    bool ok[2];
-    float4 q[2][3];
+    const float4 root = reinterpret_cast<const float4*>(nodes)[1];
+    uint32_t ch[2] = { __float_as_uint(root.z), __float_as_uint(root.w) };
+    const char* const node_base = reinterpret_cast<const char*>(nodes);
+    const char* const tri_base = reinterpret_cast<const char*>(tris);
+    const uint32_t last_leaf = nprims - 1u, last_node = nprims - 2u;
+    for (;;) {
+      // Both children's data at once: a leaf's triangle, an internal node's
+      // record (its box and children).  A child out of range (only possible
+      // for a corrupt node array) is skipped; its loads go to the array's last
+      // entry.  Offsets in 16-byte units: a node record is 2, a triangle 3.
+      bool leaf[2], ok[2];
+      uint32_t idx[2];
+      float4 q0[2], q1[2], q2[2];
+      const float4* at[2];
 #pragma unroll
-    for (int side = 0; side < 2; side++) {
-      const uint32_t c = ch[side];
-      const bool leaf = (c & kLeafBit) != 0u;
-      ok[side] = leaf ? ((c & ~kLeafBit) < nprims) : (c + 1 < nprims);
-      q[side][0] = q[side][1] = q[side][2] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-      if (ok[side]) {
-        const float4* a = reinterpret_cast<const float4*>(
-          leaf ? tris + 12 * uint64_t(c & ~kLeafBit) : nodes_f + 8 * uint64_t(c));
-        q[side][0] = a[0];
-        q[side][1] = a[1];
-        if (leaf)
-          q[side][2] = a[2];
+      for (int side = 0; side < 2; side++) {
+        leaf[side] = int32_t(ch[side]) < 0;
+        const uint32_t x = ch[side] & ~kLeafBit;
+        const uint32_t lim = leaf[side] ? last_leaf : last_node;
+        ok[side] = x <= lim;
+        idx[side] = x < lim ? x : lim;
+        const uint32_t units = idx[side] * 2u + (leaf[side] ? idx[side] : 0u);
+        const char* base = leaf[side] ? tri_base : node_base;
+        at[side] = reinterpret_cast<const float4*>(base + (uint64_t(units) << 4));
       }
-    }
-    if (stale) { // reload the top while the children are in flight
-      top = stk_load(sp - 1);
-      stale = false;
-    }
-    bool hit2[2] = { false, false };
-    float tn2[2] = { 0.0f, 0.0f };
-    uint32_t gl[2] = { 0u, 0u }, gr[2] = { 0u, 0u };
 #pragma unroll
-    for (int side = 0; side < 2; side++) {
-      if (!ok[side])
-        continue;
-      const float4 a = q[side][0], b = q[side][1], c = q[side][2];
-      if (ch[side] & kLeafBit) {
-        const uint32_t p = ch[side] & ~kLeafBit;
+      for (int side = 0; side < 2; side++) {
+        q0[side] = at[side][0];
+        q1[side] = at[side][1];
+        if (leaf[side])
+          q2[side] = at[side][2];
+      }
+      if (stale) // reload the top while the children are in flight
+        reload();
+#pragma unroll
+      for (int side = 0; side < 2; side++) {
+        if (!(leaf[side] && ok[side]))
+          continue;
+        const float4 a = q0[side], b = q1[side], c = q2[side];
         Tri tr;
         tr.p0[0] = a.x;
         tr.p0[1] = a.y;
@@ -426,19 +429,20 @@ k_trace(const Node* __restrict__ nodes, const float* __restrict__ tris, uint32_t
         tr.nrm[0] = c.y;
         tr.nrm[1] = c.z;
         tr.nrm[2] = c.w;
-        float t, u, v;
-        bool hit = (MODE == 2) ? isect_watertight(tr, r, t, u, v) : isect_reference(tr, r, t, u, v);
-        if (hit && better<MODE>(t, p, best_t, best)) {
-          best = p;
-          best_t = t;
-          best_u = u;
-          best_v = v;
-        }
-      } else {
+        if constexpr (MODE == 2)
+          isect_watertight<MODE>(tr, idx[side], r, best);
+        else
+          isect_reference<MODE>(tr, idx[side], r, best);
+      }
+      // The box tests of both sides, on a leaf's side without effect: no
+      // divergence, and a box test is cheaper than the branches around it.
+      bool hit2[2];
+      float tn2[2];
+#pragma unroll
+      for (int side = 0; side < 2; side++) {
+        const float4 a = q0[side], b = q1[side];
         const float lo[3] = { a.x, a.y, a.z };
         const float hi[3] = { a.w, b.x, b.y };
-        gl[side] = __float_as_uint(b.z);
-        gr[side] = __float_as_uint(b.w);
         float tn[3], tf[3];
 #pragma unroll
         for (int k = 0; k < 3; k++) {
@@ -449,41 +453,49 @@ k_trace(const Node* __restrict__ nodes, const float* __restrict__ tris, uint32_t
           float pf = fb * rcp[k];
           tf[k] = pf + ipos[k];
         }
-        float tmin = m_max(m_max(tn[0], tn[1]), tn[2]);
-        float tmax = m_min(m_min(tf[0], tf[1]), tf[2]);
-        hit2[side] = tmax >= m_max(0.0f, tmin);
+        const float tmin = m_max(m_max(tn[0], tn[1]), tn[2]);
+        const float tmax = m_min(m_min(tf[0], tf[1]), tf[2]);
+        // tmax >= max(0, tmin), false for a NaN on either side
+        hit2[side] = !leaf[side] && ok[side] && (tmax >= tmin) && (tmax >= 0.0f);
         tn2[side] = tmin;
       }
-    }
-    const bool lh = hit2[0], rh = hit2[1];
-    uint32_t next_l, next_r;
-    float next_t;
-    if (lh && rh) {
-      const bool left_near = tn2[0] < tn2[1];
-      const int far = left_near ? 1 : 0;
-      push(gl[far], gr[far], tn2[far]);
-      next_l = gl[1 - far];
-      next_r = gr[1 - far];
-      next_t = tn2[1 - far];
-    } else if (lh || rh) {
-      next_l = lh ? gl[0] : gl[1];
-      next_r = lh ? gr[0] : gr[1];
-      next_t = lh ? tn2[0] : tn2[1];
-    } else {
-      continue;
-    }
-    // push-then-pop of the near child: its push needs room; its pop is then
-    // pruned when a closer hit is already known
-    if (sp < kStack && !(best_t < next_t)) {
-      cl = next_l;
-      cr = next_r;
-      have = true;
+      const bool left_first = hit2[0] && (!hit2[1] || tn2[0] < tn2[1]);
+      const uint32_t gl0 = __float_as_uint(q1[0].z), gr0 = __float_as_uint(q1[0].w);
+      const uint32_t gl1 = __float_as_uint(q1[1].z), gr1 = __float_as_uint(q1[1].w);
+      const float next_t = left_first ? tn2[0] : tn2[1];
+      ch[0] = left_first ? gl0 : gl1;
+      ch[1] = left_first ? gr0 : gr1;
+      // push-then-pop of the near child: its push needs room; its pop is then
+      // pruned when a closer hit is already known
+      bool have = hit2[0] || hit2[1];
+      if (hit2[0] && hit2[1] && sp < uint32_t(kStack)) {
+        push(make_uint3(left_first ? gl1 : gl0, left_first ? gr1 : gr0,
+                        __float_as_uint(left_first ? tn2[1] : tn2[0])));
+      }
+      have = have && sp < uint32_t(kStack) && !(best.t < next_t);
+      // Pruned entries are dropped here, one after another: a trip round the
+      // outer loop for each would wait for the other lanes' visits.
+      while (!have && sp > 0) {
+        if (stale)
+          reload();
+        sp--;
+        stale = sp > 0;
+        ch[0] = top.x;
+        ch[1] = top.y;
+        have = !(best.t < __uint_as_float(top.z));
+      }
+      // Every lane meets here before the next visit: without it the compiler
+      // lets the lanes that already have a node loop on alone (twice the
+      // visits per wave, measured).
+      __builtin_amdgcn_wave_barrier();
+      if (!have)
+        break;
     }
   }
-  prim_out[i] = best;
-  t_out[i] = best_t;
+  prim_out[i] = best.prim;
+  t_out[i] = best.t;
   if (uv_out)
-    *reinterpret_cast<float2*>(uv_out + 2 * i) = make_float2(best_u, best_v);
+    *reinterpret_cast<float2*>(uv_out + 2 * i) = make_float2(best.u, best.v);
 }
 
 // ---- traversal order of a ray batch ---------------------------------------------

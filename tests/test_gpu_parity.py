@@ -90,6 +90,30 @@ def test_trace_deep_stacks_match_oracle(ctx, nrays, mode):
     bvh.destroy()
 
 
+@pytest.mark.parametrize("n", [128, 256, 513, 1024, 70000, 131072])
+def test_trace_stack_ring_depths_match_oracle(ctx, n):
+    """Concentric triangles of one centre: equal codes, so a balanced tree of
+    ceil(log2 n) levels, and every ray through the centre enters both children
+    of every node, down to stacks just below, at and past the 8 entries of the
+    LDS ring and past two rings."""
+    s = (np.arange(1, n + 1, dtype=np.float64) * 2.0 ** -20)[:, None]
+    corner = np.array([[-1, -1, -1], [1, -1, 0], [0, 1, 1]], dtype=np.float64)
+    v = np.concatenate([0.5 + s * corner[k] for k in range(3)], axis=1).astype(np.float32)
+    tri = W.make_triangles(v[np.random.default_rng(n).permutation(n)])
+    rays = W.primary_rays(9, 7)
+    rays[:, 3:6] = (0.5 - rays[:, 0:3]) + np.random.default_rng(1).normal(size=(63, 3)) * 2.0 ** -18
+    bvh = ctx.build_triangles(tri, code_bits=30, leaf_order=1)
+    nodes, _, _, _ = oracle.build(tri, 30, 1)
+    assert bvh.nodes().tobytes() == nodes.tobytes()
+    p, t, uv = ctx.trace(bvh, rays, 0)
+    op, ot, ouv = oracle.trace(nodes, tri, rays, 0)
+    assert (p != 0xFFFFFFFF).any()
+    assert np.array_equal(p, op)
+    assert np.array_equal(t.view(np.uint32), ot.view(np.uint32))
+    assert np.array_equal(uv.view(np.uint32), ouv.view(np.uint32))
+    bvh.destroy()
+
+
 @pytest.mark.parametrize("n", [2, 3, 5, 33, 4097, 70001])
 @pytest.mark.parametrize("bits,leaf", VARIANTS, ids=VIDS)
 def test_build_matches_oracle_ragged(ctx, n, bits, leaf):
