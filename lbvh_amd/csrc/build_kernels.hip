@@ -340,34 +340,38 @@ key_code(KeyT k)
     return CodeT(k);
 }
 
+// The box that changes no union: +inf low, -inf high.
+__device__ __forceinline__ Box
+empty_box()
+{
+  Box b;
+#pragma unroll
+  for (int k = 0; k < 3; k++) {
+    b.lo[k] = INFINITY;
+    b.hi[k] = -INFINITY;
+  }
+  return b;
+}
+
 // Union of element boxes [a, b] left to right, from a bottom-up segment
 // tree over m elements (leaves at bt[m + e]; bt[p] = union(bt[2p],
-// bt[2p + 1])).  std::min / std::max with the left operand kept on ties
-// are associative on non-NaN values, so any order-preserving grouping gives
-// the bits of the reference's union of its two children, recursively.
+// bt[2p + 1]); bt[0] = empty_box()).  std::min / std::max with the left
+// operand kept on ties are associative on non-NaN values, so any
+// order-preserving grouping gives the bits of the reference's union of its
+// two children, recursively -- also for a whole node's range at once.  A
+// side that takes no node at a level takes bt[0]: no branches inside.
 __device__ __forceinline__ Box
 bt_query(const Box* __restrict__ bt, int m, int a, int b)
 {
   int l = a + m, r = b + m + 1;
-  Box rl, rr;
-  bool hl = false, hr = false;
+  Box rl = empty_box(), rr = empty_box();
   while (l < r) {
-    if (l & 1) {
-      rl = hl ? box_union(rl, bt[l]) : bt[l];
-      hl = true;
-      l++;
-    }
-    if (r & 1) {
-      r--;
-      rr = hr ? box_union(bt[r], rr) : bt[r];
-      hr = true;
-    }
-    l >>= 1;
+    rl = box_union(rl, bt[(l & 1) ? l : 0]);
+    rr = box_union(bt[(r & 1) ? r - 1 : 0], rr);
+    l = (l + 1) >> 1;
     r >>= 1;
   }
-  if (hl && hr)
-    return box_union(rl, rr);
-  return hl ? rl : rr;
+  return box_union(rl, rr);
 }
 
 __device__ __forceinline__ bool
@@ -512,6 +516,8 @@ k_fit_treelets(const float* __restrict__ prims_all, int kind, Scenes sc, Node* _
       bool bad = false;
       if (t < m)
         bad = box_has_nan(s_bt[m + t] = leaf_box(prims, kind, leafprim, lo + t));
+      if (t == 0)
+        s_bt[0] = empty_box();
       const bool nan = __syncthreads_or(bad ? 1 : 0) != 0;
       // this thread's internal node k = base + t (t < m - 1): range, children, split
       const int64_t k = base + t;
@@ -545,9 +551,7 @@ k_fit_treelets(const float* __restrict__ prims_all, int kind, Scenes sc, Node* _
           __syncthreads();
         }
         if (mine) {
-          const Box lb = bt_query(s_bt, m, int(L - lo), int(g - lo));
-          const Box rb = bt_query(s_bt, m, int(g + 1 - lo), int(R - lo));
-          store_node(&nodes[k], box_union(lb, rb), lv, rv);
+          store_node(&nodes[k], bt_query(s_bt, m, int(L - lo), int(R - lo)), lv, rv);
         }
       } else {
         // children before parents: node box of base + j at s_bt[1 + j]
@@ -689,14 +693,16 @@ k_fit_top(const float* __restrict__ prims_all, int kind, Scenes sc, Node* __rest
 //     algorithm over a shorter position range) and then merges those.
 // Within a workgroup, with d[e] the delta left of element e, the node split
 // between elements j and j + 1 spans elements [a, b] where d[a] and d[b + 1]
-// are the nearest deltas below d[j + 1] on either side (searched in a min
-// tree over d); it lies in the workgroup when both exist.  Its children are
+// are the nearest deltas below d[j + 1] on either side; it lies in the
+// workgroup when both exist.  Deltas are kept as bytes, with the minimum of
+// every 8 and of every 64, and searched 8 at a time in a register pair (see
+// DeltaIndex).  Its children are
 // the elements j or j + 1 or the nodes numbered j and j + 1 in element
 // space, so boxes follow in passes, each node once both
 // children are done (the reference's union order).  Nodes and elements
 // whose parent does not lie in the workgroup -- at most two per tree level,
 // so at most kTreeSegCap -- are listed in position order
-// ({l, r, delta(l - 1), delta(r), box}).  The single workgroup of the last
+// ({l, r, delta codes of l - 1 and r, box}).  The single workgroup of the last
 // level completes every remaining node.  Segments and tickets cross
 // workgroups (and XCDs) through coherent stores, a vector-memory drain and
 // the ticket atomic; tickets reset themselves.
@@ -715,39 +721,167 @@ static_assert(kTreeFan % kTreeSubFan == 0 && kTreeSubLists * kTreeSegCap <= kTre
               "split merges fit");
 static_assert(kTreeFan <= kWave, "one wave scans a group's list counts");
 
-// A listed subtree: leaf range [l, r], delta(l - 1) and delta(r) (packed as
-// int16 pairs), box.
+// A listed subtree: leaf range [l, r], the delta codes of l - 1 and r, box.
 struct TreeEntry
 {
   uint32_t l, r;
-  uint32_t d; // (delta(l - 1) & 0xffff) | delta(r) << 16
+  uint32_t d; // code(l - 1) | code(r) << 8
   float box[6];
 };
 static_assert(sizeof(TreeEntry) == 36, "TreeEntry layout");
 
-// delta(x, x + 1) over sorted batch positions; -1 at scene edges.
+// The byte code of delta(x, x + 1) for the keys a, b of the sorted batch
+// positions x and x + 1: 0 at a scene's edge, then in delta's order.  A delta
+// below 64 is its leading equal code bits; one of equal 64-bit codes is 64
+// plus the leading zeros of a 64-bit index difference below 2^31, so at least
+// 97, and moves down to keep every code below kDeltaInf.
+constexpr uint32_t kDeltaInf = 127;
+
 template<typename KeyT, typename CodeT, bool SEG>
-__device__ __forceinline__ int
-adj_delta(const KeyT* __restrict__ keys, const uint64_t* __restrict__ prim_off, int64_t N,
-          int64_t x)
+__device__ __forceinline__ uint32_t
+delta_code(KeyT a, KeyT b, uint32_t x, const uint64_t* __restrict__ prim_off)
 {
-  if (x < 0 || x >= N - 1)
-    return -1;
-  const KeyT a = keys[x];
-  const KeyT b = keys[x + 1];
   if constexpr (SEG) {
     if ((a >> 30) != (b >> 30))
-      return -1;
+      return 0u;
   }
   const CodeT ca = key_code<KeyT, CodeT, SEG>(a);
   const CodeT cb = key_code<KeyT, CodeT, SEG>(b);
   if (ca != cb)
-    return CodeTraits<CodeT>::clz(ca ^ cb);
-  int64_t i = x;
+    return 1u + uint32_t(CodeTraits<CodeT>::clz(ca ^ cb));
+  uint32_t i = x;
   if constexpr (SEG)
-    i -= int64_t(prim_off[uint32_t(a >> 30)]);
-  return CodeTraits<CodeT>::clz(CodeT(uint64_t(i ^ (i + 1)))) + CodeTraits<CodeT>::bits;
+    i -= uint32_t(prim_off[uint32_t(a >> 30)]);
+  // clz(index difference) + bits(code): + 32 and below 64 for 32-bit codes;
+  // + 64 for 64-bit ones, where the index's upper 32 zeros make it 96 + clz32
+  const uint32_t z = uint32_t(__clz(int(i ^ (i + 1u))));
+  return CodeTraits<CodeT>::bits == 32 ? 33u + z : 65u + z;
 }
+
+// The byte codes of a workgroup's deltas d[0 .. m] with the minimum of every
+// word of 8 and of every chunk of 64 (all padded with kDeltaInf), for the
+// nearest-smaller searches.  Codes are below 128, so 8 of them are compared
+// with one value by a subtraction that never borrows across bytes: a search
+// reads at most one word at each of the levels words, chunks, words of the
+// chunk found, and codes of the word found -- 3 to 5 dependent LDS reads,
+// where a binary min tree over 512 deltas takes up to 18.
+template<int SLOTS>
+struct DeltaIndex
+{
+  static constexpr int kChunks = SLOTS / 64 + 1; // of SLOTS + 1 codes
+  static constexpr int kTop = (kChunks + 7) / 8;
+  uint64_t code[kChunks * 8];
+  uint64_t word[kChunks]; // byte q of word[c]: minimum of code[8 c + q]
+  uint64_t chunk[kTop];   // byte q of chunk[t]: minimum of word[8 t + q]
+
+  __device__ __forceinline__ uint32_t at(int e) const
+  {
+    return reinterpret_cast<const uint8_t*>(code)[e];
+  }
+  // bit 7 of every byte that is less than x (x8: x in every byte of 32 bits)
+  static __device__ __forceinline__ uint64_t less(uint64_t w, uint32_t x8)
+  {
+    constexpr uint32_t H = 0x80808080u;
+    const uint32_t lo = ~((uint32_t(w) | H) - x8) & H;
+    const uint32_t hi = ~((uint32_t(w >> 32) | H) - x8) & H;
+    return (uint64_t(hi) << 32) | lo;
+  }
+  // of the bytes below / above byte q of a word
+  static __device__ __forceinline__ uint64_t below(int q)
+  {
+    return (uint64_t(1) << (8 * q)) - 1;
+  }
+  static __device__ __forceinline__ uint64_t above(int q)
+  {
+    return ~uint64_t(0xff) << (8 * q);
+  }
+  static __device__ __forceinline__ int last(uint64_t m) { return (63 - __clzll((long long)m)) >> 3; }
+  static __device__ __forceinline__ int first(uint64_t m) { return (__ffsll((long long)m) - 1) >> 3; }
+
+  // Largest i < p with d[i] < x, or -1.
+  __device__ __forceinline__ int left_less(int p, uint32_t x) const
+  {
+    const uint32_t x8 = x * 0x01010101u;
+    int w = p >> 3;
+    uint64_t f = less(code[w], x8) & below(p & 7);
+    if (!f) {
+      int c = w >> 3;
+      f = less(word[c], x8) & below(w & 7);
+      if (!f) {
+        int k = c >> 3;
+        f = less(chunk[k], x8) & below(c & 7);
+        while (!f && k > 0)
+          f = less(chunk[--k], x8);
+        if (!f)
+          return -1;
+        c = k * 8 + last(f);
+        f = less(word[c], x8);
+      }
+      w = c * 8 + last(f);
+      f = less(code[w], x8);
+    }
+    return w * 8 + last(f);
+  }
+  // Smallest i > p with d[i] < x, or -1.
+  __device__ __forceinline__ int right_less(int p, uint32_t x) const
+  {
+    const uint32_t x8 = x * 0x01010101u;
+    int w = p >> 3;
+    uint64_t f = less(code[w], x8) & above(p & 7);
+    if (!f) {
+      int c = w >> 3;
+      f = less(word[c], x8) & above(w & 7);
+      if (!f) {
+        int k = c >> 3;
+        f = less(chunk[k], x8) & above(c & 7);
+        while (!f && k < kTop - 1)
+          f = less(chunk[++k], x8);
+        if (!f)
+          return -1;
+        c = k * 8 + first(f);
+        f = less(word[c], x8);
+      }
+      w = c * 8 + first(f);
+      f = less(code[w], x8);
+    }
+    return w * 8 + first(f);
+  }
+  // The minima, from code[] (d[0 .. m] in place); a barrier before and after.
+  __device__ __forceinline__ void build(int m, int wave, int waves)
+  {
+    const int lane = __lane_id();
+    uint8_t* const cb = reinterpret_cast<uint8_t*>(code);
+    uint8_t* const wb = reinterpret_cast<uint8_t*>(word);
+    uint8_t* const kb = reinterpret_cast<uint8_t*>(chunk);
+    for (int c = wave; c < kTop * 8; c += waves) {
+      if (c >= kChunks) {
+        if (lane == 0)
+          kb[c] = uint8_t(kDeltaInf);
+        continue;
+      }
+      const int e = c * 64 + lane;
+      uint32_t v = kDeltaInf;
+      if (e <= m)
+        v = cb[e];
+      else
+        cb[e] = uint8_t(kDeltaInf);
+#pragma unroll
+      for (int off = 1; off < 8; off <<= 1) {
+        const uint32_t o = __shfl_xor(v, off, kWave);
+        v = o < v ? o : v;
+      }
+      if ((lane & 7) == 0)
+        wb[c * 8 + (lane >> 3)] = uint8_t(v);
+#pragma unroll
+      for (int off = 8; off < 64; off <<= 1) {
+        const uint32_t o = __shfl_xor(v, off, kWave);
+        v = o < v ? o : v;
+      }
+      if (lane == 0)
+        kb[c] = uint8_t(v);
+    }
+  }
+};
 
 // One scene's arrays, located from any of its sorted positions.
 struct TreeScene
@@ -805,55 +939,18 @@ struct TreeLevels
   uint32_t ticket_base[16]; // first ticket of each level's groups
 };
 
-constexpr int kTreeLeaf0 = 2048; // leaves of the delta min-tree (>= kTreeSlots + 1)
-static_assert(kTreeLeaf0 >= kTreeSlots + 1, "delta tree size");
-constexpr int kTreeLeaf0First = 1024; // the same at level 0 (>= kTreeLeaves + 1)
-static_assert(kTreeLeaf0First >= kTreeLeaves + 1, "level-0 delta tree size");
 constexpr int kTreeUpThreads = 1024; // workgroup of the upper levels (one CU each: LDS-bound)
-constexpr int16_t kTreeInf = 0x7fff;
 
-// Largest i <= j with d[i] < x, or -1 (tree: heap-ordered minima of d,
-// leaves at leaf0 + i).
-__device__ __forceinline__ int
-tree_left_less(const int16_t* __restrict__ tree, int leaf0, int j, int x)
-{
-  int p = j + leaf0;
-  if (tree[p] < x)
-    return j;
-  while (p > 1) {
-    if ((p & 1) && tree[p - 1] < x) {
-      p = p - 1;
-      while (p < leaf0)
-        p = (tree[2 * p + 1] < x) ? 2 * p + 1 : 2 * p;
-      return p - leaf0;
-    }
-    p >>= 1;
-  }
-  return -1;
-}
-
-// Smallest i >= j with d[i] < x, or -1.
-__device__ __forceinline__ int
-tree_right_less(const int16_t* __restrict__ tree, int leaf0, int j, int x)
-{
-  int p = j + leaf0;
-  if (tree[p] < x)
-    return j;
-  while (p > 1) {
-    if (!(p & 1) && tree[p + 1] < x) {
-      p = p + 1;
-      while (p < leaf0)
-        p = (tree[2 * p] < x) ? 2 * p : 2 * p + 1;
-      return p - leaf0;
-    }
-    p >>= 1;
-  }
-  return -1;
-}
-
-// FIRST: the level-0 kernel (leaves, 512 elements, ~40 KB of LDS: four workgroups fit a CU);
+// FIRST: the level-0 kernel (leaves, 512 elements, ~38 KB of LDS: four workgroups fit a CU);
 // else the kernel of the levels above (its workgroup b starts as level-1
 // workgroup b).
+//
+// Level 0 is bound by instruction issue beside its memory traffic, the levels
+// above by their chains of dependent LDS reads.  Both were mostly binary
+// searches and box queries: searching byte codes 8 at a time and querying a
+// node's box over its whole range instead of child by child took level 0 /
+// the levels above from 685 / 116 to 531 / 92 us (16M, 30-bit) and from 63 /
+// 46 to 54 / 34 us (1M, 63-bit).
 template<typename KeyT, typename CodeT, bool SEG, bool FIRST>
 __global__ __launch_bounds__(FIRST ? kTreeLeaves : kTreeUpThreads) void
 k_tree(const KeyT* __restrict__ keys, const uint32_t* __restrict__ ids, Scenes sc,
@@ -875,11 +972,9 @@ k_tree(const KeyT* __restrict__ keys, const uint32_t* __restrict__ ids, Scenes s
   // scene of each element (batches above level 0; level 0 reads it from the key)
   __shared__ uint32_t s_el_scene[(SEG && !FIRST) ? SL : 1];
   __shared__ uint32_t s_el_val[SL]; // child value when the element is one leaf
-  // min tree over d (leaves at kTreeLeaf0): d[e] is the delta left of
-  // element e, d[m] the delta right of the last
-  __shared__ int16_t s_tree[2 * (FIRST ? kTreeLeaf0First : kTreeLeaf0)];
-  __shared__ int16_t s_dsep[FIRST ? 1 : SL + 1];
-  int16_t* const s_d = FIRST ? s_tree + kTreeLeaf0First : s_dsep; // level 0: the tree's own leaves
+  // d[e] is the delta left of element e, d[m] the delta right of the last
+  __shared__ DeltaIndex<SL> s_dx;
+  uint8_t* const s_d = reinterpret_cast<uint8_t*>(s_dx.code);
   // split j (between elements j and j + 1): its node's element range [a, b]
   __shared__ uint16_t s_na[SL];
   __shared__ uint16_t s_nb[SL];
@@ -945,9 +1040,9 @@ k_tree(const KeyT* __restrict__ keys, const uint32_t* __restrict__ ids, Scenes s
       s_el_l[e] = el;
       s_el_r[e] = er;
       s_bt[m + e] = bx;
-      s_d[e + 1] = int16_t(d >> 16);
+      s_d[e + 1] = uint8_t(d >> 8);
       if (e == 0)
-        s_d[0] = int16_t(d & 0xffffu);
+        s_d[0] = uint8_t(d);
       int64_t P = 0;
       if constexpr (SEG) {
         const uint32_t sg = uint32_t(keys[el] >> 30);
@@ -989,10 +1084,26 @@ k_tree(const KeyT* __restrict__ keys, const uint32_t* __restrict__ ids, Scenes s
     const int64_t lo = int64_t(blk) * kTreeLeaves;
     const int64_t hi = (N - lo < kTreeLeaves) ? N : lo + kTreeLeaves;
     m = int(hi - lo);
-    s_d[t] = int16_t(adj_delta<KeyT, CodeT, SEG>(keys, sc.prim_off, N, lo - 1 + t));
-    if (t == 0)
-      s_d[kTreeLeaves] =
-        int16_t(adj_delta<KeyT, CodeT, SEG>(keys, sc.prim_off, N, lo - 1 + kTreeLeaves));
+    // d[e] between the keys of positions lo + e - 1 and lo + e; 0 past either end
+    {
+      const uint32_t x = uint32_t(lo) + uint32_t(t);
+      const uint32_t last = uint32_t(N) - 1u;
+      const KeyT key = keys[x < last ? x : last];
+      KeyT before = key;
+      if (sizeof(KeyT) == 8)
+        before = (KeyT(__shfl_up(uint32_t(uint64_t(key) >> 32), 1, kWave)) << (sizeof(KeyT) * 4)) |
+                 KeyT(__shfl_up(uint32_t(key), 1, kWave));
+      else
+        before = KeyT(__shfl_up(uint32_t(key), 1, kWave));
+      if (lane == 0 && x > 0 && x <= last)
+        before = keys[x - 1];
+      s_d[t] = uint8_t((x > 0 && x <= last)
+                         ? delta_code<KeyT, CodeT, SEG>(before, key, x - 1, sc.prim_off)
+                         : 0u);
+      if (t == kTreeLeaves - 1)
+        s_d[kTreeLeaves] =
+          uint8_t(x < last ? delta_code<KeyT, CodeT, SEG>(key, keys[x + 1], x, sc.prim_off) : 0u);
+    }
     if (t < m) {
       const int64_t x = lo + t;
       const TreeScene ts = tree_scene<KeyT, SEG>(keys, sc, x, prims_all, kind, nodes_all,
@@ -1018,39 +1129,23 @@ k_tree(const KeyT* __restrict__ keys, const uint32_t* __restrict__ ids, Scenes s
 
   for (;;) {
     // ---- nodes of this workgroup: ranges from the nearest smaller deltas -------
-    // level 0: kTreeLeaf0First leaves, d already in place; above: the next power of two
-    int leaf0 = kTreeLeaf0First;
-    if constexpr (!FIRST) {
-      leaf0 = 2;
-      while (leaf0 < m + 1)
-        leaf0 <<= 1;
-      for (int q = t; q <= m; q += NT)
-        s_tree[leaf0 + q] = s_d[q];
-    }
-    for (int q = m + 1 + t; q < leaf0; q += NT)
-      s_tree[leaf0 + q] = kTreeInf;
-    __syncthreads();
+    s_dx.build(m, w, NT / kWave);
+    if (t == 0)
+      s_bt[0] = empty_box();
     // exact NaN semantics need the unions in tree order (passes below)
     int any_nan = 0;
     for (int e = t; e < m; e += NT)
       any_nan |= box_has_nan(s_bt[m + e]) ? 1 : 0;
     const bool nan = __syncthreads_or(any_nan) != 0;
-    for (int half = leaf0 / 2; half >= 1; half >>= 1) {
-      for (int q = t; q < half; q += NT) {
-        const int p = half + q;
-        const int16_t a0 = s_tree[2 * p], a1 = s_tree[2 * p + 1];
-        s_tree[p] = a0 < a1 ? a0 : a1;
-        if (!nan && p < m)
-          s_bt[p] = box_union(s_bt[2 * p], s_bt[2 * p + 1]);
-      }
-      __syncthreads();
-    }
+    int half0 = 1; // the deepest level of the box tree that holds unions
+    while (half0 * 2 < m)
+      half0 <<= 1;
     for (int j = t; j < m - 1; j += NT) {
-      const int x = s_d[j + 1];
+      const uint32_t x = s_d[j + 1];
       uint8_t inb = 0;
-      if (x >= 0) {
-        const int i = tree_left_less(s_tree, leaf0, j, x);
-        const int k = tree_right_less(s_tree, leaf0, j + 2, x);
+      if (x > 0) {
+        const int i = s_dx.left_less(j + 1, x);
+        const int k = s_dx.right_less(j + 1, x);
         if (i >= 0 && k >= 0) {
           inb = 1;
           s_na[j] = uint16_t(i);
@@ -1064,7 +1159,14 @@ k_tree(const KeyT* __restrict__ keys, const uint32_t* __restrict__ ids, Scenes s
       s_esc[e] = 0;
       s_kid[e] = 0xffff;
     }
-    __syncthreads();
+    for (int half = half0; half >= 1; half >>= 1) {
+      for (int q = t; q < half; q += NT) {
+        const int p = half + q;
+        if (!nan && p < m)
+          s_bt[p] = box_union(s_bt[2 * p], s_bt[2 * p + 1]);
+      }
+      __syncthreads();
+    }
     for (int j = t; j < m - 1; j += NT) {
       if (s_inb[j]) {
         const int a = s_na[j], b = s_nb[j];
@@ -1147,16 +1249,7 @@ k_tree(const KeyT* __restrict__ keys, const uint32_t* __restrict__ ids, Scenes s
       const int a = s_na[j], b = s_nb[j];
       const bool l_el = (a == j);
       const bool r_el = (j + 1 == b);
-      Box lb, rb, bx;
-      if (nan) {
-        lb = l_el ? s_bt[m + j] : s_bt[1 + s_kid[j]];
-        rb = r_el ? s_bt[m + j + 1] : s_bt[1 + s_kid[j + 1]];
-        bx = s_bt[1 + j];
-      } else {
-        lb = bt_query(s_bt, m, a, j);
-        rb = bt_query(s_bt, m, j + 1, b);
-        bx = box_union(lb, rb);
-      }
+      const Box bx = nan ? s_bt[1 + j] : bt_query(s_bt, m, a, b);
       const int64_t L = s_el_l[a];
       const int64_t R = s_el_r[b];
       const int64_t g = s_el_r[j];
@@ -1176,7 +1269,7 @@ k_tree(const KeyT* __restrict__ keys, const uint32_t* __restrict__ ids, Scenes s
     // ---- listed subtrees: elements and nodes whose parent is not in here ------
     auto parent_out = [&](int a, int b) {
       const int da = s_d[a], db = s_d[b + 1];
-      if (da < 0 && db < 0)
+      if (da == 0 && db == 0)
         return false; // the scene's root
       const int ps = (db > da) ? b : a - 1;
       return ps < 0 || ps > m - 2 || !s_inb[ps];
@@ -1239,7 +1332,7 @@ k_tree(const KeyT* __restrict__ keys, const uint32_t* __restrict__ ids, Scenes s
       TreeEntry* en = &out[o++];
       coherent_store_u32(&en->l, s_el_l[a]);
       coherent_store_u32(&en->r, s_el_r[b]);
-      coherent_store_u32(&en->d, (uint32_t(int(s_d[a])) & 0xffffu) | (uint32_t(int(s_d[b + 1])) << 16));
+      coherent_store_u32(&en->d, uint32_t(s_d[a]) | (uint32_t(s_d[b + 1]) << 8));
 #pragma unroll
       for (int q = 0; q < 3; q++) {
         coherent_store_f32(&en->box[q], bx.lo[q]);
