@@ -128,6 +128,12 @@ void lbvh_build_opts_init(lbvh_build_opts* o); /* 30-bit, REFERENCE leaves */
 lbvh_status lbvh_ctx_create(int device, lbvh_ctx** out);
 void lbvh_ctx_destroy(lbvh_ctx* ctx);
 lbvh_status lbvh_ctx_set_stream(lbvh_ctx* ctx, void* hip_stream);
+/* Orders the context after another stream of its device (a hipStream_t; NULL:
+ * the default stream): work queued on the context from now on starts after the
+ * work queued on `stream` so far.  Does not block the host.  Nothing to do (and
+ * nothing done) when it is the context's own stream, or while one of the two is
+ * being captured into a graph: the order is then the caller's. */
+lbvh_status lbvh_ctx_wait_stream(lbvh_ctx* ctx, void* stream);
 lbvh_status lbvh_ctx_synchronize(lbvh_ctx* ctx);
 /* Device timing of the following calls with HIP events on the context
  * stream: mode 0 off, 1 every phase, 2 one interval per call (no events

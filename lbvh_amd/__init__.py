@@ -124,6 +124,7 @@ SIGNATURES = {
     "lbvh_ctx_create": (ctypes.c_int, [ctypes.c_int, ctypes.POINTER(VP)]),
     "lbvh_ctx_destroy": (None, [VP]),
     "lbvh_ctx_set_stream": (ctypes.c_int, [VP, VP]),
+    "lbvh_ctx_wait_stream": (ctypes.c_int, [VP, VP]),
     "lbvh_ctx_synchronize": (ctypes.c_int, [VP]),
     "lbvh_ctx_set_timing": (ctypes.c_int, [VP, ctypes.c_int]),
     "lbvh_ctx_phase_ms": (ctypes.c_int, [VP, F32P, ctypes.c_uint32,
@@ -207,14 +208,25 @@ def _is_torch(x):
     return type(x).__module__.startswith("torch")
 
 
+_one_runtime = False  # seen with the engine loaded
+
+
 def _single_runtime():
-    """True when the process maps one copy of the HIP runtime."""
+    """True when the process maps one copy of the HIP runtime.  Once that was
+    seen with the engine loaded (and a torch CUDA tensor in hand) it stays
+    true: both are bound to that copy.  Reading the process's maps takes
+    longer than a small build, so it is not repeated."""
+    global _one_runtime
+    if _one_runtime:
+        return True
     try:
         with open("/proc/self/maps") as f:
             paths = set(line.split()[-1] for line in f if "libamdhip64" in line)
     except OSError:
         return True
-    return len(paths) <= 1
+    one = len(paths) <= 1
+    _one_runtime = one and _lib is not None
+    return one
 
 
 def _is_device(x):
@@ -402,6 +414,7 @@ class Batch:
             if not _is_device(tri):
                 raise ValueError("rebuild takes device triangles")
             _check_dev(tri, "triangles", (np.float32,), count=12 * self.n)
+            self.ctx._after(tri)
             p = _dptr(tri)
             self._keep = tri
         self.ctx._check(lib().lbvh_batch_rebuild(self.ctx.handle, self.handle, p, int(graph)))
@@ -413,6 +426,7 @@ class Batch:
             if not _is_device(tri):
                 raise ValueError("refit takes device triangles")
             _check_dev(tri, "triangles", (np.float32,), count=12 * self.n)
+            self.ctx._after(tri)
             p = _dptr(tri)
             self._keep = tri
         self.ctx._check(lib().lbvh_batch_refit(self.ctx.handle, self.handle, p, int(graph)))
@@ -425,6 +439,7 @@ class Batch:
             if not _is_device(ray_offsets):
                 raise ValueError("device rays need device ray offsets")
             m = _check_dev(rays, "rays", (np.float32,), width=8)
+            self.ctx._after(rays)
             _check_dev(ray_offsets, "ray offsets", (np.uint64, np.int64),
                        count=self.n_scenes + 1)
             if out is None:
@@ -617,6 +632,14 @@ class Context:
             raw = ctypes.c_void_p(int(getattr(stream, "cuda_stream", stream)))
         self._check(lib().lbvh_ctx_set_stream(self.handle, raw))
 
+    def _after(self, x):
+        """Orders the context after the stream that torch is on, when `x` is a
+        torch tensor: what it holds may still be being written there."""
+        if _is_torch(x):
+            from torch.cuda import current_stream
+            self._check(lib().lbvh_ctx_wait_stream(
+                self.handle, ctypes.c_void_p(current_stream(x.device).cuda_stream)))
+
     def synchronize(self):
         self._check(lib().lbvh_ctx_synchronize(self.handle))
 
@@ -677,6 +700,7 @@ class Context:
         out = ctypes.c_void_p()
         if _is_device(prims):
             n = _check_dev(prims, "primitives", (np.float32,), width=width)
+            self._after(prims)
             self._check(getattr(lib(), fn + "_device")(self.handle, _dptr(prims), n,
                                                        ctypes.byref(opts), ctypes.byref(out)))
             return Bvh(self, out, n, code_bits, leaf_order, keep=prims)
@@ -696,6 +720,7 @@ class Context:
         opts = _make_opts(63, leaf_order, False, sort_digit_bits, sort_tile, sort_strategy)
         if _is_device(boxes):
             n = _check_dev(boxes, "boxes", (np.float64,), width=6)
+            self._after(boxes)
             if out is None:
                 if _is_torch(boxes):
                     import torch
@@ -730,6 +755,7 @@ class Context:
             m = _check_dev(rays, "rays", (np.float64,), width=8)
             if _dev_nbytes(nodes) < 64 * max(n - 1, 0):
                 raise ValueError("nodes hold fewer than 64 (n - 1) bytes")
+            self._after(rays)
             if out is None:
                 from .hip import DeviceArray
                 prim = DeviceArray(m, np.uint64)
@@ -769,6 +795,7 @@ class Context:
         out = ctypes.c_void_p()
         if _is_device(tri):
             _check_dev(tri, "triangles", (np.float32,), count=12 * int(off[-1]))
+            self._after(tri)
             self._check(lib().lbvh_build_batch_device(self.handle, _dptr(tri), _hptr(off), nseg,
                                                       ctypes.byref(opts), ctypes.byref(out)))
             return Batch(self, out, off, leaf_order, keep=tri)
@@ -782,6 +809,7 @@ class Context:
     def refit_triangles(self, bvh, tri):
         if _is_device(tri):
             _check_dev(tri, "triangles", (np.float32,), count=12 * bvh.n)
+            self._after(tri)
             self._check(lib().lbvh_refit_triangles_device(self.handle, bvh.handle, _dptr(tri)))
             bvh._keep = tri
             return
@@ -798,6 +826,7 @@ class Context:
         reading)."""
         if _is_device(rays):
             m = _check_dev(rays, "rays", (np.float32,), width=8)
+            self._after(rays)
             if out is None:
                 from .hip import DeviceArray
                 prim = DeviceArray(m, np.uint32)

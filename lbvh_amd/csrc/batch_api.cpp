@@ -202,7 +202,7 @@ alloc_batch(lbvh_ctx* c, lbvh_batch* b, const std::vector<SortConfig>& cfgs)
   for (auto& r : req) {
     if (!r.bytes)
       continue;
-    hipError_t e = hipMalloc(r.p, r.bytes);
+    hipError_t e = dev_malloc(c->device, r.p, r.bytes);
     if (e != hipSuccess) {
       (void)hipGetLastError();
       return fail(c, LBVH_E_OOM, "device allocation for the batch failed");
@@ -511,7 +511,7 @@ lbvh_build_batch(lbvh_ctx* c, const float* tri, const uint64_t* prim_off, uint32
     return st;
   const uint64_t bytes = prim_off[n_scenes] * 48;
   float* d = nullptr;
-  if (hipMalloc(&d, bytes) != hipSuccess) {
+  if (dev_malloc(c->device, reinterpret_cast<void**>(&d), bytes) != hipSuccess) {
     (void)hipGetLastError();
     return fail(c, LBVH_E_OOM, "device allocation for triangles failed");
   }

@@ -11,6 +11,7 @@
 #include <atomic>
 #include <cstdio>
 #include <cstring>
+#include <mutex>
 #include <new>
 #include <string>
 #include <vector>
@@ -56,7 +57,7 @@ ensure(lbvh_ctx* c, DevBuf& b, uint64_t bytes, bool zero_new)
   }
   uint64_t cap = (bytes + 4095) & ~uint64_t(4095);
   void* p = nullptr;
-  hipError_t e = hipMalloc(&p, cap);
+  hipError_t e = dev_malloc(c->device, &p, cap);
   if (e != hipSuccess || !p) {
     (void)hipGetLastError();
     return fail(c, LBVH_E_OOM, "device allocation of " + std::to_string(cap) + " bytes failed");
@@ -76,6 +77,166 @@ dev_free(void* p)
 {
   if (p)
     (void)hipFree(p);
+}
+
+namespace {
+
+// One device's kept blocks, oldest first (fixed storage: nothing here
+// allocates or throws).
+struct TreePool
+{
+  struct Block
+  {
+    void* p;
+    uint64_t bytes;
+  } kept[kPoolMaxBlocks];
+  size_t count = 0;
+  uint64_t bytes = 0;
+  int contexts = 0;
+
+  Block take(size_t k)
+  {
+    const Block b = kept[k];
+    for (size_t i = k + 1; i < count; i++)
+      kept[i - 1] = kept[i];
+    count--;
+    bytes -= b.bytes;
+    return b;
+  }
+};
+
+constexpr int kPoolMaxDevices = 64;
+std::mutex g_pool_mutex;
+TreePool g_pools[kPoolMaxDevices];
+
+// Gives kept blocks of a device back, oldest first, until at most max_bytes
+// in max_blocks blocks are left.
+void
+pool_trim(int device, uint64_t max_bytes, size_t max_blocks)
+{
+  for (;;) {
+    TreePool::Block b;
+    {
+      std::lock_guard<std::mutex> g(g_pool_mutex);
+      TreePool& t = g_pools[device];
+      if (t.count == 0 || (t.bytes <= max_bytes && t.count <= max_blocks))
+        return;
+      b = t.take(0);
+    }
+    (void)hipFree(b.p); // without the lock: it waits for the device
+  }
+}
+
+bool
+pooled(int device)
+{
+  return device >= 0 && device < kPoolMaxDevices;
+}
+
+// Contexts on a device: the last one to go empties the pool.
+void
+pool_context(int device, int change)
+{
+  if (!pooled(device))
+    return;
+  bool none;
+  {
+    std::lock_guard<std::mutex> g(g_pool_mutex);
+    none = (g_pools[device].contexts += change) == 0;
+  }
+  if (none)
+    pool_trim(device, 0, 0);
+}
+
+bool
+capturing(hipStream_t s)
+{
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &st) != hipSuccess) {
+    (void)hipGetLastError();
+    return true;
+  }
+  return st != hipStreamCaptureStatusNone;
+}
+
+} // namespace
+
+uint64_t
+pool_cached(int device)
+{
+  if (!pooled(device))
+    return 0;
+  std::lock_guard<std::mutex> g(g_pool_mutex);
+  return g_pools[device].bytes;
+}
+
+void
+pool_release(int device)
+{
+  if (pooled(device))
+    pool_trim(device, 0, 0);
+}
+
+hipError_t
+dev_malloc(int device, void** p, uint64_t bytes)
+{
+  hipError_t e = hipMalloc(p, bytes);
+  if (e != hipSuccess && pool_cached(device) > 0) {
+    (void)hipGetLastError();
+    pool_release(device);
+    e = hipMalloc(p, bytes);
+  }
+  return e;
+}
+
+void*
+pool_alloc(int device, uint64_t bytes, hipStream_t stream, uint64_t* held)
+{
+  if (pooled(device) && pool_cached(device) >= bytes && !capturing(stream)) {
+    // the smallest kept block that fits without wasting more than a quarter
+    std::lock_guard<std::mutex> g(g_pool_mutex);
+    TreePool& t = g_pools[device];
+    size_t best = t.count;
+    for (size_t k = 0; k < t.count; k++)
+      if (t.kept[k].bytes >= bytes && t.kept[k].bytes - bytes <= bytes / 4 + (1u << 16) &&
+          (best == t.count || t.kept[k].bytes < t.kept[best].bytes))
+        best = k;
+    if (best < t.count) {
+      const TreePool::Block b = t.take(best);
+      *held = b.bytes;
+      return b.p;
+    }
+  }
+  void* p = nullptr;
+  if (dev_malloc(device, &p, bytes) != hipSuccess || !p) {
+    (void)hipGetLastError();
+    return nullptr;
+  }
+  *held = bytes;
+  return p;
+}
+
+void
+pool_free(int device, void* p, uint64_t held)
+{
+  if (!p)
+    return;
+  if (pooled(device) && held <= kPoolMaxBytes / 2) {
+    // every stream of the device is done with the block, as after hipFree
+    if (hipDeviceSynchronize() == hipSuccess) {
+      pool_trim(device, kPoolMaxBytes - held, kPoolMaxBlocks - 1);
+      std::lock_guard<std::mutex> g(g_pool_mutex);
+      TreePool& t = g_pools[device];
+      if (t.contexts > 0 && t.count < kPoolMaxBlocks && t.bytes + held <= kPoolMaxBytes) {
+        t.kept[t.count++] = TreePool::Block{ p, held };
+        t.bytes += held;
+        return;
+      }
+    } else {
+      (void)hipGetLastError();
+    }
+  }
+  (void)hipFree(p);
 }
 
 lbvh_status
@@ -260,12 +421,9 @@ alloc_bvh(lbvh_ctx* c, lbvh_bvh* b, bool keep_codes)
   for (auto& r : req)
     if (r.bytes)
       total += (r.bytes + 255) & ~uint64_t(255);
-  hipError_t e = hipMalloc(&b->block, total);
-  if (e != hipSuccess || !b->block) {
-    (void)hipGetLastError();
-    b->block = nullptr;
+  b->block = pool_alloc(c->device, total, c->stream, &b->block_held);
+  if (!b->block)
     return fail(c, LBVH_E_OOM, "device allocation for the tree failed");
-  }
   char* at = static_cast<char*>(b->block);
   for (auto& r : req) {
     if (!r.bytes)
@@ -285,9 +443,9 @@ free_bvh(lbvh_bvh* b)
   int cur = 0;
   (void)hipGetDevice(&cur);
   (void)hipSetDevice(b->device);
-  dev_free(b->block); // every tree buffer
+  pool_free(b->device, b->block, b->block_held); // every tree buffer
   if (b->owns_prims)
-    dev_free(b->d_prims);
+    pool_free(b->device, b->d_prims, b->prims_held);
   (void)hipSetDevice(cur);
   delete b;
 }
@@ -615,6 +773,7 @@ lbvh_ctx_create(int device, lbvh_ctx** out)
     return LBVH_E_HIP;
   }
   c->stream = c->own_stream;
+  pool_context(device, 1);
   // set-up of the allocation-free build on this device; if it fails here,
   // that entry point retries on its first call and reports the error
   if (noalloc_init(c) != LBVH_OK)
@@ -640,8 +799,11 @@ lbvh_ctx_destroy(lbvh_ctx* c)
     for (auto& e : es.ev)
       if (e)
         (void)hipEventDestroy(e);
+  if (c->wait_event)
+    (void)hipEventDestroy(c->wait_event);
   if (c->own_stream)
     (void)hipStreamDestroy(c->own_stream);
+  pool_context(c->device, -1);
   delete c;
 }
 
@@ -651,6 +813,32 @@ lbvh_ctx_set_stream(lbvh_ctx* c, void* stream)
   if (!c)
     return LBVH_E_INVALID;
   c->stream = stream ? static_cast<hipStream_t>(stream) : c->own_stream;
+  return LBVH_OK;
+}
+
+lbvh_status
+lbvh_ctx_wait_stream(lbvh_ctx* c, void* stream)
+{
+  if (!c)
+    return LBVH_E_INVALID;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  if (s == c->stream)
+    return LBVH_OK;
+  lbvh_status st = set_device(c);
+  if (st != LBVH_OK)
+    return st;
+  if (capturing(s) || capturing(c->stream))
+    return LBVH_OK;
+  hipError_t e = hipStreamQuery(s); // idle, as for inputs that are ready: nothing to wait for
+  if (e == hipSuccess)
+    return LBVH_OK;
+  (void)hipGetLastError();
+  if (e != hipErrorNotReady)
+    return hip_fail(c, e, "hipStreamQuery");
+  if (!c->wait_event)
+    HIP_TRY(c, hipEventCreateWithFlags(&c->wait_event, hipEventDisableTiming));
+  HIP_TRY(c, hipEventRecord(c->wait_event, s));
+  HIP_TRY(c, hipStreamWaitEvent(c->stream, c->wait_event, 0));
   return LBVH_OK;
 }
 
@@ -796,22 +984,22 @@ build_host(lbvh_ctx* c, const float* host, int kind, uint64_t n, const lbvh_buil
   if (st != LBVH_OK)
     return st;
   const uint64_t bytes = n * (kind == 0 ? 48 : 24);
-  float* d = nullptr;
-  if (hipMalloc(&d, bytes) != hipSuccess) {
-    (void)hipGetLastError();
+  uint64_t held = 0;
+  float* d = static_cast<float*>(pool_alloc(c->device, bytes, c->stream, &held));
+  if (!d)
     return fail(c, LBVH_E_OOM, "device allocation for primitives failed");
-  }
   hipError_t e = hipMemcpyAsync(d, host, bytes, hipMemcpyHostToDevice, c->stream);
   if (e != hipSuccess) {
-    dev_free(d);
+    pool_free(c->device, d, held);
     return hip_fail(c, e, "hipMemcpyAsync");
   }
   st = build_common(c, d, kind, n, opts, true, out);
   if (st != LBVH_OK) {
     (void)hipStreamSynchronize(c->stream);
-    dev_free(d);
+    pool_free(c->device, d, held);
     return st;
   }
+  (*out)->prims_held = held;
   st = sync_and_check(c);
   if (st != LBVH_OK) {
     free_bvh(*out);
@@ -896,11 +1084,10 @@ lbvh_refit_triangles(lbvh_ctx* c, lbvh_bvh* b, const float* tri)
   if (st != LBVH_OK)
     return st;
   if (!b->owns_prims) {
-    float* d = nullptr;
-    if (hipMalloc(&d, b->n * 48) != hipSuccess) {
-      (void)hipGetLastError();
+    float* d =
+      static_cast<float*>(pool_alloc(c->device, b->n * 48, c->stream, &b->prims_held));
+    if (!d)
       return fail(c, LBVH_E_OOM, "device allocation for primitives failed");
-    }
     b->d_prims = d;
     b->owns_prims = true;
     b->bytes += b->n * 48;

@@ -61,6 +61,7 @@ struct lbvh_ctx
   int device = 0;
   hipStream_t own_stream = nullptr;
   hipStream_t stream = nullptr;
+  hipEvent_t wait_event = nullptr; // lbvh_ctx_wait_stream
   int timing = 0; // 0 off, 1 per phase, 2 per call
   std::vector<lbvh_rt::EventSet> sets; // pool; sets[0..used) belong to timed calls
   size_t used = 0;
@@ -102,6 +103,7 @@ struct lbvh_bvh
   uint32_t* d_leafprim = nullptr; // primitive of each leaf position (primitive-id leaves)
   uint32_t* d_other_end = nullptr; // other end of each internal node's leaf range
   void* block = nullptr;           // the one allocation holding every buffer above
+  uint64_t block_held = 0, prims_held = 0; // pool bytes of block and of owned primitives
   uint64_t bytes = 0;
   lbvh_eng::SortConfig sort;       // the sort configuration the build used
   uint64_t id = 0;                 // unique per tree in the process (refit caches)
@@ -130,6 +132,24 @@ constexpr uint64_t kMaxRaysPerCall = (uint64_t(1) << 31) - 1;
 lbvh_status hip_fail(lbvh_ctx* c, hipError_t e, const char* what);
 lbvh_status ensure(lbvh_ctx* c, DevBuf& b, uint64_t bytes, bool zero_new = false);
 void dev_free(void* p);
+// Device memory of trees and of the primitives they own.  A freed block is
+// kept for the next tree of about its size: mapping and unmapping cost more
+// than the build (hipFree of a 16M-primitive tree: 20 ms).  At most
+// kPoolMaxBytes and kPoolMaxBlocks are kept per device, the oldest given back
+// first; all of it when the device's last context goes, or when an
+// allocation of the engine fails.  pool_free waits for the device first, as
+// hipFree does, so a kept block has no user left on any stream; a block
+// carries no contents from one tree to the next.  Safe from any thread.
+constexpr uint64_t kPoolMaxBytes = uint64_t(4) << 30;
+constexpr size_t kPoolMaxBlocks = 64;
+// stream: the caller's; while it is being captured the pool is left alone.
+// *held: the block's bytes, for pool_free.
+void* pool_alloc(int device, uint64_t bytes, hipStream_t stream, uint64_t* held);
+void pool_free(int device, void* p, uint64_t held);
+uint64_t pool_cached(int device);
+void pool_release(int device);
+// hipMalloc; what the pool keeps is given back and the call repeated if it fails.
+hipError_t dev_malloc(int device, void** p, uint64_t bytes);
 lbvh_status set_device(lbvh_ctx* c);
 // Finds this device's copy of the allocation-free build's scratch array (the
 // device must be current; once per device).

@@ -274,11 +274,13 @@ destroy_scene(Scene* sc)
 bool
 make_room(lbvh_server* s, uint64_t need)
 {
-  if (s->mem_used + s->dev_pool.cached + need <= s->mem_cap)
+  const uint64_t trees = pool_cached(s->device);
+  if (s->mem_used + s->dev_pool.cached + trees + need <= s->mem_cap)
     return true;
-  // cached pool buffers go first
-  if (s->dev_pool.cached) {
+  // cached pool buffers go first, those kept of freed trees among them
+  if (s->dev_pool.cached || trees) {
     s->dev_pool.release_all();
+    pool_release(s->device);
     if (s->mem_used + need <= s->mem_cap)
       return true;
   }
@@ -301,6 +303,9 @@ make_room(lbvh_server* s, uint64_t need)
     destroy_scene(sc);
     s->stats.evictions++;
   }
+  // the evicted trees' memory stays kept for the next trees only under the cap
+  if (s->mem_used + pool_cached(s->device) + need > s->mem_cap)
+    pool_release(s->device);
   return s->mem_used + need <= s->mem_cap;
 }
 
@@ -432,7 +437,7 @@ start(lbvh_server* s, Req* q, Scene* sc)
       sc->d_tri = const_cast<float*>(tri_src);
       sc->owns_tri = false;
     } else {
-      if (hipMalloc(&sc->d_tri, ntri * 48) != hipSuccess) {
+      if (dev_malloc(s->device, reinterpret_cast<void**>(&sc->d_tri), ntri * 48) != hipSuccess) {
         (void)hipGetLastError();
         return bad(LBVH_E_OOM, "scene allocation failed");
       }
@@ -468,7 +473,7 @@ start(lbvh_server* s, Req* q, Scene* sc)
         // host data for a scene whose triangles are borrowed device memory:
         // borrowed memory is only read, so the scene takes a buffer of its own
         float* own = nullptr;
-        if (hipMalloc(&own, ntri * 48) != hipSuccess) {
+        if (dev_malloc(s->device, reinterpret_cast<void**>(&own), ntri * 48) != hipSuccess) {
           (void)hipGetLastError();
           return bad(LBVH_E_OOM, "scene allocation failed");
         }

@@ -437,6 +437,53 @@ def test_torch_tensors_share_the_runtime(tmp_path):
     assert "torch interop ok" in r.stdout
 
 
+TORCH_ORDER = r"""
+import sys, numpy as np
+import torch
+sys.path.insert(0, %r)
+import lbvh_amd, oracle
+from lbvh_amd import workload as W
+v, tri = W.scene_uniform(1, 3000, 0.02)
+rays = W.primary_rays(32, 32)
+on, _, _, _ = oracle.build(tri, 30, 1)
+op, ot, _ = oracle.trace(on, tri, rays, 0)
+ctx = lbvh_amd.Context(0)
+src_tri, src_rays = torch.from_numpy(tri).cuda(), torch.from_numpy(rays).cuda()
+big = torch.randn(6144, 6144, device="cuda")
+for stream in (torch.cuda.default_stream(), torch.cuda.Stream()):
+    for k in range(3):
+        d_tri, d_rays = torch.zeros_like(src_tri), torch.zeros_like(src_rays)
+        torch.cuda.synchronize()
+        with torch.cuda.stream(stream):
+            for _ in range(4):
+                y = big @ big  # a few ms before the inputs are written
+            d_tri.copy_(src_tri)
+            b = ctx.build_triangles(d_tri, code_bits=30, leaf_order=1)
+            for _ in range(4):
+                y = big @ big
+            d_rays.copy_(src_rays)
+            prim, t, uv = ctx.trace(b, d_rays, 0)
+        ctx.synchronize()
+        assert b.nodes().tobytes() == on.tobytes()
+        assert np.array_equal(prim.numpy(), op)
+        assert np.array_equal(t.numpy().view(np.uint32), ot.view(np.uint32))
+        torch.cuda.synchronize()
+print("torch order ok")
+"""
+
+
+def test_torch_inputs_still_being_written_are_waited_for():
+    """Calls on the context's own stream with torch tensors start after the
+    work of torch's current stream, the default one or another."""
+    import subprocess
+    import sys
+    from conftest import ROOT
+    r = subprocess.run([sys.executable, "-c", TORCH_ORDER % ROOT], capture_output=True, text=True,
+                       timeout=180)
+    assert r.returncode == 0, r.stdout + r.stderr
+    assert "torch order ok" in r.stdout
+
+
 def test_cpp_dropin_conformance(tmp_path):
     """The C++ drop-in header (include/lbvh_mi355x.hpp) used with the
     reference's call shapes: builder over triangles and over a user primitive
@@ -493,6 +540,48 @@ def test_aabb_build_equals_triangle_build(ctx):
     a = ctx.build_triangles(tri, code_bits=30, leaf_order=1)
     b = ctx.build_aabbs(boxes, code_bits=30, leaf_order=1)
     assert a.nodes().tobytes() == b.nodes().tobytes()
+
+
+@pytest.mark.parametrize("leaf", [0, 1])
+def test_tree_memory_reused_across_threads_and_contexts(leaf):
+    """Freed trees' memory goes to the next trees of about their size.  Four
+    threads with a context each build, trace and free trees whose sizes hand
+    the blocks around; every node array and hit equals the oracle's, and a
+    tree outlives the context that built it."""
+    import threading
+    sizes = [2, 3000, 2900, 4097, 70001, 3500, 65536, 2]
+    rays = W.primary_rays(12, 8)
+    want = {}
+    for n in set(sizes):
+        tri = W.make_triangles(W.cluster_vertices(5000 + n, n))
+        nodes, _, _, _ = oracle.build(tri, 30, leaf)
+        want[n] = (tri, nodes, oracle.trace(nodes, tri, rays, 0)) if leaf else (tri, nodes, None)
+    bad = []
+
+    def work(k):
+        c = lbvh_amd.Context(0)
+        left = None
+        for r in range(3):
+            for n in sizes[k:] + sizes[:k]:
+                tri, nodes, hits = want[n]
+                bvh = c.build_triangles(tri, code_bits=30, leaf_order=leaf)
+                if bvh.nodes().tobytes() != nodes.tobytes():
+                    bad.append((k, r, n, "nodes"))
+                if hits is not None:
+                    p, t, _ = c.trace(bvh, rays, 0)
+                    if not (np.array_equal(p, hits[0]) and
+                            np.array_equal(t.view(np.uint32), hits[1].view(np.uint32))):
+                        bad.append((k, r, n, "hits"))
+                left = bvh # the previous one is freed here
+        c.close()
+        left.destroy()
+
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not bad, bad
 
 
 def test_phase_timing_reports_four_phases(ctx):
