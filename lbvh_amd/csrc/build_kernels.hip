@@ -36,21 +36,6 @@ constexpr uint32_t kLinkIndex = kLinkSibLeaf - 1;
 // partials (no ticket, no drain: a workgroup exits as soon as its stores are
 // issued).
 
-__device__ __forceinline__ void
-wave_reduce_box(float lo[3], float hi[3])
-{
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) {
-#pragma unroll
-    for (int k = 0; k < 3; k++) {
-      float ol = __shfl_down(lo[k], off, kWave);
-      float oh = __shfl_down(hi[k], off, kWave);
-      lo[k] = std_min(lo[k], ol);
-      hi[k] = std_max(hi[k], oh);
-    }
-  }
-}
-
 // Reduces one box per thread to thread 0 of the workgroup.
 __device__ __forceinline__ void
 block_reduce_box(float lo[3], float hi[3], float (*s_box)[6])
@@ -141,47 +126,6 @@ k_centroid_bounds(const float* __restrict__ prims, uint64_t n,
 // passes - 1 (those whose global histogram the sort reads) in LDS and adds
 // its nonzero counts to the global histogram with atomics.
 
-__device__ __forceinline__ uint32_t
-expand10(uint32_t n)
-{
-  n = (n | (n << 16)) & 0x030000ffu;
-  n = (n | (n << 8)) & 0x0300f00fu;
-  n = (n | (n << 4)) & 0x030c30c3u;
-  n = (n | (n << 2)) & 0x09249249u;
-  return n;
-}
-
-__device__ __forceinline__ uint64_t
-expand20(uint64_t n)
-{
-  n = (n | n << 32) & 0x001f00000000ffffull;
-  n = (n | n << 16) & 0x001f0000ff0000ffull;
-  n = (n | n << 8) & 0x100f00f00f00f00full;
-  n = (n | n << 4) & 0x10c30c30c30c30c3ull;
-  n = (n | n << 2) & 0x1249249249249249ull;
-  return n;
-}
-
-template<typename KeyT>
-__device__ __forceinline__ KeyT
-encode(float qx, float qy, float qz);
-
-template<>
-__device__ __forceinline__ uint32_t
-encode<uint32_t>(float qx, float qy, float qz)
-{
-  uint32_t x = uint32_t(qx), y = uint32_t(qy), z = uint32_t(qz);
-  return (expand10(x) << 2) | (expand10(y) << 1) | expand10(z);
-}
-
-template<>
-__device__ __forceinline__ uint64_t
-encode<uint64_t>(float qx, float qy, float qz)
-{
-  uint64_t x = uint64_t(qx), y = uint64_t(qy), z = uint64_t(qz);
-  return (expand20(x) << 2) | (expand20(y) << 1) | expand20(z);
-}
-
 constexpr int kHistMaxWords = 8192; // passes * radix, 32 KiB of LDS
 constexpr int kEncodeUnroll = 4;
 // 1,024 threads: one encode workgroup per sort chunk leaves a single
@@ -255,15 +199,8 @@ k_encode(const float* __restrict__ cx, const float* __restrict__ cy,
       bounds_out[3 + k] = bhi[k];
     }
   }
-  const float dom = sizeof(KeyT) == 4 ? 1024.0f : 1048576.0f;
-  float bmin[3], scale[3];
-#pragma unroll
-  for (int k = 0; k < 3; k++) {
-    bmin[k] = blo[k];
-    float ext = bhi[k] - bmin[k];
-    float den = ext + 1.0f;
-    scale[k] = dom / den;
-  }
+  float scale[3];
+  morton_scale<KeyT>(blo, bhi, scale);
   const KeyT mask = KeyT(radix - 1);
   for (uint64_t i0 = first; i0 < limit; i0 += stride * kEncodeUnroll) {
     // unconditional loads (past the end: the last centre, unused), all in
@@ -282,13 +219,7 @@ k_encode(const float* __restrict__ cx, const float* __restrict__ cy,
       uint64_t i = i0 + u * stride;
       if (i >= limit)
         continue;
-      float dx = x[u] - bmin[0];
-      float dy = y[u] - bmin[1];
-      float dz = z[u] - bmin[2];
-      float qx = dx * scale[0];
-      float qy = dy * scale[1];
-      float qz = dz * scale[2];
-      KeyT code = encode<KeyT>(qx, qy, qz);
+      const KeyT code = morton_code<KeyT>(x[u], y[u], z[u], blo, scale);
       codes[i] = code;
       for (int p = first_pass; p < passes; p++) {
         uint32_t d = uint32_t((code >> (p * digit_bits)) & mask);

@@ -383,7 +383,7 @@ valid_sort_config(const SortConfig& c, int key_bits)
 {
   if (c.strategy < 0 || c.strategy > 2)
     return false;
-  if (c.strategy == 2 && (c.global_digits < 1 ||
+  if (c.strategy == 2 && (c.global_digits < 0 ||
                           c.global_digits >= sort_passes(key_bits, c.digit_bits)))
     return false;
   if (c.strategy >= 1)
@@ -495,17 +495,24 @@ reserve_build(lbvh_ctx* c, uint64_t n, int code_bits, const SortConfig& cfg, boo
 SortConfig
 untuned_sort(int key_bits, uint64_t n)
 {
-  SortConfig c = default_sort();
-  if (n < kTuneMinPrims)
-    return c;
-  // the hybrid at 10-bit digits and 4,096-key tiles: the tuner's pick at 1M
-  // and 16M 63-bit keys and for batches
+  // the hybrid at 10-bit digits.  From 65,536 keys 4,096-key tiles: the
+  // tuner's pick at 1M and 16M 63-bit keys and for batches.  Below, where the
+  // launches are what a sort costs, one global digit and the smaller tile
+  // (more workgroups); up to kHybridTileCap keys no global digit at all.
+  // Device time of a build, us, against reduce-then-scan over every digit:
+  // 4,096 triangles 53 / 112 (30-bit), 54 / 197 (63-bit); 16,384 uniform 75 /
+  // 119, 77 / 210; 65,535 uniform 90 / 135, 92 / 228, clustered (a few full
+  // buckets) 122 / 134, 131 / 226.  Onesweep is faster on the last (98), but
+  // its state belongs to one build: a captured one could not be replayed.
   SortConfig h;
   h.digit_bits = 10;
-  h.items = 16;
+  h.items = n < kTuneMinPrims ? 8 : 16;
   h.strategy = 2;
-  h.global_digits = hybrid_global_digits(key_bits, h.digit_bits, n);
-  return h.global_digits <= sort_passes(key_bits, h.digit_bits) - 2 ? h : c;
+  if (n < kTuneMinPrims)
+    h.global_digits = n <= kHybridTileCap ? 0 : 1;
+  else
+    h.global_digits = hybrid_global_digits(key_bits, h.digit_bits, n);
+  return h.global_digits <= sort_passes(key_bits, h.digit_bits) - 2 ? h : default_sort();
 }
 
 // The sort configuration of a single-scene build: explicit options, else
@@ -598,6 +605,8 @@ build_common(lbvh_ctx* c, const float* d_prims, int kind, uint64_t n,
   // reduce-then-scan and hybrid sorts: the encode counts the first pass's
   // chunks itself (one encode workgroup per chunk)
   const bool chunked = cfg.strategy == 1 || cfg.strategy == 2;
+  // ... and one workgroup does it all for the fewest primitives
+  const bool one_wg = cfg.strategy == 2 && cfg.global_digits == 0;
   const uint32_t rts_g = chunked ? rts_groups(n, cfg, nullptr) : 0u;
   const uint32_t small_words = kSmallHist + uint32_t(passes) * radix;
   const uint64_t sw = sort_status_words(n, cfg);
@@ -645,11 +654,15 @@ build_common(lbvh_ctx* c, const float* d_prims, int kind, uint64_t n,
 
   begin_timed(c, 1);
   record(c, 0);
-  hipError_t e = launch_centroid_bounds(d_prims, kind, n, cent, cent + n, cent + 2 * n,
-                                        static_cast<float*>(c->partials.p),
-                                        small + kSmallTickets, small_words - kSmallTickets,
-                                        c->stream);
-  if (e == hipSuccess)
+  hipError_t e = hipSuccess;
+  if (one_wg)
+    e = launch_small_sort(key_bits, d_prims, kind, n, b->d_bounds, c->keys_b.p,
+                          with_ids ? static_cast<uint32_t*>(c->ids_b.p) : nullptr, c->stream);
+  else
+    e = launch_centroid_bounds(d_prims, kind, n, cent, cent + n, cent + 2 * n,
+                               static_cast<float*>(c->partials.p), small + kSmallTickets,
+                               small_words - kSmallTickets, c->stream);
+  if (e == hipSuccess && !one_wg)
     e = launch_encode(opts.code_bits, cent, cent + n, cent + 2 * n, n,
                       static_cast<const float*>(c->partials.p), b->d_bounds,
                       c->keys_a.p, ws.hist,
@@ -657,8 +670,8 @@ build_common(lbvh_ctx* c, const float* d_prims, int kind, uint64_t n,
                       chunked ? ws.counts : nullptr, rts_g,
                       chunked ? rts_chunk_keys(n, cfg) : 0, c->stream);
   record(c, 1);
-  bool in_b = false;
-  if (e == hipSuccess)
+  bool in_b = one_wg;
+  if (e == hipSuccess && !one_wg)
     e = launch_sort(key_bits, int(kw), n, c->keys_a.p, c->keys_b.p,
                     with_ids ? static_cast<uint32_t*>(c->ids_a.p) : nullptr,
                     with_ids ? static_cast<uint32_t*>(c->ids_b.p) : nullptr, cfg, ws, epoch,

@@ -31,7 +31,7 @@ choose_sort_f64(lbvh_ctx* c, const double* d_boxes, uint64_t n, const lbvh_build
     *cfg = sort_from_opts(opts, key_bits, n);
     return LBVH_OK;
   }
-  *cfg = default_sort();
+  *cfg = n < kTuneMinPrims ? untuned_sort(key_bits, n) : default_sort();
   if (!c->autotune || n < kTuneMinPrims)
     return LBVH_OK;
   const uint64_t key = tune_key(false, key_bits, n, 64);
@@ -74,7 +74,9 @@ queue_f64_build(lbvh_ctx* c, const double* d_boxes, uint64_t n, const lbvh_build
   if (!valid_sort_config(cfg, key_bits))
     return fail(c, LBVH_E_INVALID, "unsupported sort digit width / tile");
   const int passes = sort_passes(key_bits, cfg.digit_bits);
-  const int first_pass = cfg.strategy == 2 ? passes - cfg.global_digits : 0;
+  // the passes whose histogram the encode counts: at least one
+  const int first_pass =
+    cfg.strategy == 2 ? passes - (cfg.global_digits > 0 ? cfg.global_digits : 1) : 0;
   const uint32_t radix = 1u << cfg.digit_bits;
   const bool with_ids = opts.leaf_order == LBVH_LEAF_PRIMITIVE_ID;
 

@@ -252,4 +252,94 @@ popc64(uint64_t x)
   return __popcll(x);
 }
 
+// Union over the wave of one box per lane, in lane 0.
+__device__ __forceinline__ void
+wave_reduce_box(float lo[3], float hi[3])
+{
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+      float ol = __shfl_down(lo[k], off, kWave);
+      float oh = __shfl_down(hi[k], off, kWave);
+      lo[k] = std_min(lo[k], ol);
+      hi[k] = std_max(hi[k], oh);
+    }
+  }
+}
+
+// ---- Morton codes ------------------------------------------------------------
+// morton_curve_kernel (lbvh.h:1432-1473): scale = D / (extent + 1) with
+// D = 1024 (morton_domain<4>) or 2^20 (morton_domain<8>); q = trunc((c - min)
+// * scale); code = expand(qx) << 2 | expand(qy) << 1 | expand(qz) with the
+// magic-mask expansions of morton_encoder<4>/<8> (lbvh.h:1352-1358,
+// 1377-1385).  The 63-bit variant applies morton_encoder<8> to FP32 centres.
+
+__device__ __forceinline__ uint32_t
+expand10(uint32_t n)
+{
+  n = (n | (n << 16)) & 0x030000ffu;
+  n = (n | (n << 8)) & 0x0300f00fu;
+  n = (n | (n << 4)) & 0x030c30c3u;
+  n = (n | (n << 2)) & 0x09249249u;
+  return n;
+}
+
+__device__ __forceinline__ uint64_t
+expand20(uint64_t n)
+{
+  n = (n | n << 32) & 0x001f00000000ffffull;
+  n = (n | n << 16) & 0x001f0000ff0000ffull;
+  n = (n | n << 8) & 0x100f00f00f00f00full;
+  n = (n | n << 4) & 0x10c30c30c30c30c3ull;
+  n = (n | n << 2) & 0x1249249249249249ull;
+  return n;
+}
+
+template<typename KeyT>
+__device__ __forceinline__ KeyT
+encode(float qx, float qy, float qz);
+
+template<>
+__device__ __forceinline__ uint32_t
+encode<uint32_t>(float qx, float qy, float qz)
+{
+  uint32_t x = uint32_t(qx), y = uint32_t(qy), z = uint32_t(qz);
+  return (expand10(x) << 2) | (expand10(y) << 1) | expand10(z);
+}
+
+template<>
+__device__ __forceinline__ uint64_t
+encode<uint64_t>(float qx, float qy, float qz)
+{
+  uint64_t x = uint64_t(qx), y = uint64_t(qy), z = uint64_t(qz);
+  return (expand20(x) << 2) | (expand20(y) << 1) | expand20(z);
+}
+
+template<typename KeyT>
+__device__ __forceinline__ void
+morton_scale(const float lo[3], const float hi[3], float scale[3])
+{
+  const float dom = sizeof(KeyT) == 4 ? 1024.0f : 1048576.0f;
+#pragma unroll
+  for (int k = 0; k < 3; k++) {
+    float ext = hi[k] - lo[k];
+    float den = ext + 1.0f;
+    scale[k] = dom / den;
+  }
+}
+
+template<typename KeyT>
+__device__ __forceinline__ KeyT
+morton_code(float x, float y, float z, const float lo[3], const float scale[3])
+{
+  float dx = x - lo[0];
+  float dy = y - lo[1];
+  float dz = z - lo[2];
+  float qx = dx * scale[0];
+  float qy = dy * scale[1];
+  float qz = dz * scale[2];
+  return encode<KeyT>(qx, qy, qz);
+}
+
 } // namespace lbvh_dev

@@ -17,7 +17,8 @@ struct SortConfig
                       // 2: hybrid (top digits by reduce-then-scan, then every
                       //    run of equal top bits sorted by the full key in LDS)
   int groups = 0;     // reduce-then-scan: target number of chunks (0 = about two tiles each, 512-2,048)
-  int global_digits = 0; // hybrid: digits sorted by global passes (the top ones)
+  int global_digits = 0; // hybrid: digits sorted by global passes (the top ones); 0:
+                         // at most kHybridTileCap keys, in the LDS of one workgroup
 };
 
 // Hybrid strategy: keys per workgroup of the LDS sort (nominal and maximum).
@@ -90,6 +91,11 @@ hipError_t launch_sort(int key_bits, int key_bytes, uint64_t n, void* keys_a, vo
                        uint32_t* ids_a,
                        uint32_t* ids_b, const SortConfig& cfg, const SortWorkspace& ws,
                        uint32_t epoch, bool* result_in_b, hipStream_t s);
+// The sorted codes and ids (ids may be null) of 2 .. kHybridTileCap
+// primitives, with their centroid bounds (6 floats), in one launch: bounds,
+// encode and sort of a build with SortConfig::global_digits 0.
+hipError_t launch_small_sort(int key_bits, const float* prims, int kind, uint64_t n,
+                             float* bounds, void* keys, uint32_t* ids, hipStream_t s);
 uint64_t sort_status_words(uint64_t n, const SortConfig& cfg);
 // 32-bit words of ws.counts the sort needs for n keys.
 uint64_t sort_counts_words(uint64_t n, const SortConfig& cfg);

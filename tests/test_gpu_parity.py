@@ -127,6 +127,40 @@ def test_build_matches_oracle_ragged(ctx, n, bits, leaf):
     assert np.array_equal(ids, oids)
 
 
+@pytest.mark.parametrize("n", [2, 64, 65, 511, 513, 2049, 4095, 4096, 4097, 20001, 65535])
+@pytest.mark.parametrize("dist", ["uniform", "clustered", "equal", "two"])
+def test_small_builds_match_oracle(ctx, n, dist):
+    """Builds below 65,536 primitives sort in one workgroup (up to 4,096) or
+    with one global digit: wave and block remainders, runs of a few dense
+    spots, one code for everything, two far groups; triangles and boxes, both
+    code widths and leaf orders."""
+    rng = np.random.default_rng(n)
+    if dist == "uniform":
+        v = W.uniform_vertices(n, n, 0.01)
+    elif dist == "clustered":
+        v = W.cluster_vertices(n, n, 5, 0.0005, 0.0005)
+    else:
+        c = np.zeros((n, 1), np.float32) if dist == "equal" else (rng.integers(0, 2, (n, 1)) * 100.0)
+        v = (np.tile(rng.random((1, 9)), (n, 1)) + c).astype(np.float32)
+    tri = W.make_triangles(v)
+    for bits, leaf in VARIANTS:
+        bvh = ctx.build_triangles(tri, code_bits=bits, leaf_order=leaf, keep_codes=True)
+        on, ob, osc, oids = oracle.build(tri, bits, leaf)
+        sc, ids, bounds = bvh.codes()
+        assert np.array_equal(sc, osc)
+        assert np.array_equal(ids, oids)
+        assert np.array_equal(bounds, np.asarray(ob, np.float32).reshape(-1))
+        assert bvh.nodes().tobytes() == on.tobytes()
+        bvh.destroy()
+    p0, p1, p2 = tri[:, 0:3], tri[:, 0:3] - tri[:, 3:6], tri[:, 0:3] + tri[:, 6:9]
+    boxes = np.concatenate([np.minimum(np.minimum(p0, p1), p2), np.maximum(np.maximum(p0, p1), p2)],
+                           axis=1)
+    for bits, leaf in VARIANTS:
+        bvh = ctx.build_aabbs(boxes, code_bits=bits, leaf_order=leaf)
+        assert bvh.nodes().tobytes() == oracle.build(tri, bits, leaf)[0].tobytes()
+        bvh.destroy()
+
+
 @pytest.mark.parametrize("slots", ["1", "200"])
 @pytest.mark.parametrize("n", [9000, 70001, 300001])
 @pytest.mark.parametrize("bits,leaf", [(30, 0), (63, 1)], ids=["b30_ref", "b63_pid"])
