@@ -49,6 +49,54 @@ status_ready(uint64_t s, uint32_t epoch)
   return uint32_t(s >> 40) == (epoch & 0xffffffu) && ((s >> 32) & 0xff) != 0;
 }
 
+// Steps B .. RBITS - 1 of the digit matching that `vary` holds: of the lanes
+// lo, hi, those whose bit B of d is this lane's (a & ~(m ^ s): s this lane's
+// bit in every bit, m the ballot; one three-input operation each half).  The
+// bit is extracted in assembly because the compiler turns the builtin back
+// into two shifts.  Lanes that hold no key have to be out of lo, hi from the
+// start; their bits then do not matter.
+template<int B, int RBITS>
+__device__ __forceinline__ void
+match_bits(uint32_t d, uint32_t vary, uint32_t& lo, uint32_t& hi)
+{
+  if constexpr (B < RBITS) {
+    if ((vary >> B) & 1u) { // uniform
+      int32_t s;
+      asm("v_bfe_i32 %0, %1, %2, 1" : "=v"(s) : "v"(d), "n"(B));
+      const uint64_t m = ballot(s != 0);
+      lo = uint32_t(__builtin_amdgcn_bitop3_b32(int(lo), int(uint32_t(m)), s, 0x90));
+      hi = uint32_t(__builtin_amdgcn_bitop3_b32(int(hi), int(uint32_t(m >> 32)), s, 0x90));
+    }
+    match_bits<B + 1, RBITS>(d, vary, lo, hi);
+  }
+}
+
+// The wave's lanes that hold a key (valid) of digit d, among RBITS-bit
+// digits, and the number of them below this lane.  The ranking kernels are
+// bound by these instructions: RBITS x 4 and a few.  Written with ballots of
+// (valid && bit) and 64-bit selects they were 128 for 8 bits.  16M 30-bit
+// keys: downsweep 58 -> 47 us, upsweep 40 -> 25 us a pass; 15.7M batch keys,
+// 10-bit downsweep 146 -> 117 us.
+struct Peers
+{
+  uint32_t lo, hi;
+  __device__ __forceinline__ uint32_t below() const
+  {
+    return __builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, 0u));
+  }
+  __device__ __forceinline__ uint32_t count() const { return uint32_t(__popc(lo) + __popc(hi)); }
+};
+
+template<int RBITS>
+__device__ __forceinline__ Peers
+match_digit(uint32_t d, bool valid)
+{
+  const uint64_t v = ballot(valid);
+  Peers p = { uint32_t(v), uint32_t(v >> 32) };
+  match_bits<0, RBITS>(d, ~0u, p.lo, p.hi);
+  return p;
+}
+
 // Exclusive scan of one value per thread across the workgroup.
 __device__ __forceinline__ uint32_t
 block_exclusive_scan(uint32_t x, uint32_t* s_tmp, uint32_t* total)
@@ -124,23 +172,16 @@ k_onesweep(const KeyT* __restrict__ kin, KeyT* __restrict__ kout,
   }
 
   // ---- stable ranking within the wave ----
-  const uint64_t lt = lanemask_lt();
 #pragma unroll
   for (int j = 0; j < ITEMS; j++) {
     const uint32_t idx = base + uint32_t(j) * kWave;
     const bool valid = idx < n;
     const uint32_t d = uint32_t((key[j] >> shift) & dmask);
-    uint64_t peers = ballot(valid);
-#pragma unroll
-    for (int b = 0; b < RBITS; b++) {
-      const bool bit = (d >> b) & 1u;
-      const uint64_t m = ballot(valid && bit);
-      peers &= bit ? m : ~m;
-    }
+    const Peers peers = match_digit<RBITS>(d, valid);
     uint32_t r = 0;
     if (valid) {
-      const uint32_t below = uint32_t(popc64(peers & lt));
-      const uint32_t cnt = uint32_t(popc64(peers));
+      const uint32_t below = peers.below();
+      const uint32_t cnt = peers.count();
       const uint32_t wbase = s_wcnt[w][d];
       r = wbase + below;
       if (below == 0)
@@ -305,7 +346,6 @@ k_rts_upsweep(const KeyT* __restrict__ keys, uint32_t n, int shift, uint32_t chu
   uint32_t begin, end;
   chunk_range(g, n, chunk_keys, chunks, &begin, &end);
   const KeyT dmask = KeyT(RADIX - 1);
-  const uint64_t lt = lanemask_lt();
   for (uint32_t base = begin; base < end; base += kSortBlock * kUpsweepUnroll) {
     KeyT k[kUpsweepUnroll];
 #pragma unroll
@@ -318,15 +358,9 @@ k_rts_upsweep(const KeyT* __restrict__ keys, uint32_t n, int shift, uint32_t chu
       const uint32_t i = base + u * kSortBlock + tid;
       const bool valid = i < end;
       const uint32_t d = uint32_t((k[u] >> shift) & dmask);
-      uint64_t peers = ballot(valid);
-#pragma unroll
-      for (int b = 0; b < RBITS; b++) {
-        const bool bit = (d >> b) & 1u;
-        const uint64_t m = ballot(valid && bit);
-        peers &= bit ? m : ~m;
-      }
-      if (valid && (peers & lt) == 0)
-        s_h[w][d] += uint32_t(popc64(peers));
+      const Peers peers = match_digit<RBITS>(d, valid);
+      if (valid && peers.below() == 0)
+        s_h[w][d] += peers.count();
     }
   }
   __syncthreads();
@@ -450,7 +484,6 @@ k_rts_downsweep(const KeyT* __restrict__ kin, KeyT* __restrict__ kout,
     const size_t d = size_t(tid) * DPT + dd;
     running[dd] = offsets[chunks ? size_t(g) * RADIX + d : d * groups + g];
   }
-  const uint64_t lt = lanemask_lt();
   uint32_t cbegin, cend;
   chunk_range(g, n, uint64_t(chunk_tiles) * TILE, chunks, &cbegin, &cend);
 
@@ -476,17 +509,11 @@ k_rts_downsweep(const KeyT* __restrict__ kin, KeyT* __restrict__ kout,
       const uint32_t idx = base + uint32_t(j) * kWave;
       const bool valid = idx < cend;
       const uint32_t d = uint32_t((key[j] >> shift) & dmask);
-      uint64_t peers = ballot(valid);
-#pragma unroll
-      for (int b = 0; b < RBITS; b++) {
-        const bool bit = (d >> b) & 1u;
-        const uint64_t m = ballot(valid && bit);
-        peers &= bit ? m : ~m;
-      }
+      const Peers peers = match_digit<RBITS>(d, valid);
       uint32_t r = 0;
       if (valid) {
-        const uint32_t below = uint32_t(popc64(peers & lt));
-        const uint32_t cnt = uint32_t(popc64(peers));
+        const uint32_t below = peers.below();
+        const uint32_t cnt = peers.count();
         const uint32_t wbase = s_wcnt[w][d];
         r = wbase + below;
         if (below == 0)
@@ -733,26 +760,19 @@ rank_digits(const uint32_t (&dg)[kTileItems], int ipw, uint32_t lbase, uint32_t 
             uint32_t (&rank)[kTileItems], uint32_t (*s_wcnt)[kTileRadix])
 {
   const int w = threadIdx.x / kWave;
-  const uint64_t lt = lanemask_lt();
 #pragma unroll
   for (int j = 0; j < kTileItems; j++) {
     if (j >= ipw)
       break; // block-uniform
     const bool valid = lbase + uint32_t(j) * kWave < m;
     const uint32_t d = dg[j];
-    uint64_t peers = ballot(valid);
-#pragma unroll
-    for (int b = 0; b < 8; b++) {
-      if ((dvar >> b) & 1u) {
-        const bool bit = (d >> b) & 1u;
-        const uint64_t mm = ballot(valid && bit);
-        peers &= bit ? mm : ~mm;
-      }
-    }
+    const uint64_t vm = ballot(valid);
+    Peers peers = { uint32_t(vm), uint32_t(vm >> 32) };
+    match_bits<0, 8>(d, dvar, peers.lo, peers.hi);
     uint32_t r = 0;
     if (valid) {
-      const uint32_t below = uint32_t(popc64(peers & lt));
-      const uint32_t cnt = uint32_t(popc64(peers));
+      const uint32_t below = peers.below();
+      const uint32_t cnt = peers.count();
       const uint32_t wbase = s_wcnt[w][d];
       r = wbase + below;
       if (below == 0)
@@ -789,14 +809,13 @@ flag_prefix(const bool (&flag)[kTileItems], int ipw, uint32_t (&pre)[kTileItems]
 {
   const int lane = __lane_id();
   const int w = threadIdx.x / kWave;
-  const uint64_t lt = lanemask_lt();
   uint32_t running = 0;
 #pragma unroll
   for (int j = 0; j < kTileItems; j++) {
     if (j >= ipw)
       break;
     const uint64_t mask = ballot(flag[j]);
-    pre[j] = running + uint32_t(popc64(mask & lt));
+    pre[j] = running + Peers{ uint32_t(mask), uint32_t(mask >> 32) }.below();
     running += uint32_t(popc64(mask));
   }
   if (lane == 0)
