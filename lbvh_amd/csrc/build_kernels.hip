@@ -285,7 +285,7 @@ empty_box()
 }
 
 // Union of element boxes [a, b] left to right, from a bottom-up segment
-// tree over m elements (leaves at bt[m + e]; bt[p] = union(bt[2p],
+// tree over m slots (leaves at bt[m + e]; bt[p] = union(bt[2p],
 // bt[2p + 1]); bt[0] = empty_box()).  std::min / std::max with the left
 // operand kept on ties are associative on non-NaN values, so any
 // order-preserving grouping gives the bits of the reference's union of its
@@ -814,52 +814,6 @@ struct DeltaIndex
   }
 };
 
-// One scene's arrays, located from any of its sorted positions.
-struct TreeScene
-{
-  int64_t P, n;
-  const float* prims;
-  Node* nodes;
-  uint32_t* parent;
-  uint32_t* leafprim;
-  uint32_t* flags;
-  uint32_t* other_end;
-};
-
-template<typename KeyT, bool SEG>
-__device__ __forceinline__ TreeScene
-tree_scene(const KeyT* __restrict__ keys, const Scenes& sc, int64_t x, const float* prims_all,
-           int kind, Node* nodes_all, uint32_t* parent_all,
-           uint32_t* leafprim_all, uint32_t* flags_all, uint32_t* other_end_all)
-{
-  uint32_t seg = 0;
-  int64_t P = 0, n = sc.n;
-  if constexpr (SEG) {
-    seg = uint32_t(keys[x] >> 30);
-    P = int64_t(sc.prim_off[seg]);
-    n = int64_t(sc.prim_off[seg + 1]) - P;
-  }
-  const int64_t nb = P - int64_t(seg);
-  const int64_t lb = 2 * P - int64_t(seg);
-  TreeScene t;
-  t.P = P;
-  t.n = n;
-  t.prims = prims_all + int64_t(prim_stride(kind)) * P;
-  t.nodes = nodes_all + nb;
-  t.parent = parent_all + lb;
-  t.leafprim = leafprim_all ? leafprim_all + P : nullptr;
-  t.flags = flags_all + nb;
-  t.other_end = other_end_all + nb;
-  return t;
-}
-
-// Child value of the leaf at sorted position x.
-__device__ __forceinline__ uint32_t
-tree_leaf_value(const TreeScene& ts, const uint32_t* __restrict__ ids, int64_t x)
-{
-  return (ts.leafprim ? uint32_t(int64_t(ids[x]) - ts.P) : uint32_t(x - ts.P)) | kLeafBit;
-}
-
 struct TreeLevels
 {
   int levels;
@@ -872,7 +826,7 @@ struct TreeLevels
 
 constexpr int kTreeUpThreads = 1024; // workgroup of the upper levels (one CU each: LDS-bound)
 
-// FIRST: the level-0 kernel (leaves, 512 elements, ~38 KB of LDS: four workgroups fit a CU);
+// FIRST: the level-0 kernel (leaves, 512 elements, 32 KB of LDS: four workgroups fill a CU's threads);
 // else the kernel of the levels above (its workgroup b starts as level-1
 // workgroup b).
 //
@@ -881,7 +835,8 @@ constexpr int kTreeUpThreads = 1024; // workgroup of the upper levels (one CU ea
 // searches and box queries: searching byte codes 8 at a time and querying a
 // node's box over its whole range instead of child by child took level 0 /
 // the levels above from 685 / 116 to 531 / 92 us (16M, 30-bit) and from 63 /
-// 46 to 54 / 34 us (1M, 63-bit).
+// 46 to 54 / 34 us (1M, 63-bit); single-trip loops, 32-bit positions and
+// records after the last barrier to 465 / 89 and 50 / 32 us.
 template<typename KeyT, typename CodeT, bool SEG, bool FIRST>
 __global__ __launch_bounds__(FIRST ? kTreeLeaves : kTreeUpThreads) void
 k_tree(const KeyT* __restrict__ keys, const uint32_t* __restrict__ ids, Scenes sc,
@@ -895,11 +850,16 @@ k_tree(const KeyT* __restrict__ keys, const uint32_t* __restrict__ ids, Scenes s
   constexpr int NT = FIRST ? kTreeLeaves : kTreeUpThreads;  // threads
   constexpr int EPT = (SL + NT - 1) / NT;                   // elements per thread (lists)
   // elements (level 0: leaves; then listed subtrees), in position order
-  __shared__ uint32_t s_el_l[SL];
-  __shared__ uint32_t s_el_r[SL];
-  // element boxes at s_bt[m + e]; below m: the segment tree over them, or
-  // (NaN boxes present) node j's box at s_bt[1 + j]
-  __shared__ Box s_bt[2 * SL];
+  // (a level-0 element is the leaf at its position)
+  __shared__ uint32_t s_el_l[FIRST ? 1 : SL];
+  __shared__ uint32_t s_el_r[FIRST ? 1 : SL];
+  // element boxes at s_bt[M + e], M the power of two from m up (at least 64);
+  // below M: the segment tree over them, or (NaN boxes present) node j's box
+  // at s_bt[1 + j].  Slots past element m - 1, and the tree nodes over them,
+  // hold nothing and are in no query.
+  constexpr int kMaxM = FIRST ? kTreeLeaves : 2048;
+  static_assert(kMaxM >= SL, "box tree size");
+  __shared__ Box s_bt[2 * kMaxM];
   // scene of each element (batches above level 0; level 0 reads it from the key)
   __shared__ uint32_t s_el_scene[(SEG && !FIRST) ? SL : 1];
   __shared__ uint32_t s_el_val[SL]; // child value when the element is one leaf
@@ -924,10 +884,46 @@ k_tree(const KeyT* __restrict__ keys, const uint32_t* __restrict__ ids, Scenes s
   int level = FIRST ? 0 : 1;
   uint32_t blk = blockIdx.x;
   int m = 0;
+  int M = kMaxM;
+  uint32_t lo = 0;        // level 0: the workgroup's first position
+  uint32_t my_seg = 0;    // level 0: this thread's element's scene, its first
+  uint32_t my_P = 0;      // position and its size
+  uint32_t my_n = uint32_t(N);
+
+  // f(i) for this thread's share of [0, count): at level 0 at most one i
+  auto each = [&](int count, auto&& f) {
+    if constexpr (FIRST) {
+      if (t < count)
+        f(t);
+    } else {
+      for (int i = t; i < count; i += NT)
+        f(i);
+    }
+  };
+  auto el_l = [&](int e) -> uint32_t {
+    if constexpr (FIRST)
+      return lo + uint32_t(e);
+    else
+      return s_el_l[e];
+  };
+  auto el_r = [&](int e) -> uint32_t {
+    if constexpr (FIRST)
+      return lo + uint32_t(e);
+    else
+      return s_el_r[e];
+  };
+  auto is_leaf = [&](int e) -> bool {
+    if constexpr (FIRST)
+      return true;
+    else
+      return s_el_l[e] == s_el_r[e];
+  };
 
   // Elements from the lists of segments [first, first + nl), in position
   // order; false (nothing loaded) when they number more than cap.
   auto load_lists = [&](uint32_t first, uint32_t nl, uint32_t cap) -> bool {
+    if constexpr (FIRST)
+      return false; // never called
     if (t < kWave) {
       const uint32_t cnt = uint32_t(t) < nl ? coherent_load_u32(&seg_count[first + t]) : 0u;
       uint32_t incl = cnt;
@@ -949,6 +945,9 @@ k_tree(const KeyT* __restrict__ keys, const uint32_t* __restrict__ ids, Scenes s
       return false;
     }
     m = int(total);
+    M = kWave;
+    while (M < m)
+      M <<= 1;
     for (int e = t; e < m; e += NT) {
       uint32_t c = 0, chi = nl; // the last list starting at or before e
       while (chi - c > 1) {
@@ -968,9 +967,11 @@ k_tree(const KeyT* __restrict__ keys, const uint32_t* __restrict__ ids, Scenes s
         bx.lo[q] = coherent_load_f32(&en->box[q]);
         bx.hi[q] = coherent_load_f32(&en->box[3 + q]);
       }
-      s_el_l[e] = el;
-      s_el_r[e] = er;
-      s_bt[m + e] = bx;
+      if constexpr (!FIRST) {
+        s_el_l[e] = el;
+        s_el_r[e] = er;
+      }
+      s_bt[M + e] = bx;
       s_d[e + 1] = uint8_t(d >> 8);
       if (e == 0)
         s_d[0] = uint8_t(d);
@@ -1012,12 +1013,12 @@ k_tree(const KeyT* __restrict__ keys, const uint32_t* __restrict__ ids, Scenes s
 
   if constexpr (FIRST) {
     // ---- level 0 elements: the leaves -------------------------------------------
-    const int64_t lo = int64_t(blk) * kTreeLeaves;
-    const int64_t hi = (N - lo < kTreeLeaves) ? N : lo + kTreeLeaves;
-    m = int(hi - lo);
+    lo = blk * uint32_t(kTreeLeaves);
+    const uint32_t rest = uint32_t(N) - lo;
+    m = rest < uint32_t(kTreeLeaves) ? int(rest) : kTreeLeaves;
     // d[e] between the keys of positions lo + e - 1 and lo + e; 0 past either end
     {
-      const uint32_t x = uint32_t(lo) + uint32_t(t);
+      const uint32_t x = lo + uint32_t(t);
       const uint32_t last = uint32_t(N) - 1u;
       const KeyT key = keys[x < last ? x : last];
       KeyT before = key;
@@ -1036,22 +1037,22 @@ k_tree(const KeyT* __restrict__ keys, const uint32_t* __restrict__ ids, Scenes s
           uint8_t(x < last ? delta_code<KeyT, CodeT, SEG>(key, keys[x + 1], x, sc.prim_off) : 0u);
     }
     if (t < m) {
-      const int64_t x = lo + t;
-      const TreeScene ts = tree_scene<KeyT, SEG>(keys, sc, x, prims_all, kind, nodes_all,
-                                                 parent_all, leafprim_all, flags_all,
-                                                 other_end_all);
-      const int64_t lx = x - ts.P;
-      if (lx < ts.n - 1)
-        ts.flags[lx] = 0u; // fit flags (refits) start at 0
-      uint32_t prim = uint32_t(lx);
-      if (ts.leafprim) {
-        prim = uint32_t(int64_t(ids[x]) - ts.P);
-        ts.leafprim[lx] = prim;
+      const uint32_t x = lo + uint32_t(t);
+      if constexpr (SEG) {
+        my_seg = uint32_t(keys[x] >> 30);
+        my_P = uint32_t(sc.prim_off[my_seg]);
+        my_n = uint32_t(sc.prim_off[my_seg + 1]) - my_P;
       }
-      s_el_l[t] = uint32_t(x);
-      s_el_r[t] = uint32_t(x);
+      const uint32_t lx = x - my_P;
+      if (lx < my_n - 1)
+        flags_all[my_P - my_seg + lx] = 0u; // fit flags (refits) start at 0
+      uint32_t prim = lx;
+      if (leafprim_all) {
+        prim = ids[x] - my_P;
+        leafprim_all[x] = prim;
+      }
       s_el_val[t] = prim | kLeafBit;
-      s_bt[m + t] = load_prim_box(ts.prims, kind, uint64_t(prim));
+      s_bt[M + t] = load_prim_box(prims_all, kind, uint64_t(my_P) + prim);
     }
     __syncthreads();
   } else {
@@ -1065,45 +1066,56 @@ k_tree(const KeyT* __restrict__ keys, const uint32_t* __restrict__ ids, Scenes s
       s_bt[0] = empty_box();
     // exact NaN semantics need the unions in tree order (passes below)
     int any_nan = 0;
-    for (int e = t; e < m; e += NT)
-      any_nan |= box_has_nan(s_bt[m + e]) ? 1 : 0;
+    each(m, [&](int e) { any_nan |= box_has_nan(s_bt[M + e]) ? 1 : 0; });
     const bool nan = __syncthreads_or(any_nan) != 0;
-    int half0 = 1; // the deepest level of the box tree that holds unions
-    while (half0 * 2 < m)
-      half0 <<= 1;
-    for (int j = t; j < m - 1; j += NT) {
+    each(m - 1, [&](int j) {
       const uint32_t x = s_d[j + 1];
       uint8_t inb = 0;
       if (x > 0) {
         const int i = s_dx.left_less(j + 1, x);
-        const int k = s_dx.right_less(j + 1, x);
-        if (i >= 0 && k >= 0) {
+        const int q = s_dx.right_less(j + 1, x);
+        if (i >= 0 && q >= 0) {
           inb = 1;
           s_na[j] = uint16_t(i);
-          s_nb[j] = uint16_t(k - 1);
+          s_nb[j] = uint16_t(q - 1);
         }
       }
       s_inb[j] = inb;
       s_round[j] = 0;
-    }
-    for (int e = t; e < m; e += NT) {
+    });
+    each(m, [&](int e) {
       s_esc[e] = 0;
       s_kid[e] = 0xffff;
-    }
-    for (int half = half0; half >= 1; half >>= 1) {
-      for (int q = t; q < half; q += NT) {
-        const int p = half + q;
-        if (!nan && p < m)
-          s_bt[p] = box_union(s_bt[2 * p], s_bt[2 * p + 1]);
+    });
+    // the box tree: each wave the 6 levels over its chunks of 64 elements
+    // (LDS operations of one wave complete in order: no barrier between
+    // levels), then one wave the levels over the chunks
+    if (!nan) {
+      for (int c = w; c * kWave < m; c += NT / kWave) {
+#pragma unroll
+        for (int d = 1; d <= 6; d++) {
+          if (lane < (kWave >> d)) {
+            const int p = (M >> d) + c * (kWave >> d) + lane;
+            s_bt[p] = box_union(s_bt[2 * p], s_bt[2 * p + 1]);
+          }
+          __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        }
       }
-      __syncthreads();
     }
-    for (int j = t; j < m - 1; j += NT) {
+    __syncthreads();
+    if (!nan && w == 0) {
+      for (int half = M / kWave / 2; half >= 1; half >>= 1) {
+        if (lane < half)
+          s_bt[half + lane] = box_union(s_bt[2 * (half + lane)], s_bt[2 * (half + lane) + 1]);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      }
+    }
+    each(m - 1, [&](int j) {
       if (s_inb[j]) {
         const int a = s_na[j], b = s_nb[j];
         s_kid[(s_d[b + 1] > s_d[a]) ? b : a] = uint16_t(j);
       }
-    }
+    });
     __syncthreads();
     // ---- boxes, children before parents (LDS only: a barrier waits for every
     // outstanding global store, so the records are written afterwards) ------
@@ -1128,74 +1140,14 @@ k_tree(const KeyT* __restrict__ keys, const uint32_t* __restrict__ ids, Scenes s
           if (rd == 0 || rd >= pass)
             continue;
         }
-        const Box lb = l_el ? s_bt[m + j] : s_bt[1 + lc];
-        const Box rb = r_el ? s_bt[m + j + 1] : s_bt[1 + rc];
+        const Box lb = l_el ? s_bt[M + j] : s_bt[1 + lc];
+        const Box rb = r_el ? s_bt[M + j + 1] : s_bt[1 + rc];
         s_bt[1 + j] = box_union(lb, rb);
         s_round[j] = uint8_t(pass);
         changed = 1;
       }
       if (!__syncthreads_or(changed))
         break;
-    }
-    // ---- records of the completed nodes ------------------------------------------
-    // children's parent links by split (consecutive positions), node records
-    // by node number (consecutive records)
-    auto node_scene = [&](int j, int64_t& P, int64_t& n, uint32_t& seg) {
-      P = 0;
-      n = N;
-      seg = 0;
-      if constexpr (SEG) {
-        if constexpr (FIRST)
-          seg = uint32_t(keys[s_el_l[j]] >> 30);
-        else
-          seg = s_el_scene[j];
-        P = int64_t(sc.prim_off[seg]);
-        n = int64_t(sc.prim_off[seg + 1]) - P;
-      }
-    };
-    for (int j = t; j < m - 1; j += NT) {
-      if (!s_inb[j])
-        continue;
-      const int a = s_na[j], b = s_nb[j];
-      const int64_t L = s_el_l[a];
-      const int64_t R = s_el_r[b];
-      const int64_t g = s_el_r[j];
-      int64_t P, n;
-      uint32_t seg;
-      node_scene(j, P, n, seg);
-      const int64_t k = (int(s_d[b + 1]) > int(s_d[a])) ? R - P : L - P;
-      const bool lleaf = (a == j) && s_el_l[j] == s_el_r[j];
-      const bool rleaf = (j + 1 == b) && s_el_l[j + 1] == s_el_r[j + 1];
-      const int64_t lg = g - P;
-      const uint32_t up = uint32_t(k) | ((R - L + 1) > kTreelet ? kLinkGlobal : 0u);
-      uint32_t* parent = parent_all + (2 * P - int64_t(seg));
-      parent[lleaf ? (n - 1) + lg : lg] = up | (rleaf ? kLinkSibLeaf : 0u);
-      parent[rleaf ? (n - 1) + lg + 1 : lg + 1] = up | kLinkRight | (lleaf ? kLinkSibLeaf : 0u);
-    }
-    for (int e = t; e < m; e += NT) {
-      const uint32_t jj = s_kid[e];
-      if (jj == 0xffffu)
-        continue; // no node is numbered e
-      const int j = int(jj);
-      const int a = s_na[j], b = s_nb[j];
-      const bool l_el = (a == j);
-      const bool r_el = (j + 1 == b);
-      const Box bx = nan ? s_bt[1 + j] : bt_query(s_bt, m, a, b);
-      const int64_t L = s_el_l[a];
-      const int64_t R = s_el_r[b];
-      const int64_t g = s_el_r[j];
-      int64_t P, n;
-      uint32_t seg;
-      node_scene(j, P, n, seg);
-      const int64_t nb = P - int64_t(seg);
-      const int64_t k = (int(s_d[b + 1]) > int(s_d[a])) ? R - P : L - P;
-      const bool lleaf = l_el && s_el_l[j] == s_el_r[j];
-      const bool rleaf = r_el && s_el_l[j + 1] == s_el_r[j + 1];
-      const int64_t lg = g - P;
-      const uint32_t lvv = lleaf ? s_el_val[j] : uint32_t(lg);
-      const uint32_t rvv = rleaf ? s_el_val[j + 1] : uint32_t(lg + 1);
-      store_node(&nodes_all[nb + k], bx, lvv, rvv);
-      other_end_all[nb + k] = uint32_t((k == L - P) ? R - P : L - P);
     }
     // ---- listed subtrees: elements and nodes whose parent is not in here ------
     auto parent_out = [&](int a, int b) {
@@ -1205,13 +1157,14 @@ k_tree(const KeyT* __restrict__ keys, const uint32_t* __restrict__ ids, Scenes s
       const int ps = (db > da) ? b : a - 1;
       return ps < 0 || ps > m - 2 || !s_inb[ps];
     };
-    for (int e = t; e < m; e += NT)
+    each(m, [&](int e) {
       if (parent_out(e, e))
-        s_esc[e] = uint16_t(e + 1); // an element stands alone
-    __syncthreads();
-    for (int j = t; j < m - 1; j += NT)
+        s_esc[e] = uint16_t(e + 1); // an element stands alone (in no completed node)
+    });
+    each(m - 1, [&](int j) {
       if (s_inb[j] && parent_out(s_na[j], s_nb[j]))
         s_esc[s_na[j]] = uint16_t(kTreeSlots + 1 + j); // a completed node
+    });
     __syncthreads();
     // position order of the listed subtrees: exclusive count of list starts
     // (thread t holds elements [t * EPT, t * EPT + EPT))
@@ -1255,14 +1208,14 @@ k_tree(const KeyT* __restrict__ keys, const uint32_t* __restrict__ ids, Scenes s
         const int j = int(tag) - kTreeSlots - 1;
         a = s_na[j];
         b = s_nb[j];
-        bx = nan ? s_bt[1 + j] : bt_query(s_bt, m, a, b);
+        bx = nan ? s_bt[1 + j] : bt_query(s_bt, M, a, b);
       } else {
         a = b = e;
-        bx = s_bt[m + e];
+        bx = s_bt[M + e];
       }
       TreeEntry* en = &out[o++];
-      coherent_store_u32(&en->l, s_el_l[a]);
-      coherent_store_u32(&en->r, s_el_r[b]);
+      coherent_store_u32(&en->l, el_l(a));
+      coherent_store_u32(&en->r, el_r(b));
       coherent_store_u32(&en->d, uint32_t(s_d[a]) | (uint32_t(s_d[b + 1]) << 8));
 #pragma unroll
       for (int q = 0; q < 3; q++) {
@@ -1273,6 +1226,56 @@ k_tree(const KeyT* __restrict__ keys, const uint32_t* __restrict__ ids, Scenes s
     if (t == 0)
       coherent_store_u32(&seg_count[FIRST ? blk : out_seg],
                          total < uint32_t(kTreeSegCap) ? total : uint32_t(kTreeSegCap));
+    // ---- records of the completed nodes, last: a barrier after them would wait
+    // for their stores ---------------------------------------------------------
+    // children's parent links by split (consecutive positions), node records
+    // by node number (consecutive records)
+    // (a node's range lies in one scene: at level 0 the scene of any element
+    // in it, so of this thread's own)
+    auto node_scene = [&](int j, uint32_t& P, uint32_t& n, uint32_t& seg) {
+      P = my_P;
+      n = my_n;
+      seg = my_seg;
+      if constexpr (SEG && !FIRST) {
+        seg = s_el_scene[j];
+        P = uint32_t(sc.prim_off[seg]);
+        n = uint32_t(sc.prim_off[seg + 1]) - P;
+      }
+    };
+    each(m - 1, [&](int j) {
+      if (!s_inb[j])
+        return;
+      const int a = s_na[j], b = s_nb[j];
+      const uint32_t L = el_l(a), R = el_r(b);
+      uint32_t P, n, seg;
+      node_scene(j, P, n, seg);
+      const uint32_t up = ((s_d[b + 1] > s_d[a]) ? R - P : L - P) |
+                          ((R - L + 1) > uint32_t(kTreelet) ? kLinkGlobal : 0u);
+      const bool lleaf = (a == j) && is_leaf(j);
+      const bool rleaf = (j + 1 == b) && is_leaf(j + 1);
+      const uint32_t lg = el_r(j) - P; // the split: the left child's last leaf
+      uint32_t* parent = parent_all + (2 * size_t(P) - seg);
+      parent[lleaf ? (n - 1) + lg : lg] = up | (rleaf ? kLinkSibLeaf : 0u);
+      parent[rleaf ? n + lg : lg + 1] = up | kLinkRight | (lleaf ? kLinkSibLeaf : 0u);
+    });
+    each(m, [&](int e) {
+      const uint32_t jj = s_kid[e];
+      if (jj == 0xffffu)
+        return; // no node is numbered e
+      const int j = int(jj);
+      const int a = s_na[j], b = s_nb[j];
+      const Box bx = nan ? s_bt[1 + j] : bt_query(s_bt, M, a, b);
+      const uint32_t L = el_l(a), R = el_r(b);
+      uint32_t P, n, seg;
+      node_scene(j, P, n, seg);
+      const bool at_r = s_d[b + 1] > s_d[a]; // a left child, numbered by its last leaf
+      const size_t at = size_t(P - seg) + ((at_r ? R : L) - P);
+      const uint32_t lg = el_r(j) - P;
+      const uint32_t lvv = (a == j && is_leaf(j)) ? s_el_val[j] : lg;
+      const uint32_t rvv = (j + 1 == b && is_leaf(j + 1)) ? s_el_val[j + 1] : lg + 1;
+      store_node(&nodes_all[at], bx, lvv, rvv);
+      other_end_all[at] = (at_r ? L : R) - P;
+    });
     if constexpr (FIRST)
       return; // level 0 hands over to the next kernel
     if (nsub) {
