@@ -10,13 +10,12 @@
 //   2. k_f64_encode: u64 codes (lbvh.h:1432-1473) and the digit histograms
 //      of the radix passes the engine's sort reads (u64 keys, stable by
 //      primitive id: one legal output of lbvh.h:1126-1134);
-//   3. k_f64_karras: divide_node (lbvh.h:1588-1688) for every internal node
-//      (builder_kernel, lbvh.h:1713-1731), plus parent links and range ends;
-//   4. k_f64_fit_local / k_f64_fit_top: bottom-up box fit, the second
-//      arrival at a node computes union_of(left, right) (lbvh.h:1827-1866:
-//      box of the left child, then the union with the right, left operand
-//      first); nodes inside a workgroup's chunk of leaves finish in LDS, the
-//      few whose range crosses a chunk boundary in a second kernel.
+//   3. k_f64_tree_local / k_f64_tree_top: the tree and its boxes bottom up in
+//      one pass, to the nodes of divide_node (lbvh.h:1588-1688, numbers
+//      included) and union_of(left, right) (lbvh.h:1827-1866: box of the left
+//      child, then the union with the right, left operand first); nodes
+//      inside a workgroup's chunk of leaves finish in LDS, the few whose range
+//      crosses a chunk boundary in a second kernel.
 // The input is the converter's boxes (boxes48[i] = converter(primitives[i]),
 // 6 doubles, 16-byte aligned).  Traffic is HBM-bound integer/FP64 work with
 // no reuse beyond the sort, so the kernels stream with grid-stride loops.
@@ -225,8 +224,11 @@ k_f64_encode(const double* __restrict__ boxes, uint64_t n, const double* __restr
         double d = c[k] - bmin[k];
         q[k] = uint64_t(d * scale[k]);
       }
+      // an extent of 2^53 or more can give cell 2^20; the sort reads 60 bits and
+      // the tree needs the order of exactly those
       const uint64_t code =
-        (expand20_d(q[0]) << 2) | (expand20_d(q[1]) << 1) | expand20_d(q[2]);
+        ((expand20_d(q[0]) << 2) | (expand20_d(q[1]) << 1) | expand20_d(q[2])) &
+        ((uint64_t(1) << 60) - 1);
       codes[i] = code;
       for (int p = first_pass; p < passes; p++)
         atomicAdd(&s_hist[(p - first_pass) * radix + int((code >> (p * digit_bits)) & mask)],
@@ -239,111 +241,6 @@ k_f64_encode(const double* __restrict__ boxes, uint64_t n, const double* __restr
     if (v)
       atomicAdd(&hist[j], v);
   }
-}
-
-// Sorted codes around a workgroup's nodes, kept in LDS: positions [lo, hi)
-// read from LDS, the rest (far probes of large ranges) from memory.
-struct CodeWindow
-{
-  const uint64_t* __restrict__ g;
-  const uint64_t* s;
-  int64_t lo, hi;
-  __device__ __forceinline__ uint64_t at(int64_t k) const
-  {
-    return (k >= lo && k < hi) ? s[k - lo] : g[k];
-  }
-};
-
-// calc_delta (lbvh.h:1602-1621) for u64 codes: -1 out of range, clz of the
-// code difference, or clz(j ^ k) + 64 for equal codes.  code_j is the code
-// at j (the node's own position).
-__device__ __forceinline__ int64_t
-delta64(const CodeWindow& c, int64_t n, int64_t j, uint64_t code_j, int64_t k)
-{
-  if (k < 0 || k >= n)
-    return -1;
-  const uint64_t b = c.at(k);
-  if (code_j == b)
-    return int64_t(__clzll((long long)(uint64_t(j) ^ uint64_t(k)))) + 64;
-  return __clzll((long long)(code_j ^ b));
-}
-
-// Nodes per Karras workgroup and the codes kept in LDS on either side.
-constexpr int kKarrasBlock = 1024;
-constexpr int kKarrasMargin = 1024;
-
-// divide_node (lbvh.h:1588-1688) for internal node i, int64 offsets as the
-// reference's int_type for u64 codes; writes left / right (leaf flag bit 63),
-// the other end j of the node's leaf range [min(i, j), max(i, j)], and the
-// parent link of both children (internal child c at parent[c], leaf k at
-// parent[n - 1 + k]; bit 31 set for a right child).
-__global__ __launch_bounds__(kKarrasBlock) void
-k_f64_karras(const uint64_t* __restrict__ codes, uint64_t n_, const uint32_t* __restrict__ ids,
-             uint64_t* __restrict__ node_words, uint32_t* __restrict__ parent,
-             uint32_t* __restrict__ other_end)
-{
-  __shared__ uint64_t s_codes[kKarrasBlock + 2 * kKarrasMargin];
-  const int64_t n = int64_t(n_);
-  const int64_t i0 = int64_t(blockIdx.x) * kKarrasBlock;
-  CodeWindow cw;
-  cw.g = codes;
-  cw.s = s_codes;
-  cw.lo = i0 > kKarrasMargin ? i0 - kKarrasMargin : 0;
-  cw.hi = i0 + kKarrasBlock + kKarrasMargin < n ? i0 + kKarrasBlock + kKarrasMargin : n;
-  for (int64_t k = cw.lo + threadIdx.x; k < cw.hi; k += kKarrasBlock)
-    s_codes[k - cw.lo] = codes[k];
-  __syncthreads();
-  const int64_t i = i0 + threadIdx.x;
-  if (i >= n - 1)
-    return;
-  const uint64_t ci = cw.at(i);
-  const int64_t d = (delta64(cw, n, i, ci, i + 1) - delta64(cw, n, i, ci, i - 1)) < 0 ? -1 : 1;
-  const int64_t delta_min = delta64(cw, n, i, ci, i - d);
-  int64_t l_max = 128;
-  for (;;) {
-    const int64_t k = i + l_max * d;
-    if (k >= n)
-      break;
-    if (!(delta64(cw, n, i, ci, k) > delta_min))
-      break;
-    l_max *= 4;
-  }
-  // div = 2^sh: the reference's l_max / div and ceil_div(l, div) on
-  // non-negative values are shifts
-  int64_t l = 0;
-  for (int sh = 1;; sh++) {
-    const int64_t t = l_max >> sh;
-    if (delta64(cw, n, i, ci, i + (l + t) * d) > delta_min)
-      l += t;
-    if (t == 1)
-      break;
-  }
-  const int64_t j = i + l * d;
-  const int64_t delta_node = delta64(cw, n, i, ci, j);
-  int64_t s = 0;
-  for (int sh = 1;; sh++) {
-    const int64_t div = int64_t(1) << sh;
-    const int64_t t = (l + (div - 1)) >> sh;
-    if (delta64(cw, n, i, ci, i + (s + t) * d) > delta_node)
-      s += t;
-    if (div >= l)
-      break;
-  }
-  const int64_t g = i + s * d + (d < 0 ? d : 0);
-  const int64_t mn = i < j ? i : j;
-  const int64_t mx = j > i ? j : i;
-  const bool l_leaf = mn == g, r_leaf = mx == g + 1;
-  uint64_t left = uint64_t(g), right = uint64_t(g + 1);
-  // a leaf names its sorted position, or (ids != nullptr) the primitive there
-  if (l_leaf)
-    left = (ids ? uint64_t(ids[g]) : left) | kLeafBit64;
-  if (r_leaf)
-    right = (ids ? uint64_t(ids[g + 1]) : right) | kLeafBit64;
-  node_words[size_t(i) * 8 + 6] = left;
-  node_words[size_t(i) * 8 + 7] = right;
-  other_end[i] = uint32_t(j);
-  parent[l_leaf ? size_t(n - 1 + g) : size_t(g)] = uint32_t(i);
-  parent[r_leaf ? size_t(n - 1 + g + 1) : size_t(g + 1)] = uint32_t(i) | 0x80000000u;
 }
 
 __device__ __forceinline__ Box64
@@ -367,151 +264,215 @@ store_box64(double* p, const Box64& b)
   q[2] = make_double2(b.hi[1], b.hi[2]);
 }
 
-// Leaves per fit workgroup (one thread each).
-constexpr int kF64FitLeaves = 512;
-constexpr uint32_t kQueueLeaf = 0x80000000u;
+// Leaves per tree workgroup (one thread each).
+constexpr int kF64Leaves = 512;
 
-// Bottom-up fit, part 1: one thread per sorted leaf position.  A node whose
-// leaf range lies inside the workgroup's chunk of kF64FitLeaves positions is
-// finished in LDS: each arriving child leaves its box in the node's left or
-// right LDS slot and counts its arrival; the second arrival takes the union
-// (left operand first, union_of of lbvh.h:1208-1213) and climbs on.  A child
-// whose parent's range crosses the chunk boundary stops there: its box goes
-// to `stage` and the child is queued for part 2 in the chunk's own queue
-// segment (2 kF64FitLeaves entries: queued nodes are leaves or internal
-// nodes numbered inside the chunk), its count in queue_count[chunk].
-__device__ __forceinline__ void
-climb_local(const double* __restrict__ boxes, uint64_t n, const uint32_t* __restrict__ ids,
-            uint64_t* __restrict__ node_words, uint32_t leaf_link, double* s_box,
-            uint32_t* s_flag, const uint32_t* s_oe, const uint32_t* s_par, uint64_t first,
-            uint64_t k, double* __restrict__ stage, uint32_t* __restrict__ my_queue,
-            uint32_t* s_queued)
+// calc_delta (lbvh.h:1602-1621) of sorted positions k - 1 and k, plus one: the
+// common leading bits of the codes, of the positions after them for equal
+// codes, 0 beyond either end.  At most 128.
+__device__ __forceinline__ uint8_t
+delta_before(const uint64_t* __restrict__ codes, uint64_t n, uint64_t k)
 {
-  const uint64_t last = (first + kF64FitLeaves < n ? first + kF64FitLeaves : n) - 1;
-  Box64 box = load_box64(boxes, ids ? uint64_t(ids[k]) : k);
-  uint64_t child = kLeafBit64 | k;
-  uint32_t link = leaf_link;
-  for (;;) {
-    const uint32_t p = link & 0x7fffffffu;
-    const bool right = (link >> 31) != 0;
-    const bool in_chunk = p >= first && p <= last; // p <= n - 2 always
-    const uint32_t oe = in_chunk ? s_oe[p - first] : 0u;
-    const bool local = in_chunk && (p < oe ? p : oe) >= first && (p > oe ? p : oe) <= last;
-    if (!local) {
-      if (!(child & kLeafBit64))
-        store_box64(stage + child * 6, box);
-      const uint32_t e = (child & kLeafBit64) ? (uint32_t(k) | kQueueLeaf) : uint32_t(child);
-      my_queue[atomicAdd(s_queued, 1u)] = e;
-      return;
-    }
-    const uint32_t slot = p - uint32_t(first);
-    double* mine = s_box + (slot * 2 + (right ? 1 : 0)) * 6;
-#pragma unroll
-    for (int c = 0; c < 3; c++) {
-      mine[c] = box.lo[c];
-      mine[3 + c] = box.hi[c];
-    }
-    if (__hip_atomic_fetch_add(&s_flag[slot], 1u, __ATOMIC_ACQ_REL,
-                               __HIP_MEMORY_SCOPE_WORKGROUP) == 0u)
-      return;
-    const double* other = s_box + (slot * 2 + (right ? 0 : 1)) * 6;
-    Box64 ob;
-#pragma unroll
-    for (int c = 0; c < 3; c++) {
-      ob.lo[c] = other[c];
-      ob.hi[c] = other[3 + c];
-    }
-    box = right ? box_union64(ob, box) : box_union64(box, ob);
-    store_box64(reinterpret_cast<double*>(node_words + size_t(p) * 8), box);
-    child = p;
-    if (p == 0)
-      return;
-    link = s_par[p - first];
-  }
+  if (k == 0 || k >= n)
+    return 0;
+  const uint64_t a = codes[k - 1], b = codes[k];
+  return uint8_t(a == b ? __clzll((long long)((k - 1) ^ k)) + 65
+                        : __clzll((long long)(a ^ b)) + 1);
 }
 
-__global__ __launch_bounds__(kF64FitLeaves) void
-k_f64_fit_local(const double* __restrict__ boxes, uint64_t n, const uint32_t* __restrict__ ids,
-                uint64_t* __restrict__ node_words, const uint32_t* __restrict__ parent,
-                const uint32_t* __restrict__ other_end, double* __restrict__ stage,
-                uint32_t* __restrict__ queue, uint32_t* __restrict__ queue_count)
+// The number of the node over positions [l, r], whose deltas to the outside
+// are dl and dr (delta_before of l and of r + 1): the side of the larger one
+// is where its sibling lies, and divide_node (lbvh.h:1588-1688) numbers a
+// left child by its last position, a right child by its first and the root 0.
+// The deltas around a node are different, but for the root's.
+__device__ __forceinline__ uint32_t
+node_number(uint32_t l, uint32_t r, uint32_t dl, uint32_t dr)
 {
-  __shared__ double s_box[kF64FitLeaves * 2 * 6];
-  __shared__ uint32_t s_flag[kF64FitLeaves];
-  // range ends and parent links of the internal nodes numbered inside the
-  // chunk (every node finished in LDS is one of them)
-  __shared__ uint32_t s_oe[kF64FitLeaves];
-  __shared__ uint32_t s_par[kF64FitLeaves];
+  return dl >= dr ? l : r;
+}
+
+// A node's 64-byte record; the children meet between positions g and g + 1.  A
+// leaf names its sorted position, or (ids != nullptr) the primitive there.
+__device__ __forceinline__ void
+store_node64(uint64_t* __restrict__ node_words, uint32_t p, const Box64& b,
+             const uint32_t* __restrict__ ids, uint32_t l, uint32_t g, uint32_t r)
+{
+  uint64_t left = g, right = uint64_t(g) + 1;
+  if (l == g)
+    left = (ids ? uint64_t(ids[g]) : left) | kLeafBit64;
+  if (r == g + 1)
+    right = (ids ? uint64_t(ids[g + 1]) : right) | kLeafBit64;
+  uint64_t* q = node_words + size_t(p) * 8;
+  store_box64(reinterpret_cast<double*>(q), b);
+  *reinterpret_cast<ulonglong2*>(q + 6) = make_ulonglong2(left, right);
+}
+
+// Tree and boxes bottom up, part 1: one thread per sorted leaf position.  A
+// node knows from the deltas on its two sides which one its parent's split g
+// is on, and the two children of a split meet there: each leaves its box in
+// LDS under its own number (a leaf's is its position; the internal node of
+// that number holds this leaf, so it is made after the leaf's box was read)
+// and exchanges the far end of its range with the split's flag; the second
+// takes the union (left operand first, union_of of lbvh.h:1208-1213) and
+// climbs on.  No search for ranges and splits and no parent links.
+// What is left over (a child whose split is at the chunk's edge, or whose
+// sibling reaches beyond it: then its flag is still set at the end) goes to
+// the chunk's queue as {number, far end}, its box to `stage`.
+// Bound by the climb (the deepest lane's steps, each LDS to LDS).  One box per
+// number and not per child keeps it to 27 KB of LDS: four workgroups a CU.  1M
+// boxes, this kernel + part 2: 58 + 53 us, where divide_node's searches, a
+// flag clear and two fit kernels over parent links took 41 + 5 + 59 + 58; with
+// 1,024 leaves a workgroup 64 + 52.
+__global__ __launch_bounds__(kF64Leaves) void
+k_f64_tree_local(const uint64_t* __restrict__ codes, const double* __restrict__ boxes, uint64_t n,
+                 const uint32_t* __restrict__ ids, uint64_t* __restrict__ node_words,
+                 uint8_t* __restrict__ deltas, uint32_t* __restrict__ flags,
+                 double* __restrict__ stage, uint2* __restrict__ queue,
+                 uint32_t* __restrict__ queue_count)
+{
+  __shared__ double s_box[6][kF64Leaves];
+  __shared__ uint32_t s_flag[kF64Leaves];
+  __shared__ uint8_t s_delta[kF64Leaves + 1];
   __shared__ uint32_t s_queued;
-  const uint64_t first = uint64_t(blockIdx.x) * kF64FitLeaves;
-  const uint64_t k = first + threadIdx.x;
-  s_flag[threadIdx.x] = 0u;
-  if (threadIdx.x == 0)
+  const uint32_t first = uint32_t(blockIdx.x) * uint32_t(kF64Leaves);
+  const uint32_t t = threadIdx.x;
+  const uint32_t m = uint32_t(n - first < uint64_t(kF64Leaves) ? n - first : kF64Leaves);
+  uint2* my_queue = queue + size_t(blockIdx.x) * kF64Leaves;
+  const auto push = [&](uint32_t number, uint32_t far, const Box64& b) {
+    if (number != far)
+      store_box64(stage + size_t(first + number) * 6, b);
+    my_queue[atomicAdd(&s_queued, 1u)] = make_uint2(first + number, first + far);
+  };
+  s_flag[t] = 0u;
+  if (t == 0) {
     s_queued = 0u;
-  if (k < n - 1) {
-    s_oe[threadIdx.x] = other_end[k];
-    s_par[threadIdx.x] = parent[k];
+    s_delta[m] = delta_before(codes, n, uint64_t(first) + m);
+    if (first + m == n)
+      deltas[n] = 0;
+  }
+  Box64 box;
+  if (t < m) {
+    const uint32_t k = first + t;
+    const uint8_t d = delta_before(codes, n, k);
+    s_delta[t] = d;
+    deltas[k] = d;
+    flags[k] = 0u; // for part 2
+    box = load_box64(boxes, ids ? ids[k] : k);
   }
   __syncthreads();
-  if (k < n)
-    climb_local(boxes, n, ids, node_words, parent[n - 1 + k], s_box, s_flag, s_oe, s_par,
-                first, k, stage, queue + size_t(blockIdx.x) * (2 * kF64FitLeaves), &s_queued);
+  if (t < m) {
+    uint32_t l = t, r = t, dl = s_delta[t], dr = s_delta[t + 1];
+    for (;;) {
+      const bool right = dl > dr;
+      const uint32_t number = right ? l : r, far = right ? r : l;
+      if (right ? l == 0 : r + 1 == m) {
+        push(number, far, box);
+        break;
+      }
+      const uint32_t g = right ? l - 1 : r;
+#pragma unroll
+      for (int c = 0; c < 3; c++) {
+        s_box[c][number] = box.lo[c];
+        s_box[3 + c][number] = box.hi[c];
+      }
+      const uint32_t met = __hip_atomic_exchange(&s_flag[g], far + 1, __ATOMIC_ACQ_REL,
+                                                 __HIP_MEMORY_SCOPE_WORKGROUP);
+      if (met == 0u)
+        break;
+      s_flag[g] = 0u;
+      const uint32_t other = right ? g : g + 1;
+      Box64 ob;
+#pragma unroll
+      for (int c = 0; c < 3; c++) {
+        ob.lo[c] = s_box[c][other];
+        ob.hi[c] = s_box[3 + c][other];
+      }
+      if (right) {
+        l = met - 1;
+        dl = s_delta[l];
+        box = box_union64(ob, box);
+      } else {
+        r = met - 1;
+        dr = s_delta[r + 1];
+        box = box_union64(box, ob);
+      }
+      store_node64(node_words, first + node_number(l, r, dl, dr), box, ids, first + l, first + g,
+                   first + r);
+      if (dl == dr) // the root
+        break;
+    }
+  }
   __syncthreads();
-  if (threadIdx.x == 0)
+  const uint32_t met = s_flag[t];
+  if (met) {
+    const uint32_t far = met - 1, number = far <= t ? t : t + 1;
+#pragma unroll
+    for (int c = 0; c < 3; c++) {
+      box.lo[c] = s_box[c][number];
+      box.hi[c] = s_box[3 + c][number];
+    }
+    push(number, far, box);
+  }
+  __syncthreads();
+  if (t == 0)
     queue_count[blockIdx.x] = s_queued;
 }
 
-// Bottom-up fit, part 2: the nodes whose range crosses a chunk boundary
-// (all ancestors of such a node do too).  One wave per chunk takes the
-// chunk's queued children; each climbs with a device-scope arrival count
-// per node: the second arrival reads the sibling's box (input box for a
-// leaf, `stage` otherwise), writes the node's box, publishes it to `stage`
-// with device-coherent stores and drains them before counting its arrival
-// at the next node.  flags[] must be zero.
+// Part 2: the nodes whose range crosses a chunk boundary (all ancestors of
+// such a node do too).  One wave per chunk takes the chunk's queued children;
+// each climbs by exchanging far ends with a device-scope flag per split: the
+// second arrival reads the sibling's box (input box for a leaf, `stage`
+// otherwise), writes the node's record, publishes its box to `stage` with
+// device-coherent stores and drains them before the next exchange.  flags[]
+// is zero from part 1.  Bound by that chain (drain, exchange, load) a level;
+// storing the record after the exchange instead takes nothing off it.
 __global__ __launch_bounds__(kWave) void
-k_f64_fit_top(const double* __restrict__ boxes, uint64_t n, const uint32_t* __restrict__ ids,
-              uint64_t* __restrict__ node_words, const uint32_t* __restrict__ parent,
-              uint32_t* flags, uint64_t* stage, const uint32_t* __restrict__ queue,
-              const uint32_t* __restrict__ queue_count)
+k_f64_tree_top(const double* __restrict__ boxes, uint64_t n, const uint32_t* __restrict__ ids,
+               uint64_t* __restrict__ node_words, const uint8_t* __restrict__ deltas,
+               uint32_t* flags, uint64_t* stage, const uint2* __restrict__ queue,
+               const uint32_t* __restrict__ queue_count)
 {
   const uint32_t count = queue_count[blockIdx.x];
-  const uint32_t* my_queue = queue + size_t(blockIdx.x) * (2 * kF64FitLeaves);
+  const uint2* my_queue = queue + size_t(blockIdx.x) * kF64Leaves;
   for (uint32_t q = threadIdx.x; q < count; q += kWave) {
-    const uint32_t e = my_queue[q];
-    const uint32_t c0 = e & ~kQueueLeaf;
-    Box64 box;
-    uint32_t link;
-    if (e & kQueueLeaf) {
-      box = load_box64(boxes, ids ? uint64_t(ids[c0]) : uint64_t(c0));
-      link = parent[n - 1 + c0];
-    } else {
-      box = load_box64(reinterpret_cast<const double*>(stage), c0);
-      link = parent[c0];
-    }
+    const uint2 e = my_queue[q];
+    uint32_t l = e.x < e.y ? e.x : e.y, r = e.x < e.y ? e.y : e.x;
+    uint32_t dl = deltas[l], dr = deltas[size_t(r) + 1];
+    Box64 box = l == r ? load_box64(boxes, ids ? ids[l] : l)
+                       : load_box64(reinterpret_cast<const double*>(stage), e.x);
     for (;;) {
-      const uint32_t p = link & 0x7fffffffu;
-      const bool right = (link >> 31) != 0;
-      // the sibling and the next parent link do not depend on the arrival
-      // count: their loads complete under the drain below
-      const uint64_t sib = node_words[size_t(p) * 8 + (right ? 6 : 7)];
-      const uint32_t next = parent[p];
+      const bool right = dl > dr;
+      const uint32_t g = right ? l - 1 : r;
+      const uint32_t other = right ? g : g + 1;
       vmem_drain();
-      if (atomic_add_agent(&flags[p], 1u) == 0u)
+      const uint32_t met = atomic_exch_agent(&flags[g], (right ? r : l) + 1);
+      if (met == 0u)
         break;
+      const uint32_t far = met - 1;
+      const uint32_t d = deltas[right ? size_t(far) : size_t(far) + 1];
       Box64 ob;
-      if (sib & kLeafBit64) {
-        ob = load_box64(boxes, sib & ~kLeafBit64);
+      if (far == other) {
+        ob = load_box64(boxes, ids ? ids[other] : other);
       } else {
-        const uint64_t* st = stage + sib * 6;
+        const uint64_t* st = stage + size_t(other) * 6;
 #pragma unroll
         for (int c = 0; c < 3; c++) {
           ob.lo[c] = __longlong_as_double((long long)coherent_load_u64(st + c));
           ob.hi[c] = __longlong_as_double((long long)coherent_load_u64(st + 3 + c));
         }
       }
-      box = right ? box_union64(ob, box) : box_union64(box, ob);
-      store_box64(reinterpret_cast<double*>(node_words + size_t(p) * 8), box);
-      if (p == 0)
+      if (right) {
+        l = far;
+        dl = d;
+        box = box_union64(ob, box);
+      } else {
+        r = far;
+        dr = d;
+        box = box_union64(box, ob);
+      }
+      const uint32_t p = node_number(l, r, dl, dr);
+      store_node64(node_words, p, box, ids, l, g, r);
+      if (dl == dr) // the root
         break;
       uint64_t* st = stage + size_t(p) * 6;
 #pragma unroll
@@ -519,7 +480,6 @@ k_f64_fit_top(const double* __restrict__ boxes, uint64_t n, const uint32_t* __re
         coherent_store_u64(st + c, (uint64_t)__double_as_longlong(box.lo[c]));
         coherent_store_u64(st + 3 + c, (uint64_t)__double_as_longlong(box.hi[c]));
       }
-      link = next;
     }
   }
 }
@@ -564,70 +524,64 @@ launch_f64_encode(const double* boxes, uint64_t n, const double* bounds, uint64_
   return hipGetLastError();
 }
 
-// Scratch of the FP64 tree, in order: parent links [2n - 1], range ends
-// [n - 1], fit flags [n - 1], queue counts [chunks], fit queues [chunks * 2
-// kF64FitLeaves] (u32), then 16-byte aligned staging boxes [n - 1] of 48
-// bytes.
+// Scratch of the FP64 tree, in order: fit queues [chunks * kF64Leaves] (8
+// bytes an entry), fit flags [n], queue counts [chunks] (u32), deltas [n + 1]
+// (u8), then 16-byte aligned staging boxes [n - 1] of 48 bytes.
 struct F64Scratch
 {
-  uint32_t *parent, *other_end, *flags, *count, *queue;
+  uint2* queue;
+  uint32_t *flags, *count;
+  uint8_t* deltas;
   double* stage;
 };
 
 static uint64_t
-f64_fit_chunks(uint64_t n)
+f64_chunks(uint64_t n)
 {
-  return (n + kF64FitLeaves - 1) / kF64FitLeaves;
+  return (n + kF64Leaves - 1) / kF64Leaves;
 }
 
 static uint64_t
-f64_scratch_words(uint64_t n)
+f64_stage_offset(uint64_t n)
 {
-  return (2 * n - 1) + 2 * (n - 1) + f64_fit_chunks(n) * (1 + 2 * kF64FitLeaves);
+  const uint64_t b = f64_chunks(n) * (8 * kF64Leaves + 4) + 4 * n + (n + 1);
+  return (b + 15) & ~uint64_t(15);
 }
 
 static F64Scratch
 f64_scratch(void* base, uint64_t n)
 {
   F64Scratch f;
-  f.parent = static_cast<uint32_t*>(base);
-  f.other_end = f.parent + (2 * n - 1);
-  f.flags = f.other_end + (n - 1);
-  f.count = f.flags + (n - 1);
-  f.queue = f.count + f64_fit_chunks(n);
-  f.stage = reinterpret_cast<double*>(static_cast<char*>(base) +
-                                      ((4 * f64_scratch_words(n) + 15) & ~uint64_t(15)));
+  f.queue = static_cast<uint2*>(base);
+  f.flags = reinterpret_cast<uint32_t*>(f.queue + f64_chunks(n) * kF64Leaves);
+  f.count = f.flags + n;
+  f.deltas = reinterpret_cast<uint8_t*>(f.count + f64_chunks(n));
+  f.stage = reinterpret_cast<double*>(static_cast<char*>(base) + f64_stage_offset(n));
   return f;
 }
 
 uint64_t
 f64_tree_scratch_bytes(uint64_t n)
 {
-  return ((4 * f64_scratch_words(n) + 15) & ~uint64_t(15)) + 48 * (n - 1);
+  return f64_stage_offset(n) + 48 * (n - 1);
 }
 
 hipError_t
 launch_f64_tree(const uint64_t* sorted, const uint32_t* ids, const double* boxes, uint64_t n,
                 void* nodes, void* scratch, hipStream_t s)
 {
-  if (n < 2)
+  if (n < 2 || n > 0x7fffffffull)
     return hipErrorInvalidValue;
   uint64_t* w = static_cast<uint64_t*>(nodes);
   const F64Scratch f = f64_scratch(scratch, n);
-  const uint64_t gi = (n - 1 + kKarrasBlock - 1) / kKarrasBlock;
-  hipLaunchKernelGGL(k_f64_karras, dim3(uint32_t(gi)), dim3(kKarrasBlock), 0, s, sorted, n, ids,
-                     w, f.parent, f.other_end);
-  hipError_t e = launch_fill_u32(f.flags, n - 1, 0u, s);
-  if (e != hipSuccess)
-    return e;
-  const uint32_t chunks = uint32_t(f64_fit_chunks(n));
-  hipLaunchKernelGGL(k_f64_fit_local, dim3(chunks), dim3(kF64FitLeaves), 0, s, boxes, n, ids, w,
-                     static_cast<const uint32_t*>(f.parent),
-                     static_cast<const uint32_t*>(f.other_end), f.stage, f.queue, f.count);
-  hipLaunchKernelGGL(k_f64_fit_top, dim3(chunks), dim3(kWave), 0, s, boxes, n, ids, w,
-                     static_cast<const uint32_t*>(f.parent), f.flags,
-                     reinterpret_cast<uint64_t*>(f.stage), static_cast<const uint32_t*>(f.queue),
-                     static_cast<const uint32_t*>(f.count));
+  const uint32_t chunks = uint32_t(f64_chunks(n));
+  hipLaunchKernelGGL(k_f64_tree_local, dim3(chunks), dim3(kF64Leaves), 0, s, sorted, boxes, n, ids,
+                     w, f.deltas, f.flags, f.stage, f.queue, f.count);
+  if (chunks > 1) // else the one workgroup made the root
+    hipLaunchKernelGGL(k_f64_tree_top, dim3(chunks), dim3(kWave), 0, s, boxes, n, ids, w,
+                       static_cast<const uint8_t*>(f.deltas), f.flags,
+                       reinterpret_cast<uint64_t*>(f.stage), static_cast<const uint2*>(f.queue),
+                       static_cast<const uint32_t*>(f.count));
   return hipGetLastError();
 }
 

@@ -232,6 +232,11 @@ atomic_add_agent(uint32_t* p, uint32_t v)
 {
   return __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
+__device__ __forceinline__ uint32_t
+atomic_exch_agent(uint32_t* p, uint32_t v)
+{
+  return __hip_atomic_exchange(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
 
 // ---- wave helpers ----------------------------------------------------------
 

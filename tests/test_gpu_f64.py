@@ -94,6 +94,23 @@ def test_f64_tuner_times_candidates_on_a_fresh_context():
     c.close()
 
 
+@pytest.mark.parametrize("n", [2, 513, 5000])
+def test_f64_extents_beyond_the_code_range_give_a_whole_tree(ctx, n):
+    """Past an extent of 2^53 a centre can fall into cell 2^20, one bit more
+    than the sort reads: every leaf and every node is still reached once."""
+    print("f64 extents beyond 2^53 n=%d" % n, flush=True)
+    rng = np.random.default_rng(n)
+    lo = rng.uniform(-1e17, 1e17, size=(n, 3))
+    got = ctx.build_aabbs_f64(np.concatenate([lo, lo], axis=1), 1).view(np.uint64).reshape(-1, 8)
+    links = got[:, 6:].ravel()
+    leaf = (links >> np.uint64(63)) != 0
+    inner = np.sort(links[~leaf])
+    assert np.array_equal(np.sort(links[leaf] & np.uint64(2**63 - 1)), np.arange(n))
+    assert np.array_equal(inner, np.arange(1, n - 1))
+    box = got[0, :6].view(np.float64)
+    assert np.array_equal(box, np.concatenate([lo.min(axis=0), lo.max(axis=0)]))
+
+
 def test_f64_large_matches_oracle(ctx):
     n = 4_000_037
     print("f64 build n=%d clustered" % n, flush=True)
