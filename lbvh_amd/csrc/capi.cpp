@@ -4,7 +4,8 @@
 // device workspace reused across builds, and optional per-phase HIP-event
 // timing.  A bvh handle owns its node array, parent links, fit flags and
 // centroid bounds, and either owns a device copy of its primitives (host
-// builds) or borrows the caller's device pointer (*_device builds).
+// builds) or borrows the caller's device pointer (*_device builds).  Freed
+// trees' memory is kept in a bounded pool per device for the next tree.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

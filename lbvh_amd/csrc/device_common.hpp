@@ -245,12 +245,6 @@ ballot(bool p)
 {
   return __ballot(p);
 }
-__device__ __forceinline__ uint64_t
-lanemask_lt()
-{
-  uint32_t lane = __lane_id();
-  return (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-}
 __device__ __forceinline__ int
 popc64(uint64_t x)
 {

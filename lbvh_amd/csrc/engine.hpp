@@ -219,10 +219,10 @@ uint32_t scene_encode_groups(uint64_t n);
 // builder<double>: centroid bounds of FP64 boxes (6 doubles each, 16-byte
 // aligned) via f64_bounds_blocks(n) partials of 6 doubles; u64 codes with the
 // digit histograms of passes first_pass .. passes - 1 added to hist[p <<
-// digit_bits ...] (zero before); and the tree over sorted
-// codes into node<double> records (64 B) with f64_tree_scratch_bytes(n) of
-// scratch (queues, fit flags cleared by the launch, deltas, staging boxes).  ids != nullptr: leaves name ids[position] instead of the
-// position.
+// digit_bits ...] (zero before); and the tree over sorted codes into
+// node<double> records (64 B) with f64_tree_scratch_bytes(n) of scratch
+// (queues, fit flags cleared by the launch, deltas, staging boxes).  ids !=
+// nullptr: leaves name ids[position] instead of the position.
 uint32_t f64_bounds_blocks(uint64_t n);
 hipError_t launch_f64_bounds(const double* boxes, uint64_t n, double* partials, double* bounds,
                              hipStream_t s);

@@ -10,8 +10,9 @@
 //   1. take a virtual tile id from an atomic ticket (tiles are numbered in
 //      the order workgroups start, so every tile a workgroup waits on is
 //      already running);
-//   2. rank keys stably inside each wave with ballot-based digit matching
-//      (wave-striped tile order: item j of lane l is key j * 64 + l);
+//   2. rank keys stably inside each wave by matching digits bit by bit
+//      (match_bits; wave-striped tile order: item j of lane l is key
+//      j * 64 + l);
 //   3. publish the tile's digit counts, then resolve each digit's global
 //      offset by decoupled look-back over earlier tiles' epoch-tagged status
 //      words (windowed: several predecessors are read per step);

@@ -164,7 +164,8 @@ lbvh_status sync_and_check(lbvh_ctx* c);
 // build options override the choice (then the tuner is not consulted).
 SortConfig default_sort();
 // The sort a single build uses without tuning (tuner off, or before a
-// bucket is tuned): the hybrid from 65,536 keys, else the default.
+// bucket is tuned): the hybrid, with fewer global digits for fewer keys (none
+// for what one workgroup sorts).
 SortConfig untuned_sort(int key_bits, uint64_t n);
 // Grows a context's workspace to what a build of n primitives with this
 // code width and sort configuration needs.
@@ -188,7 +189,7 @@ int ceil_log2_u64(uint64_t x);
 // its begin_timed()/record() calls (per-call timing forced on meanwhile).
 template<class Q>
 float time_call(lbvh_ctx* c, const Q& queue, lbvh_status* st);
-// Sizes below this are launch-bound: the default is used without tuning.
+// Sizes below this are launch-bound: untuned_sort's choice is used.
 constexpr uint64_t kTuneMinPrims = 1u << 16;
 
 } // namespace lbvh_rt
