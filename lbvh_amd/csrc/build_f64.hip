@@ -27,6 +27,9 @@ namespace lbvh_dev {
 constexpr int kF64Block = 256;
 constexpr uint32_t kF64BoundsBlocks = 1024;
 constexpr uint32_t kF64EncodeBlocks = 512;
+// Two encode workgroups a CU at 1M boxes (one per sort chunk) keep 16 waves
+// with four boxes each in flight.
+constexpr int kF64EncodeBlock = 512;
 constexpr int kF64Unroll = 4;
 constexpr uint64_t kLeafBit64 = 0x8000000000000000ull;
 
@@ -107,8 +110,10 @@ block_bounds(double lo[3], double hi[3], double* s_part)
   __syncthreads();
 }
 
+// Also clears zero[0 .. zero_words).
 __global__ __launch_bounds__(kF64Block) void
-k_f64_bounds(const double* __restrict__ boxes, uint64_t n, double* __restrict__ partials)
+k_f64_bounds(const double* __restrict__ boxes, uint64_t n, double* __restrict__ partials,
+             uint32_t* __restrict__ zero, uint32_t zero_words)
 {
   __shared__ double s_part[6 * (kF64Block / kWave)];
   double lo[3], hi[3];
@@ -118,6 +123,8 @@ k_f64_bounds(const double* __restrict__ boxes, uint64_t n, double* __restrict__ 
     hi[k] = -__builtin_inf();
   }
   const uint64_t stride = uint64_t(gridDim.x) * kF64Block;
+  for (uint64_t j = uint64_t(blockIdx.x) * kF64Block + threadIdx.x; j < zero_words; j += stride)
+    zero[j] = 0u;
   for (uint64_t i0 = uint64_t(blockIdx.x) * kF64Block + threadIdx.x; i0 < n;
        i0 += stride * kF64Unroll) {
     // all loads in flight together (past the end: the last box again, which
@@ -182,16 +189,20 @@ expand20_d(uint64_t n)
 // Codes (lbvh.h:1432-1473 in FP64: scale = 2^20 / (extent + 1), q = (c -
 // min) * scale truncated to u64) and the digit histograms of passes
 // first_pass .. passes - 1, counted in LDS and added to hist[(p - first_pass)
-// * radix + d] (zero before).
-__global__ __launch_bounds__(kF64Block) void
+// * radix + d] (zero before).  counts != nullptr: workgroup g encodes the sort
+// chunk [g * chunk, (g + 1) * chunk) and also writes its counts of pass
+// first_pass to counts[d * gridDim.x + g], so the sort's first pass needs no
+// count pass of its own.  1M boxes: 21 us and a count pass of 9-10 -> 17-19 us
+// (a clearing launch of 2 us went to the bounds kernel).
+__global__ __launch_bounds__(kF64EncodeBlock) void
 k_f64_encode(const double* __restrict__ boxes, uint64_t n, const double* __restrict__ bounds,
              uint64_t* __restrict__ codes, uint32_t* __restrict__ hist, int digit_bits,
-             int first_pass, int passes)
+             int first_pass, int passes, uint32_t* __restrict__ counts, uint64_t chunk)
 {
   extern __shared__ uint32_t s_hist[];
   const int radix = 1 << digit_bits;
   const int words = radix * (passes - first_pass);
-  for (int j = threadIdx.x; j < words; j += kF64Block)
+  for (int j = threadIdx.x; j < words; j += kF64EncodeBlock)
     s_hist[j] = 0u;
   double bmin[3], scale[3];
 #pragma unroll
@@ -202,19 +213,26 @@ k_f64_encode(const double* __restrict__ boxes, uint64_t n, const double* __restr
   }
   __syncthreads();
   const uint64_t mask = uint64_t(radix - 1);
-  const uint64_t stride = uint64_t(gridDim.x) * kF64Block;
-  for (uint64_t i0 = uint64_t(blockIdx.x) * kF64Block + threadIdx.x; i0 < n;
-       i0 += stride * kF64Unroll) {
+  uint64_t first = uint64_t(blockIdx.x) * kF64EncodeBlock + threadIdx.x;
+  uint64_t limit = n;
+  uint64_t stride = uint64_t(gridDim.x) * kF64EncodeBlock;
+  if (counts) {
+    const uint64_t b = uint64_t(blockIdx.x) * chunk;
+    first = b + threadIdx.x;
+    limit = b + chunk < n ? b + chunk : n;
+    stride = kF64EncodeBlock;
+  }
+  for (uint64_t i0 = first; i0 < limit; i0 += stride * kF64Unroll) {
     Box64 b[kF64Unroll];
 #pragma unroll
     for (int u = 0; u < kF64Unroll; u++) {
       const uint64_t i = i0 + u * stride;
-      b[u] = load_box64(boxes, i < n ? i : n - 1);
+      b[u] = load_box64(boxes, i < limit ? i : limit - 1);
     }
 #pragma unroll
     for (int u = 0; u < kF64Unroll; u++) {
       const uint64_t i = i0 + u * stride;
-      if (i >= n)
+      if (i >= limit)
         continue;
       double c[3];
       centre64(b[u], c);
@@ -236,11 +254,14 @@ k_f64_encode(const double* __restrict__ boxes, uint64_t n, const double* __restr
     }
   }
   __syncthreads();
-  for (int j = threadIdx.x; j < words; j += kF64Block) {
+  for (int j = threadIdx.x; j < words; j += kF64EncodeBlock) {
     const uint32_t v = s_hist[j];
     if (v)
       atomicAdd(&hist[j], v);
   }
+  if (counts)
+    for (int d = threadIdx.x; d < radix; d += kF64EncodeBlock)
+      counts[size_t(d) * gridDim.x + blockIdx.x] = s_hist[d];
 }
 
 __device__ __forceinline__ Box64
@@ -498,10 +519,12 @@ f64_bounds_blocks(uint64_t n)
 }
 
 hipError_t
-launch_f64_bounds(const double* boxes, uint64_t n, double* partials, double* bounds, hipStream_t s)
+launch_f64_bounds(const double* boxes, uint64_t n, double* partials, double* bounds,
+                  uint32_t* zero, uint32_t zero_words, hipStream_t s)
 {
   const uint32_t g = f64_bounds_blocks(n);
-  hipLaunchKernelGGL(k_f64_bounds, dim3(g), dim3(kF64Block), 0, s, boxes, n, partials);
+  hipLaunchKernelGGL(k_f64_bounds, dim3(g), dim3(kF64Block), 0, s, boxes, n, partials, zero,
+                     zero_words);
   hipLaunchKernelGGL(k_f64_bounds_final, dim3(1), dim3(kF64Block), 0, s,
                      static_cast<const double*>(partials), g, bounds);
   return hipGetLastError();
@@ -509,18 +532,20 @@ launch_f64_bounds(const double* boxes, uint64_t n, double* partials, double* bou
 
 hipError_t
 launch_f64_encode(const double* boxes, uint64_t n, const double* bounds, uint64_t* codes,
-                  uint32_t* hist, int digit_bits, int first_pass, int passes, hipStream_t s)
+                  uint32_t* hist, int digit_bits, int first_pass, int passes, uint32_t* counts,
+                  uint32_t chunks, uint64_t chunk, hipStream_t s)
 {
   const size_t lds = (size_t(4) << digit_bits) * size_t(passes - first_pass);
-  if (first_pass < 0 || first_pass >= passes || lds > 64 * 1024)
+  if (first_pass < 0 || first_pass >= passes || lds > 64 * 1024 ||
+      (counts && (!chunks || uint64_t(chunks) * chunk < n)))
     return hipErrorInvalidValue;
-  // few workgroups: each flushes up to passes x radix histogram words
-  uint64_t b = (n + kF64Block * kF64Unroll - 1) / (kF64Block * kF64Unroll);
-  const uint32_t g = uint32_t(b < kF64EncodeBlocks ? (b ? b : 1) : kF64EncodeBlocks);
+  // without chunks few workgroups: each flushes up to passes x radix histogram words
+  uint64_t b = (n + kF64EncodeBlock * kF64Unroll - 1) / (kF64EncodeBlock * kF64Unroll);
+  const uint32_t g = counts ? chunks : uint32_t(b < kF64EncodeBlocks ? b : kF64EncodeBlocks);
   // the kernel counts pass p at (p - first_pass) * radix of its pointer
-  hipLaunchKernelGGL(k_f64_encode, dim3(g), dim3(kF64Block), lds, s, boxes, n, bounds, codes,
-                     hist + size_t(first_pass) * (size_t(1) << digit_bits), digit_bits,
-                     first_pass, passes);
+  hipLaunchKernelGGL(k_f64_encode, dim3(g), dim3(kF64EncodeBlock), lds, s, boxes, n, bounds,
+                     codes, hist + size_t(first_pass) * (size_t(1) << digit_bits), digit_bits,
+                     first_pass, passes, counts, chunk);
   return hipGetLastError();
 }
 

@@ -501,10 +501,11 @@ untuned_sort(int key_bits, uint64_t n)
   // launches are what a sort costs, one global digit and the smaller tile
   // (more workgroups); up to kHybridTileCap keys no global digit at all.
   // Device time of a build, us, against reduce-then-scan over every digit:
-  // 4,096 triangles 53 / 112 (30-bit), 54 / 197 (63-bit); 16,384 uniform 75 /
-  // 119, 77 / 210; 65,535 uniform 90 / 135, 92 / 228, clustered (a few full
-  // buckets) 122 / 134, 131 / 226.  Onesweep is faster on the last (98), but
-  // its state belongs to one build: a captured one could not be replayed.
+  // 4,096 triangles 47 / 95 (30-bit), 49 / 163 (63-bit); 16,384 uniform 70 /
+  // 101, 71 / 175; 65,535 uniform 84 / 117, 86 / 192, clustered (a few full
+  // buckets) 116 / 117, 117 / 191.  Onesweep is faster on the last's 30 bits
+  // (90), but its state belongs to one build: a captured one could not be
+  // replayed.
   SortConfig h;
   h.digit_bits = 10;
   h.items = n < kTuneMinPrims ? 8 : 16;

@@ -124,19 +124,22 @@ queue_f64_build(lbvh_ctx* c, const double* d_boxes, uint64_t n, const lbvh_build
   ws.err = small + kSmallErr;
   ws.counts = static_cast<uint32_t*>(c->counts.p);
   ws.counts_words = c->counts.cap / 4;
-  ws.first_counts = false;
+  // the encode writes the first pass's chunk counts (as in FP32 builds)
+  const bool chunked = cfg.strategy == 1 || (cfg.strategy == 2 && cfg.global_digits > 0);
+  ws.first_counts = chunked;
 
   double* partials = static_cast<double*>(c->partials.p);
   double* bounds = partials + 6 * size_t(f64_bounds_blocks(n));
 
   begin_timed(c, 1);
   record(c, 0);
-  hipError_t e = launch_fill_u32(small + kSmallTickets, small_words - kSmallTickets, 0u, c->stream);
-  if (e == hipSuccess)
-    e = launch_f64_bounds(d_boxes, n, partials, bounds, c->stream);
+  hipError_t e = launch_f64_bounds(d_boxes, n, partials, bounds, small + kSmallTickets,
+                                   small_words - kSmallTickets, c->stream);
   if (e == hipSuccess)
     e = launch_f64_encode(d_boxes, n, bounds, static_cast<uint64_t*>(c->keys_a.p), ws.hist,
-                          cfg.digit_bits, first_pass, passes, c->stream);
+                          cfg.digit_bits, first_pass, passes, chunked ? ws.counts : nullptr,
+                          chunked ? rts_groups(n, cfg, nullptr) : 0u,
+                          chunked ? rts_chunk_keys(n, cfg) : 0u, c->stream);
   record(c, 1);
   bool in_b = false;
   if (e == hipSuccess)

@@ -181,8 +181,8 @@ bool same_sort(const SortConfig& a, const SortConfig& b);
 int hybrid_global_digits(int key_bits, int digit_bits, uint64_t n);
 constexpr uint64_t kHybridMeanBucket = 64;
 // FP64 builds have buckets of their own: their pipeline around the sort
-// differs (no encode-written chunk counts), so a pick timed on one kind of
-// build does not carry over to the other.
+// differs, so a pick timed on one kind of build does not carry over to the
+// other.
 uint64_t tune_key(bool batch, int key_bits, uint64_t n, int scalar_bits = 32);
 int ceil_log2_u64(uint64_t x);
 // Device milliseconds of the work `queue` puts on the context stream between
