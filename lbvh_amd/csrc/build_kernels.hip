@@ -124,7 +124,8 @@ k_centroid_bounds(const float* __restrict__ prims, uint64_t n,
 // 1377-1385).  The 63-bit variant applies morton_encoder<8> to FP32 centres.
 // Each workgroup also counts the digits of the radix passes first_pass ..
 // passes - 1 (those whose global histogram the sort reads) in LDS and adds
-// its nonzero counts to the global histogram with atomics.
+// its nonzero counts to the global histogram with atomics.  window: their
+// digits end at the highest code bit in use instead of at fixed bits.
 
 constexpr int kHistMaxWords = 8192; // passes * radix, 32 KiB of LDS
 constexpr int kEncodeUnroll = 4;
@@ -143,7 +144,7 @@ k_encode(const float* __restrict__ cx, const float* __restrict__ cy,
          const float* __restrict__ cz, uint64_t n,
          const float* __restrict__ partials, uint32_t nparts, float* __restrict__ bounds_out,
          KeyT* __restrict__ codes,
-         uint32_t* __restrict__ hist, int digit_bits, int first_pass, int passes,
+         uint32_t* __restrict__ hist, int digit_bits, int first_pass, int passes, bool window,
          uint32_t* __restrict__ counts, uint64_t chunk)
 {
   extern __shared__ uint32_t s_hist[];
@@ -192,15 +193,21 @@ k_encode(const float* __restrict__ cx, const float* __restrict__ cy,
       blo[k] = std_min(blo[k], s_pbox[ww][k]);
       bhi[k] = std_max(bhi[k], s_pbox[ww][3 + k]);
     }
+  float scale[3];
+  morton_scale<KeyT>(blo, bhi, scale);
+  const uint32_t used = used_code_bits<KeyT>(blo, bhi, scale);
   if (blockIdx.x == 0 && threadIdx.x == 0) {
 #pragma unroll
     for (int k = 0; k < 3; k++) {
       bounds_out[k] = blo[k];
       bounds_out[3 + k] = bhi[k];
     }
+    reinterpret_cast<uint32_t*>(bounds_out)[6] = used;
   }
-  float scale[3];
-  morton_scale<KeyT>(blo, bhi, scale);
+  const int digits = passes - first_pass;
+  int shift0 = first_pass * digit_bits;
+  if (window)
+    shift0 = int(used) > digits * digit_bits ? int(used) - digits * digit_bits : 0;
   const KeyT mask = KeyT(radix - 1);
   for (uint64_t i0 = first; i0 < limit; i0 += stride * kEncodeUnroll) {
     // unconditional loads (past the end: the last centre, unused), all in
@@ -221,9 +228,9 @@ k_encode(const float* __restrict__ cx, const float* __restrict__ cy,
         continue;
       const KeyT code = morton_code<KeyT>(x[u], y[u], z[u], blo, scale);
       codes[i] = code;
-      for (int p = first_pass; p < passes; p++) {
-        uint32_t d = uint32_t((code >> (p * digit_bits)) & mask);
-        atomicAdd(&s_hist[(p - first_pass) * radix + d], 1u);
+      for (int p = 0; p < digits; p++) {
+        uint32_t d = uint32_t((code >> (shift0 + p * digit_bits)) & mask);
+        atomicAdd(&s_hist[p * radix + d], 1u);
       }
     }
   }
@@ -1452,8 +1459,8 @@ launch_centroid_bounds(const float* prims, int kind, uint64_t n, float* cx, floa
 hipError_t
 launch_encode(int code_bits, const float* cx, const float* cy, const float* cz, uint64_t n,
               const float* partials, float* bounds, void* codes, uint32_t* hist,
-              int digit_bits, int first_pass, int passes, uint32_t* counts, uint32_t groups,
-              uint64_t chunk, hipStream_t s)
+              int digit_bits, int first_pass, int passes, bool window, uint32_t* counts,
+              uint32_t groups, uint64_t chunk, hipStream_t s)
 {
   if (first_pass < 0 || first_pass >= passes)
     return hipErrorInvalidValue;
@@ -1472,11 +1479,11 @@ launch_encode(int code_bits, const float* cx, const float* cy, const float* cz, 
   if (code_bits == 30)
     hipLaunchKernelGGL(k_encode<uint32_t>, dim3(g), dim3(kEncodeBlock), lds, s, cx, cy, cz, n,
                        partials, nparts, bounds, static_cast<uint32_t*>(codes), h, digit_bits,
-                       first_pass, passes, counts, chunk);
+                       first_pass, passes, window, counts, chunk);
   else
     hipLaunchKernelGGL(k_encode<uint64_t>, dim3(g), dim3(kEncodeBlock), lds, s, cx, cy, cz, n,
                        partials, nparts, bounds, static_cast<uint64_t*>(codes), h, digit_bits,
-                       first_pass, passes, counts, chunk);
+                       first_pass, passes, window, counts, chunk);
   return hipGetLastError();
 }
 

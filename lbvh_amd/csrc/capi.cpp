@@ -458,8 +458,7 @@ lbvh_status build_common(lbvh_ctx* c, const float* d_prims, int kind, uint64_t n
 lbvh_status
 reserve_build(lbvh_ctx* c, uint64_t n, int code_bits, const SortConfig& cfg, bool with_ids)
 {
-  const int key_bits = code_bits == 30 ? 30 : 60;
-  const int passes = sort_passes(key_bits, cfg.digit_bits);
+  const int passes = sort_passes(code_key_bits(code_bits), cfg.digit_bits);
   const uint64_t kw = code_bits == 30 ? 4 : 8;
   lbvh_status st;
   if ((st = ensure(c, c->cent, 12 * n)) != LBVH_OK)
@@ -524,7 +523,7 @@ lbvh_status
 choose_sort(lbvh_ctx* c, const float* d_prims, int kind, uint64_t n, const lbvh_build_opts& opts,
             SortConfig* cfg)
 {
-  const int key_bits = opts.code_bits == 30 ? 30 : 60;
+  const int key_bits = nominal_key_bits(int(opts.code_bits));
   if (sort_overridden(opts)) {
     *cfg = sort_from_opts(opts, key_bits, n);
     return LBVH_OK;
@@ -593,9 +592,9 @@ build_common(lbvh_ctx* c, const float* d_prims, int kind, uint64_t n,
     if (st0 != LBVH_OK)
       return st0;
   }
-  const int key_bits = opts.code_bits == 30 ? 30 : 60;
-  if (!valid_sort_config(cfg, key_bits))
+  if (!valid_sort_config(cfg, nominal_key_bits(int(opts.code_bits))))
     return fail(c, LBVH_E_INVALID, "unsupported sort digit width / tile");
+  const int key_bits = code_key_bits(int(opts.code_bits));
   const int passes = sort_passes(key_bits, cfg.digit_bits);
   const uint32_t radix = 1u << cfg.digit_bits;
   const size_t kw = opts.code_bits == 30 ? 4 : 8;
@@ -653,12 +652,13 @@ build_common(lbvh_ctx* c, const float* d_prims, int kind, uint64_t n,
   ws.counts = static_cast<uint32_t*>(c->counts.p);
   ws.counts_words = c->counts.cap / 4;
   ws.first_counts = chunked;
+  ws.top = reinterpret_cast<const uint32_t*>(b->d_bounds) + 6;
 
   begin_timed(c, 1);
   record(c, 0);
   hipError_t e = hipSuccess;
   if (one_wg)
-    e = launch_small_sort(key_bits, d_prims, kind, n, b->d_bounds, c->keys_b.p,
+    e = launch_small_sort(int(opts.code_bits), d_prims, kind, n, b->d_bounds, c->keys_b.p,
                           with_ids ? static_cast<uint32_t*>(c->ids_b.p) : nullptr, c->stream);
   else
     e = launch_centroid_bounds(d_prims, kind, n, cent, cent + n, cent + 2 * n,
@@ -669,7 +669,7 @@ build_common(lbvh_ctx* c, const float* d_prims, int kind, uint64_t n,
                       static_cast<const float*>(c->partials.p), b->d_bounds,
                       c->keys_a.p, ws.hist,
                       cfg.digit_bits, cfg.strategy == 2 ? passes - cfg.global_digits : 0, passes,
-                      chunked ? ws.counts : nullptr, rts_g,
+                      cfg.strategy == 2, chunked ? ws.counts : nullptr, rts_g,
                       chunked ? rts_chunk_keys(n, cfg) : 0, c->stream);
   record(c, 1);
   bool in_b = one_wg;

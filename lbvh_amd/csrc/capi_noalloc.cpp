@@ -62,9 +62,8 @@ align256(uint64_t x)
 Layout
 layout_for(uint64_t n, int code_bits, const SortConfig& cfg)
 {
-  const int key_bits = code_bits == 30 ? 30 : 60;
   const uint64_t kw = code_bits == 30 ? 4 : 8;
-  const int passes = sort_passes(key_bits, cfg.digit_bits);
+  const int passes = sort_passes(code_key_bits(code_bits), cfg.digit_bits);
   Layout L;
   const uint64_t ticket_words = (tree_ticket_words(n) + 3) & ~uint64_t(3);
   L.small_words = kSmallHist + uint32_t(passes) * (1u << cfg.digit_bits);
@@ -103,7 +102,7 @@ layout_for(uint64_t n, int code_bits, const SortConfig& cfg)
 lbvh_status
 sort_for(lbvh_ctx* c, const lbvh_build_opts& o, uint64_t n, SortConfig* cfg)
 {
-  const int key_bits = o.code_bits == 30 ? 30 : 60;
+  const int key_bits = nominal_key_bits(int(o.code_bits));
   if (sort_overridden(o)) {
     *cfg = sort_from_opts(o, key_bits, n);
   } else {
@@ -193,7 +192,7 @@ lbvh_build_triangles_noalloc(lbvh_ctx* c, const float* d_tri, uint64_t n,
   char* base = static_cast<char*>(scratch_of(c->device));
   auto at = [&](uint64_t off) { return static_cast<void*>(base + off); };
 
-  const int key_bits = opts.code_bits == 30 ? 30 : 60;
+  const int key_bits = code_key_bits(int(opts.code_bits));
   const int passes = sort_passes(key_bits, cfg.digit_bits);
   const size_t kw = opts.code_bits == 30 ? 4 : 8;
   const bool with_ids = opts.leaf_order == LBVH_LEAF_PRIMITIVE_ID;
@@ -212,6 +211,7 @@ lbvh_build_triangles_noalloc(lbvh_ctx* c, const float* d_tri, uint64_t n,
   ws.counts = static_cast<uint32_t*>(at(L.counts));
   ws.counts_words = L.counts_words;
   ws.first_counts = true;
+  ws.top = reinterpret_cast<const uint32_t*>(bounds) + 6;
 
   // The previous call left its tickets at zero unless it failed part way:
   // clear the tree tickets and the error flag.  The centroid-bounds kernel
@@ -226,8 +226,8 @@ lbvh_build_triangles_noalloc(lbvh_ctx* c, const float* d_tri, uint64_t n,
     e = launch_encode(int(opts.code_bits), cent, cent + n, cent + 2 * n, n,
                       static_cast<const float*>(at(L.partials)), bounds,
                       at(L.keys_a), ws.hist, cfg.digit_bits,
-                      cfg.strategy == 2 ? passes - cfg.global_digits : 0, passes, ws.counts,
-                      rts_g, rts_chunk_keys(n, cfg), c->stream);
+                      cfg.strategy == 2 ? passes - cfg.global_digits : 0, passes,
+                      cfg.strategy == 2, ws.counts, rts_g, rts_chunk_keys(n, cfg), c->stream);
   bool in_b = false;
   if (e == hipSuccess)
     e = launch_sort(key_bits, int(kw), n, at(L.keys_a), at(L.keys_b),

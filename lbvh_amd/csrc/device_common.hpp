@@ -328,6 +328,29 @@ morton_scale(const float lo[3], const float hi[3], float scale[3])
   }
 }
 
+// The number of low bits that codes over centroid bounds [lo, hi] use: no
+// centre's cell on an axis is beyond hi's (subtraction, multiplication by the
+// positive scale and truncation are monotone), so the highest code bit is one
+// of the far corner's.  At most 30; with 64-bit codes 63, as `extent + 1`
+// rounds to the extent from 2^24 on and hi then falls into cell 2^20.
+template<typename KeyT>
+__device__ __forceinline__ uint32_t
+used_code_bits(const float lo[3], const float hi[3], const float scale[3])
+{
+  constexpr KeyT kCells = sizeof(KeyT) == 4 ? 1023u : 0x1fffffu; // what the expansions keep
+  uint32_t used = 0;
+#pragma unroll
+  for (int k = 0; k < 3; k++) {
+    float d = hi[k] - lo[k];
+    KeyT q = KeyT(d * scale[k]);
+    q = q < kCells ? q : kCells;
+    const uint32_t cell_bits = q ? 32u - uint32_t(__clz(int(uint32_t(q)))) : 0u;
+    const uint32_t u = cell_bits ? 3u * cell_bits - uint32_t(k) : 0u;
+    used = u > used ? u : used;
+  }
+  return used;
+}
+
 template<typename KeyT>
 __device__ __forceinline__ KeyT
 morton_code(float x, float y, float z, const float lo[3], const float scale[3])

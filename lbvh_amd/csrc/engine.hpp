@@ -25,6 +25,23 @@ struct SortConfig
 constexpr uint32_t kHybridTileKeys = 2048;
 constexpr uint32_t kHybridTileCap = 4096;
 
+// Key bits the sort of a single scene's codes has to order.  63-bit codes hold
+// 20-bit cells, and cell 2^20 for a centre at the far end of an axis of 2^24 or
+// more (FP32; 2^53 in FP64), so bits 60-62 can be set.
+inline int
+code_key_bits(int code_bits)
+{
+  return code_bits == 30 ? 30 : 63;
+}
+
+// The bits that codes of ordinary extents fill: what the tuner's buckets are
+// named by and the number of a hybrid's global digits is chosen for.
+inline int
+nominal_key_bits(int code_bits)
+{
+  return code_bits == 30 ? 30 : 60;
+}
+
 inline int
 sort_passes(int key_bits, int digit_bits)
 {
@@ -42,6 +59,10 @@ struct SortWorkspace
   uint32_t* counts = nullptr;  // reduce-then-scan chunk counts [radix * groups]
   uint64_t counts_words = 0;
   bool first_counts = false;   // the first reduce-then-scan pass's counts are in place
+  // Device word: the number of low key bits in use, from which the hybrid's
+  // global digits count down (single scenes; launch_encode writes it).
+  // nullptr: key_bits, in steps of the digit width from bit 0.
+  const uint32_t* top = nullptr;
   // Scene batches (keys (scene << 30 | code), grouped by scene in ascending
   // order): chunks that each lie in one scene.  When set and the hybrid's
   // global digits hold at most one digit of code bits, one pass over these
@@ -71,15 +92,18 @@ uint32_t centroid_partials_needed(uint64_t n);
 // Morton codes (u32 for 30-bit, u64 for 63-bit) and the digit histograms of
 // passes first_pass .. passes - 1, added into hist[p << digit_bits ...] (zero
 // before).  The centroid bounds are the union of launch_centroid_bounds'
-// partials for the same n; they are also written to `bounds` (6 floats).
+// partials for the same n; they are also written to `bounds` (6 floats, then
+// the number of low bits that the codes use as a 32-bit word).  Pass p is the
+// digit at bit p * digit_bits; with `window` the passes' digits are instead the
+// highest ones in use (SortWorkspace::top).
 // counts != nullptr: `groups` workgroups encode chunks of `chunk` keys and
 // also write the chunk counts of pass first_pass (counts[d * groups + g]),
 // the reduce-then-scan layout.
 hipError_t launch_encode(int code_bits, const float* cx, const float* cy, const float* cz,
                          uint64_t n, const float* partials, float* bounds, void* codes,
                          uint32_t* hist,
-                         int digit_bits, int first_pass, int passes, uint32_t* counts,
-                         uint32_t groups, uint64_t chunk, hipStream_t s);
+                         int digit_bits, int first_pass, int passes, bool window,
+                         uint32_t* counts, uint32_t groups, uint64_t chunk, hipStream_t s);
 uint32_t encode_groups(uint64_t n);
 
 // LSD onesweep radix sort of (key, id) pairs in place across ping-pong
@@ -94,7 +118,7 @@ hipError_t launch_sort(int key_bits, int key_bytes, uint64_t n, void* keys_a, vo
 // The sorted codes and ids (ids may be null) of 2 .. kHybridTileCap
 // primitives, with their centroid bounds (6 floats), in one launch: bounds,
 // encode and sort of a build with SortConfig::global_digits 0.
-hipError_t launch_small_sort(int key_bits, const float* prims, int kind, uint64_t n,
+hipError_t launch_small_sort(int code_bits, const float* prims, int kind, uint64_t n,
                              float* bounds, void* keys, uint32_t* ids, hipStream_t s);
 uint64_t sort_status_words(uint64_t n, const SortConfig& cfg);
 // 32-bit words of ws.counts the sort needs for n keys.

@@ -311,6 +311,23 @@ k_onesweep(const KeyT* __restrict__ kin, KeyT* __restrict__ kout,
 
 constexpr int kUpsweepUnroll = 8;
 
+// Where a pass's digit starts: at bit `shift`, or (top != nullptr) `shift` bits
+// into the window of the `span` bits below bit *top -- of the bits from 0 when
+// fewer are in use.
+struct DigitAt
+{
+  const uint32_t* top;
+  int span;
+  int shift;
+  __device__ __forceinline__ int bit() const
+  {
+    if (!top)
+      return shift;
+    const int t = __builtin_amdgcn_readfirstlane(int(*top));
+    return (t > span ? t - span : 0) + shift;
+  }
+};
+
 // Key range [*begin, *end) of chunk g: fixed chunks of chunk_keys keys, or
 // the scene-aligned chunk table (begin, end pairs) when chunks != nullptr.
 __device__ __forceinline__ void
@@ -332,7 +349,7 @@ chunk_range(uint32_t g, uint32_t n, uint64_t chunk_keys, const uint32_t* __restr
 // counts[g * RADIX + d] (chunk-major) with a chunk table.
 template<typename KeyT, int RBITS>
 __global__ __launch_bounds__(kSortBlock) void
-k_rts_upsweep(const KeyT* __restrict__ keys, uint32_t n, int shift, uint32_t chunk_keys,
+k_rts_upsweep(const KeyT* __restrict__ keys, uint32_t n, DigitAt at, uint32_t chunk_keys,
               uint32_t groups, uint32_t* __restrict__ counts,
               const uint32_t* __restrict__ chunks)
 {
@@ -347,6 +364,7 @@ k_rts_upsweep(const KeyT* __restrict__ keys, uint32_t n, int shift, uint32_t chu
   uint32_t begin, end;
   chunk_range(g, n, chunk_keys, chunks, &begin, &end);
   const KeyT dmask = KeyT(RADIX - 1);
+  const int shift = at.bit();
   for (uint32_t base = begin; base < end; base += kSortBlock * kUpsweepUnroll) {
     KeyT k[kUpsweepUnroll];
 #pragma unroll
@@ -461,7 +479,7 @@ template<typename KeyT, bool VALS, int RBITS, int ITEMS>
 __global__ __launch_bounds__(kSortBlock) void
 k_rts_downsweep(const KeyT* __restrict__ kin, KeyT* __restrict__ kout,
                 const uint32_t* __restrict__ vin, uint32_t* __restrict__ vout, uint32_t n,
-                int shift, uint32_t chunk_tiles, uint32_t groups,
+                DigitAt at, uint32_t chunk_tiles, uint32_t groups,
                 const uint32_t* __restrict__ offsets, const uint32_t* __restrict__ chunks)
 {
   constexpr int RADIX = 1 << RBITS;
@@ -478,6 +496,7 @@ k_rts_downsweep(const KeyT* __restrict__ kin, KeyT* __restrict__ kout,
   const int lane = __lane_id();
   const int w = tid / kWave;
   const KeyT dmask = KeyT(RADIX - 1);
+  const int shift = at.bit();
   const uint32_t g = blockIdx.x;
   uint32_t running[DPT];
 #pragma unroll
@@ -853,9 +872,10 @@ constexpr uint32_t kCountRankBudget = 64;
 // When the runs are too long for step 3, LDS passes over every low digit
 // and then b finish the sort instead.
 //
-// SRC: kTileBuckets, the buckets that start in this workgroup's nominal tile.
-// Otherwise one workgroup sorts all n <= kHybridTileCap keys as one bucket,
-// from the top two digits down: kTileKeys, keys kin with ids 0 .. n - 1;
+// SRC: kTileBuckets, the buckets that start in this workgroup's nominal tile
+// (hi: where their bits start).  Otherwise one workgroup sorts all n <=
+// kHybridTileCap keys as one bucket, from the two digits below the highest bit
+// that varies down: kTileKeys, keys kin with ids 0 .. n - 1;
 // kTileTriangles / kTileBoxes, from the primitives themselves -- centres and
 // their bounds (as k_centroid_bounds), codes (as k_encode), sort.  A build of
 // so few is bound by its launches: this one takes the place of thirteen, and
@@ -866,7 +886,7 @@ template<typename KeyT, bool VALS, int SRC>
 __global__ __launch_bounds__(kTileThreads) void
 k_tile_sort(const KeyT* __restrict__ kin, KeyT* __restrict__ kout,
             const uint32_t* __restrict__ vin, uint32_t* __restrict__ vout, uint32_t n,
-            int hi_shift, uint32_t* __restrict__ big,
+            DigitAt hi, uint32_t* __restrict__ big,
             uint32_t* __restrict__ big_count, uint32_t big_cap,
             const float* __restrict__ prims, float* __restrict__ bounds_out)
 {
@@ -888,7 +908,9 @@ k_tile_sort(const KeyT* __restrict__ kin, KeyT* __restrict__ kout,
   const int w = tid / kWave;
   uint32_t start = 0, end = 0;
   uint32_t m = n;
+  int hi_shift = 0;
   if constexpr (SRC == kTileBuckets) {
+    hi_shift = hi.bit();
     const uint64_t t0 = uint64_t(blockIdx.x) * T;
     if (t0 >= n)
       return;
@@ -1026,6 +1048,8 @@ k_tile_sort(const KeyT* __restrict__ kin, KeyT* __restrict__ kout,
     }
   }
   const KeyT var = block_varying_bits(k_and, k_or, s_and, s_or); // also orders the clear
+  if constexpr (SRC != kTileBuckets)
+    hi_shift = var ? 64 - __clzll((long long)uint64_t(var)) : 0;
   const uint32_t bmask = nb > 1 ? (0xFFFFFFFFu >> __clz(nb - 1)) : 0u;
   const int kmax = (hi_shift + 7) / 8; // 8-bit digits below the top bits
   bool staged = false;
@@ -1452,14 +1476,14 @@ run_rts(int key_bits, uint64_t n, KeyT* ka, KeyT* kb, uint32_t* va, uint32_t* vb
   uint32_t* vdst = vb;
   bool cur_b = false;
   for (int p = 0; p < passes; p++) {
-    const int shift = p * RBITS;
+    const DigitAt at = { nullptr, 0, p * RBITS };
     if (p > 0 || !ws.first_counts)
       hipLaunchKernelGGL((k_rts_upsweep<KeyT, RBITS>), dim3(groups), dim3(kSortBlock), 0, s, src,
-                         uint32_t(n), shift, chunk_tiles * TILE, groups, ws.counts, nullptr);
+                         uint32_t(n), at, chunk_tiles * TILE, groups, ws.counts, nullptr);
     hipLaunchKernelGGL((k_rts_scan<RBITS>), dim3(RADIX), dim3(kSortBlock), 0, s, ws.counts,
                        groups, ws.hist + size_t(p) * RADIX, nullptr);
     hipLaunchKernelGGL((k_rts_downsweep<KeyT, VALS, RBITS, ITEMS>), dim3(groups),
-                       dim3(kSortBlock), 0, s, src, dst, vsrc, vdst, uint32_t(n), shift,
+                       dim3(kSortBlock), 0, s, src, dst, vsrc, vdst, uint32_t(n), at,
                        chunk_tiles, groups, ws.counts, nullptr);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess)
@@ -1478,16 +1502,16 @@ run_rts(int key_bits, uint64_t n, KeyT* ka, KeyT* kb, uint32_t* va, uint32_t* vb
 }
 
 // The hybrid's LDS stage: keys src (grouped into buckets of equal
-// key >> hi_shift, in bucket order) sorted into dst; *in_b = dst_is_b.
+// key >> hi.bit(), in bucket order) sorted into dst; *in_b = dst_is_b.
 template<typename KeyT, bool VALS>
 static hipError_t
 bucket_sorts(int key_bits, uint64_t n, KeyT* src, KeyT* dst, uint32_t* vsrc, uint32_t* vdst,
-             int hi_shift, uint32_t* big, uint32_t* big_count, uint64_t big_cap, bool dst_is_b,
-             bool* in_b, hipStream_t s)
+             const DigitAt& hi, uint32_t* big, uint32_t* big_count, uint64_t big_cap,
+             bool dst_is_b, bool* in_b, hipStream_t s)
 {
   const uint32_t tiles = uint32_t((n + kHybridTileKeys - 1) / kHybridTileKeys);
   hipLaunchKernelGGL((k_tile_sort<KeyT, VALS, kTileBuckets>), dim3(tiles), dim3(kTileThreads), 0,
-                     s, src, dst, vsrc, vdst, uint32_t(n), hi_shift, big, big_count,
+                     s, src, dst, vsrc, vdst, uint32_t(n), hi, big, big_count,
                      uint32_t(big_cap), nullptr, nullptr);
   if (n > kHybridTileCap) // else no range is too long for the tile sort
     hipLaunchKernelGGL((k_big_sort<KeyT, VALS>), dim3(kBigBlocks), dim3(kTileThreads), 0, s, src,
@@ -1511,7 +1535,7 @@ run_hybrid(int key_bits, uint64_t n, KeyT* ka, KeyT* kb, uint32_t* va, uint32_t*
     if (n > kHybridTileCap)
       return hipErrorInvalidValue;
     hipLaunchKernelGGL((k_tile_sort<KeyT, VALS, kTileKeys>), dim3(1), dim3(kTileThreads), 0, s, ka,
-                       kb, nullptr, vb, uint32_t(n), key_bits, nullptr, nullptr, 0u, nullptr,
+                       kb, nullptr, vb, uint32_t(n), DigitAt{}, nullptr, nullptr, 0u, nullptr,
                        nullptr);
     *in_b = true;
     return hipGetLastError();
@@ -1525,7 +1549,9 @@ run_hybrid(int key_bits, uint64_t n, KeyT* ka, KeyT* kb, uint32_t* va, uint32_t*
   KeyT* dst = kb;
   uint32_t* vsrc = nullptr;
   uint32_t* vdst = vb;
-  const int hi_shift = (passes - gd) * RBITS;
+  // the global digits' lowest bit
+  const DigitAt hi = ws.top ? DigitAt{ ws.top, gd * RBITS, 0 }
+                            : DigitAt{ nullptr, 0, (passes - gd) * RBITS };
   if (ws.seg_chunks && seg_pass_applies(key_bits, cfg)) {
     // keys grouped by scene (bits 30 and up) in ascending order, and the
     // global digits hold one digit of code bits: sort each scene by that
@@ -1537,31 +1563,32 @@ run_hybrid(int key_bits, uint64_t n, KeyT* ka, KeyT* kb, uint32_t* va, uint32_t*
     uint32_t* big = big_count + 2;
     if (!ws.first_counts)
       hipLaunchKernelGGL((k_rts_upsweep<KeyT, RBITS>), dim3(sg), dim3(kSortBlock), 0, s, src,
-                         uint32_t(n), hi_shift, 0u, sg, ws.counts, ws.seg_chunks);
+                         uint32_t(n), hi, 0u, sg, ws.counts, ws.seg_chunks);
     hipLaunchKernelGGL((k_seg_scan<RBITS>), dim3(ws.nseg), dim3(kSortBlock), 0, s, ws.counts,
                        ws.seg_first, ws.seg_off, big_count);
     hipLaunchKernelGGL((k_rts_downsweep<KeyT, VALS, RBITS, ITEMS>), dim3(sg), dim3(kSortBlock),
-                       0, s, src, dst, vsrc, vdst, uint32_t(n), hi_shift, 0u, sg, ws.counts,
+                       0, s, src, dst, vsrc, vdst, uint32_t(n), hi, 0u, sg, ws.counts,
                        ws.seg_chunks);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess)
       return e;
     return bucket_sorts<KeyT, VALS>(key_bits, n, dst, src, VALS ? vdst : nullptr,
-                                    VALS ? (vdst == vb ? va : vb) : nullptr, hi_shift, big,
+                                    VALS ? (vdst == vb ? va : vb) : nullptr, hi, big,
                                     big_count, big_cap, src == kb, in_b, s);
   }
   uint32_t* big_count = ws.counts + size_t(groups) * RADIX;
   uint32_t* big = big_count + 2;
   for (int p = passes - gd; p < passes; p++) {
-    const int shift = p * RBITS;
+    DigitAt at = hi;
+    at.shift += (p - (passes - gd)) * RBITS;
     if (p > passes - gd || !ws.first_counts)
       hipLaunchKernelGGL((k_rts_upsweep<KeyT, RBITS>), dim3(groups), dim3(kSortBlock), 0, s, src,
-                         uint32_t(n), shift, chunk_tiles * TILE, groups, ws.counts, nullptr);
+                         uint32_t(n), at, chunk_tiles * TILE, groups, ws.counts, nullptr);
     hipLaunchKernelGGL((k_rts_scan<RBITS>), dim3(RADIX), dim3(kSortBlock), 0, s, ws.counts,
                        groups, ws.hist + size_t(p) * RADIX,
                        p == passes - gd ? big_count : nullptr);
     hipLaunchKernelGGL((k_rts_downsweep<KeyT, VALS, RBITS, ITEMS>), dim3(groups),
-                       dim3(kSortBlock), 0, s, src, dst, vsrc, vdst, uint32_t(n), shift,
+                       dim3(kSortBlock), 0, s, src, dst, vsrc, vdst, uint32_t(n), at,
                        chunk_tiles, groups, ws.counts, nullptr);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess)
@@ -1574,8 +1601,8 @@ run_hybrid(int key_bits, uint64_t n, KeyT* ka, KeyT* kb, uint32_t* va, uint32_t*
       vdst = (vdst == vb) ? va : vb;
     }
   }
-  return bucket_sorts<KeyT, VALS>(key_bits, n, src, dst, vsrc, vdst, hi_shift, big, big_count,
-                                  big_cap, dst == kb, in_b, s);
+  return bucket_sorts<KeyT, VALS>(key_bits, n, src, dst, vsrc, vdst, hi, big, big_count, big_cap,
+                                  dst == kb, in_b, s);
 }
 
 uint64_t
@@ -1633,36 +1660,36 @@ dispatch(int key_bits, uint64_t n, KeyT* ka, KeyT* kb, uint32_t* va, uint32_t* v
 
 template<typename KeyT, bool VALS>
 static void
-small_sort(int key_bits, const float* prims, int kind, uint64_t n, float* bounds, void* keys,
-           uint32_t* ids, hipStream_t s)
+small_sort(const float* prims, int kind, uint64_t n, float* bounds, void* keys, uint32_t* ids,
+           hipStream_t s)
 {
   KeyT* k = static_cast<KeyT*>(keys);
   if (kind == kPrimTriangle)
     hipLaunchKernelGGL((k_tile_sort<KeyT, VALS, kTileTriangles>), dim3(1), dim3(kTileThreads), 0,
-                       s, nullptr, k, nullptr, ids, uint32_t(n), key_bits, nullptr, nullptr, 0u,
+                       s, nullptr, k, nullptr, ids, uint32_t(n), DigitAt{}, nullptr, nullptr, 0u,
                        prims, bounds);
   else
     hipLaunchKernelGGL((k_tile_sort<KeyT, VALS, kTileBoxes>), dim3(1), dim3(kTileThreads), 0, s,
-                       nullptr, k, nullptr, ids, uint32_t(n), key_bits, nullptr, nullptr, 0u,
+                       nullptr, k, nullptr, ids, uint32_t(n), DigitAt{}, nullptr, nullptr, 0u,
                        prims, bounds);
 }
 
 hipError_t
-launch_small_sort(int key_bits, const float* prims, int kind, uint64_t n, float* bounds,
+launch_small_sort(int code_bits, const float* prims, int kind, uint64_t n, float* bounds,
                   void* keys, uint32_t* ids, hipStream_t s)
 {
-  if (n < 2 || n > kHybridTileCap || (key_bits != 30 && key_bits != 60))
+  if (n < 2 || n > kHybridTileCap || (code_bits != 30 && code_bits != 63))
     return hipErrorInvalidValue;
-  if (key_bits == 30) {
+  if (code_bits == 30) {
     if (ids)
-      small_sort<uint32_t, true>(key_bits, prims, kind, n, bounds, keys, ids, s);
+      small_sort<uint32_t, true>(prims, kind, n, bounds, keys, ids, s);
     else
-      small_sort<uint32_t, false>(key_bits, prims, kind, n, bounds, keys, nullptr, s);
+      small_sort<uint32_t, false>(prims, kind, n, bounds, keys, nullptr, s);
   } else {
     if (ids)
-      small_sort<uint64_t, true>(key_bits, prims, kind, n, bounds, keys, ids, s);
+      small_sort<uint64_t, true>(prims, kind, n, bounds, keys, ids, s);
     else
-      small_sort<uint64_t, false>(key_bits, prims, kind, n, bounds, keys, nullptr, s);
+      small_sort<uint64_t, false>(prims, kind, n, bounds, keys, nullptr, s);
   }
   return hipGetLastError();
 }

@@ -450,7 +450,7 @@ start(lbvh_server* s, Req* q, Scene* sc)
     uint64_t want = 2;
     while (want < ntri)
       want <<= 1;
-    const int key_bits = o.code_bits == 30 ? 30 : 60;
+    const int key_bits = nominal_key_bits(int(o.code_bits));
     lbvh_status rs = reserve_build(lane, want, int(o.code_bits), untuned_sort(key_bits, want),
                                    o.leaf_order == LBVH_LEAF_PRIMITIVE_ID);
     if (rs != LBVH_OK)
@@ -761,7 +761,7 @@ lbvh_server_create(int device, const lbvh_server_opts* opts, lbvh_server** out)
       uint64_t want = 2;
       while (want < o.reserve_prims)
         want <<= 1;
-      const int key_bits = o.code_bits == 30 ? 30 : 60;
+      const int key_bits = nominal_key_bits(int(o.code_bits));
       st = reserve_build(c, want, int(o.code_bits), untuned_sort(key_bits, want),
                          o.leaf_order == LBVH_LEAF_PRIMITIVE_ID);
       if (st != LBVH_OK) {

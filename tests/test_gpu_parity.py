@@ -161,6 +161,45 @@ def test_small_builds_match_oracle(ctx, n, dist):
         bvh.destroy()
 
 
+@pytest.mark.parametrize("extent", [0.01, 2.0 ** 24, 2.0 ** 25, 3e7, 1e8, 1e30])
+@pytest.mark.parametrize("n", [200, 4096, 4097, 60000, 70000])
+def test_every_sort_orders_all_code_bits(ctx, n, extent):
+    """From an extent of 2^24 a centre at the far end of an axis falls into
+    cell 2^20, so 63-bit codes use bits 60-62; codes of a small scene leave
+    the top bits empty.  Every sort strategy, the untuned choice, the tuner's
+    and the allocation-free build give the oracle's codes, ids and nodes."""
+    print("code bits n=%d extent=%g" % (n, extent), flush=True)
+    rng = np.random.default_rng(n)
+    c = (rng.random((n, 1, 3)) * extent).astype(np.float32)
+    c[0], c[n // 2], c[-1] = extent, 0.0, extent  # the far corner, out of input order
+    tri = W.make_triangles(np.tile(c, (1, 3, 1)).reshape(n, 9))
+    plain = lbvh_amd.Context(0)
+    plain.set_autotune(False)
+    for bits, leaf in [(63, 1), (63, 0), (30, 1)]:
+        on, _, osc, oids = oracle.build(tri, bits, leaf)
+        assert (bits == 63 and extent == 2.0 ** 24) <= bool((osc >> 60).any())
+        builds = [(plain, {}), (ctx, {})]
+        builds += [(plain, dict(sort_strategy=s, sort_digit_bits=d, sort_tile=t))
+                   for s, d, t in SORT_CONFIGS]
+        for c2, opts in builds:
+            bvh = c2.build_triangles(tri, code_bits=bits, leaf_order=leaf, keep_codes=True, **opts)
+            sc, ids, _ = bvh.codes()
+            assert np.array_equal(sc, osc), opts
+            assert np.array_equal(ids, oids), opts
+            assert bvh.nodes().tobytes() == on.tobytes(), opts
+            bvh.destroy()
+        import ctypes
+        from lbvh_amd.hip import DeviceArray
+        d_tri, d_nodes = DeviceArray.from_host(tri), DeviceArray(32 * (n - 1), np.uint8)
+        opts = lbvh_amd._make_opts(bits, leaf, False, 10, 4096, lbvh_amd.SORT_HYBRID)
+        plain._check(lbvh_amd.lib().lbvh_build_triangles_noalloc(
+            plain.handle, ctypes.c_void_p(d_tri.ptr), n, ctypes.byref(opts),
+            ctypes.c_void_p(d_nodes.ptr)))
+        plain.synchronize()
+        assert d_nodes.numpy().tobytes() == on.tobytes()
+    plain.close()
+
+
 @pytest.mark.parametrize("slots", ["1", "200"])
 @pytest.mark.parametrize("n", [9000, 70001, 300001])
 @pytest.mark.parametrize("bits,leaf", [(30, 0), (63, 1)], ids=["b30_ref", "b63_pid"])

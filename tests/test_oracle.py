@@ -112,6 +112,32 @@ def test_sort_is_numpy_stable_sort(bits):
     assert np.array_equal(sc, codes[order])
 
 
+@pytest.mark.parametrize("bits", [30, 63])
+@pytest.mark.parametrize("extent", [0.0, 1e-7, 0.01, 0.3, 1.0, 100.0, 2.0 ** 23, 2.0 ** 24, 3e7, 1e8, 1e30])
+def test_far_corner_bounds_the_code_bits(bits, extent):
+    """The rule that places the hybrid sort's digits: no code has a bit above
+    the highest of the cells of the bounds' far corner, so digits that end
+    there and stable sorts of the bits below them give the codes' order."""
+    rng = np.random.default_rng(3)
+    f = np.float32
+    for axes in ((1, 1, 1), (1, 0, 0.01), (0, 1e-6, 1)):
+        c = (rng.random((500, 1, 3)) * extent * np.array(axes)).astype(f)
+        tri = W.make_triangles(np.tile(c, (1, 3, 1)).reshape(500, 9))
+        _, ob, osc, oids = oracle.build(tri, bits, 1)
+        b = np.asarray(ob, f).reshape(-1)
+        ext = b[3:] - b[:3]
+        cells = np.minimum((ext * (f(1024 if bits == 30 else 2 ** 20) / (ext + f(1)))).astype(np.uint64),
+                           np.uint64(1023 if bits == 30 else 2 ** 21 - 1))
+        top = max([3 * int(q).bit_length() - k for k, q in enumerate(cells) if q] or [0])
+        assert int(np.bitwise_or.reduce(osc)).bit_length() <= top <= bits
+        code = np.empty(500, np.uint64)
+        code[oids] = osc
+        for span in (8, 10, 20):
+            base = np.uint64(max(top - span, 0))
+            o = np.argsort((code >> base) & np.uint64((1 << span) - 1), kind="stable")
+            assert np.array_equal(o[np.lexsort((code[o], code[o] >> base))], oids)
+
+
 def _karras_bruteforce(codes, code_bits):
     """Binary radix tree over index-augmented keys, numbered as Karras
     (internal node of range [lo, hi] is hi if it is a left child, lo if a
