@@ -151,6 +151,21 @@ k_f64_bounds(const double* __restrict__ boxes, uint64_t n, double* __restrict__ 
     partials[size_t(blockIdx.x) * 6 + threadIdx.x] = s_part[threadIdx.x];
 }
 
+// scale = 2^20 / (extent + 1) of every axis (lbvh.h:1432-1473).
+__device__ __forceinline__ void
+morton_scale64(const double* lo, const double* hi, double scale[3])
+{
+#pragma unroll
+  for (int k = 0; k < 3; k++) {
+    double ext = hi[k] - lo[k];
+    scale[k] = 1048576.0 / (ext + 1.0);
+  }
+}
+
+// The union of the partials to bounds[0 .. 6), and in the first word of
+// bounds[6] the number of low bits that the codes use: the highest of the far
+// corner's (no cell is beyond hi's), 61 to 63 when `extent + 1` rounds to the
+// extent and hi falls into cell 2^20.
 __global__ __launch_bounds__(kF64Block) void
 k_f64_bounds_final(const double* __restrict__ partials, uint32_t nparts,
                    double* __restrict__ bounds)
@@ -172,6 +187,20 @@ k_f64_bounds_final(const double* __restrict__ partials, uint32_t nparts,
   block_bounds(lo, hi, s_part);
   if (threadIdx.x < 6)
     bounds[threadIdx.x] = s_part[threadIdx.x];
+  if (threadIdx.x == 0) {
+    double scale[3];
+    morton_scale64(s_part, s_part + 3, scale);
+    uint32_t used = 0;
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+      double d = s_part[3 + k] - s_part[k];
+      uint64_t q = uint64_t(d * scale[k]);
+      q = q < 0x1fffffull ? q : 0x1fffffull; // what the expansion keeps
+      const uint32_t u = q ? 3u * (64u - uint32_t(__clzll((long long)q))) - uint32_t(k) : 0u;
+      used = u > used ? u : used;
+    }
+    *reinterpret_cast<uint32_t*>(bounds + 6) = used;
+  }
 }
 
 // morton_encoder<8>::expand (lbvh.h:1377-1385): 20 bits to every third bit.
@@ -189,7 +218,8 @@ expand20_d(uint64_t n)
 // Codes (lbvh.h:1432-1473 in FP64: scale = 2^20 / (extent + 1), q = (c -
 // min) * scale truncated to u64) and the digit histograms of passes
 // first_pass .. passes - 1, counted in LDS and added to hist[(p - first_pass)
-// * radix + d] (zero before).  counts != nullptr: workgroup g encodes the sort
+// * radix + d] (zero before).  window: those passes' digits end at the highest
+// code bit in use (bounds[6]) instead of starting at p * digit_bits.  counts != nullptr: workgroup g encodes the sort
 // chunk [g * chunk, (g + 1) * chunk) and also writes its counts of pass
 // first_pass to counts[d * gridDim.x + g], so the sort's first pass needs no
 // count pass of its own.  1M boxes: 21 us and a count pass of 9-10 -> 17-19 us
@@ -197,19 +227,24 @@ expand20_d(uint64_t n)
 __global__ __launch_bounds__(kF64EncodeBlock) void
 k_f64_encode(const double* __restrict__ boxes, uint64_t n, const double* __restrict__ bounds,
              uint64_t* __restrict__ codes, uint32_t* __restrict__ hist, int digit_bits,
-             int first_pass, int passes, uint32_t* __restrict__ counts, uint64_t chunk)
+             int first_pass, int passes, bool window, uint32_t* __restrict__ counts,
+             uint64_t chunk)
 {
   extern __shared__ uint32_t s_hist[];
   const int radix = 1 << digit_bits;
-  const int words = radix * (passes - first_pass);
+  const int digits = passes - first_pass;
+  const int words = radix * digits;
   for (int j = threadIdx.x; j < words; j += kF64EncodeBlock)
     s_hist[j] = 0u;
   double bmin[3], scale[3];
 #pragma unroll
-  for (int k = 0; k < 3; k++) {
+  for (int k = 0; k < 3; k++)
     bmin[k] = bounds[k];
-    double ext = bounds[3 + k] - bmin[k];
-    scale[k] = 1048576.0 / (ext + 1.0);
+  morton_scale64(bmin, bounds + 3, scale);
+  int shift0 = first_pass * digit_bits;
+  if (window) {
+    const int used = int(*reinterpret_cast<const uint32_t*>(bounds + 6));
+    shift0 = used > digits * digit_bits ? used - digits * digit_bits : 0;
   }
   __syncthreads();
   const uint64_t mask = uint64_t(radix - 1);
@@ -242,15 +277,11 @@ k_f64_encode(const double* __restrict__ boxes, uint64_t n, const double* __restr
         double d = c[k] - bmin[k];
         q[k] = uint64_t(d * scale[k]);
       }
-      // an extent of 2^53 or more can give cell 2^20; the sort reads 60 bits and
-      // the tree needs the order of exactly those
       const uint64_t code =
-        ((expand20_d(q[0]) << 2) | (expand20_d(q[1]) << 1) | expand20_d(q[2])) &
-        ((uint64_t(1) << 60) - 1);
+        (expand20_d(q[0]) << 2) | (expand20_d(q[1]) << 1) | expand20_d(q[2]);
       codes[i] = code;
-      for (int p = first_pass; p < passes; p++)
-        atomicAdd(&s_hist[(p - first_pass) * radix + int((code >> (p * digit_bits)) & mask)],
-                  1u);
+      for (int p = 0; p < digits; p++)
+        atomicAdd(&s_hist[p * radix + int((code >> (shift0 + p * digit_bits)) & mask)], 1u);
     }
   }
   __syncthreads();
@@ -532,8 +563,8 @@ launch_f64_bounds(const double* boxes, uint64_t n, double* partials, double* bou
 
 hipError_t
 launch_f64_encode(const double* boxes, uint64_t n, const double* bounds, uint64_t* codes,
-                  uint32_t* hist, int digit_bits, int first_pass, int passes, uint32_t* counts,
-                  uint32_t chunks, uint64_t chunk, hipStream_t s)
+                  uint32_t* hist, int digit_bits, int first_pass, int passes, bool window,
+                  uint32_t* counts, uint32_t chunks, uint64_t chunk, hipStream_t s)
 {
   const size_t lds = (size_t(4) << digit_bits) * size_t(passes - first_pass);
   if (first_pass < 0 || first_pass >= passes || lds > 64 * 1024 ||
@@ -545,7 +576,7 @@ launch_f64_encode(const double* boxes, uint64_t n, const double* bounds, uint64_
   // the kernel counts pass p at (p - first_pass) * radix of its pointer
   hipLaunchKernelGGL(k_f64_encode, dim3(g), dim3(kF64EncodeBlock), lds, s, boxes, n, bounds,
                      codes, hist + size_t(first_pass) * (size_t(1) << digit_bits), digit_bits,
-                     first_pass, passes, counts, chunk);
+                     first_pass, passes, window, counts, chunk);
   return hipGetLastError();
 }
 

@@ -26,7 +26,7 @@ lbvh_status
 choose_sort_f64(lbvh_ctx* c, const double* d_boxes, uint64_t n, const lbvh_build_opts& opts,
                 void* d_nodes, SortConfig* cfg)
 {
-  const int key_bits = 60;
+  const int key_bits = nominal_key_bits(63);
   if (sort_overridden(opts)) {
     *cfg = sort_from_opts(opts, key_bits, n);
     return LBVH_OK;
@@ -70,9 +70,9 @@ lbvh_status
 queue_f64_build(lbvh_ctx* c, const double* d_boxes, uint64_t n, const lbvh_build_opts& opts,
                 void* d_nodes, const SortConfig& cfg)
 {
-  const int key_bits = 60;
-  if (!valid_sort_config(cfg, key_bits))
+  if (!valid_sort_config(cfg, nominal_key_bits(63)))
     return fail(c, LBVH_E_INVALID, "unsupported sort digit width / tile");
+  const int key_bits = code_key_bits(63);
   const int passes = sort_passes(key_bits, cfg.digit_bits);
   // the passes whose histogram the encode counts: at least one
   const int first_pass =
@@ -91,8 +91,8 @@ queue_f64_build(lbvh_ctx* c, const double* d_boxes, uint64_t n, const lbvh_build
     if ((st = ensure(c, c->ids_b, 4 * n)) != LBVH_OK)
       return st;
   }
-  // bounds partials, then the final bounds
-  if ((st = ensure(c, c->partials, 48ull * (f64_bounds_blocks(n) + 1))) != LBVH_OK)
+  // bounds partials, then the final bounds and the number of code bits in use
+  if ((st = ensure(c, c->partials, 48ull * (f64_bounds_blocks(n) + 1) + 8)) != LBVH_OK)
     return st;
   const uint32_t small_words = kSmallHist + uint32_t(passes) * radix;
   if ((st = ensure(c, c->small, 4ull * small_words, true)) != LBVH_OK)
@@ -130,6 +130,7 @@ queue_f64_build(lbvh_ctx* c, const double* d_boxes, uint64_t n, const lbvh_build
 
   double* partials = static_cast<double*>(c->partials.p);
   double* bounds = partials + 6 * size_t(f64_bounds_blocks(n));
+  ws.top = reinterpret_cast<const uint32_t*>(bounds + 6);
 
   begin_timed(c, 1);
   record(c, 0);
@@ -137,7 +138,8 @@ queue_f64_build(lbvh_ctx* c, const double* d_boxes, uint64_t n, const lbvh_build
                                    small_words - kSmallTickets, c->stream);
   if (e == hipSuccess)
     e = launch_f64_encode(d_boxes, n, bounds, static_cast<uint64_t*>(c->keys_a.p), ws.hist,
-                          cfg.digit_bits, first_pass, passes, chunked ? ws.counts : nullptr,
+                          cfg.digit_bits, first_pass, passes, cfg.strategy == 2,
+                          chunked ? ws.counts : nullptr,
                           chunked ? rts_groups(n, cfg, nullptr) : 0u,
                           chunked ? rts_chunk_keys(n, cfg) : 0u, c->stream);
   record(c, 1);

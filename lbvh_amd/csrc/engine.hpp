@@ -242,10 +242,12 @@ uint32_t scene_encode_groups(uint64_t n);
 
 // builder<double>: centroid bounds of FP64 boxes (6 doubles each, 16-byte
 // aligned) via f64_bounds_blocks(n) partials of 6 doubles, clearing zero[0 ..
-// zero_words); u64 codes with the digit histograms of passes first_pass ..
-// passes - 1 added to hist[p << digit_bits ...] (zero before) and, counts !=
-// nullptr, the chunk counts of the sort's first pass over `chunks` chunks of
-// `chunk` keys; and the tree over sorted codes into
+// zero_words), to 6 doubles and, as a 32-bit word after them, the number of low
+// bits that the codes use; u64 codes with the digit histograms of passes
+// first_pass .. passes - 1 (`window` as in launch_encode) added to hist[p <<
+// digit_bits ...] (zero before) and, counts != nullptr, the chunk counts of the
+// sort's first pass over `chunks` chunks of `chunk` keys; and the tree over
+// sorted codes into
 // node<double> records (64 B) with f64_tree_scratch_bytes(n) of scratch
 // (queues, fit flags cleared by the launch, deltas, staging boxes).  ids !=
 // nullptr: leaves name ids[position] instead of the position.
@@ -254,8 +256,8 @@ hipError_t launch_f64_bounds(const double* boxes, uint64_t n, double* partials, 
                              uint32_t* zero, uint32_t zero_words, hipStream_t s);
 hipError_t launch_f64_encode(const double* boxes, uint64_t n, const double* bounds,
                              uint64_t* codes, uint32_t* hist, int digit_bits, int first_pass,
-                             int passes, uint32_t* counts, uint32_t chunks, uint64_t chunk,
-                             hipStream_t s);
+                             int passes, bool window, uint32_t* counts, uint32_t chunks,
+                             uint64_t chunk, hipStream_t s);
 uint64_t f64_tree_scratch_bytes(uint64_t n);
 hipError_t launch_f64_tree(const uint64_t* sorted, const uint32_t* ids, const double* boxes,
                            uint64_t n, void* nodes, void* scratch, hipStream_t s);

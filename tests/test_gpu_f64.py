@@ -97,7 +97,8 @@ def test_f64_tuner_times_candidates_on_a_fresh_context():
 @pytest.mark.parametrize("n", [2, 513, 5000])
 def test_f64_extents_beyond_the_code_range_give_a_whole_tree(ctx, n):
     """Past an extent of 2^53 a centre can fall into cell 2^20, one bit more
-    than the sort reads: every leaf and every node is still reached once."""
+    than the other cells: every leaf and every node is still reached once, and
+    the tree is the oracle's."""
     print("f64 extents beyond 2^53 n=%d" % n, flush=True)
     rng = np.random.default_rng(n)
     lo = rng.uniform(-1e17, 1e17, size=(n, 3))
@@ -109,6 +110,34 @@ def test_f64_extents_beyond_the_code_range_give_a_whole_tree(ctx, n):
     assert np.array_equal(inner, np.arange(1, n - 1))
     box = got[0, :6].view(np.float64)
     assert np.array_equal(box, np.concatenate([lo.min(axis=0), lo.max(axis=0)]))
+    want, _, _ = oracle.build_f64(np.concatenate([lo, lo], axis=1), 1)
+    assert got.tobytes() == want.tobytes()
+
+
+@pytest.mark.parametrize("extent", [0.01, 2.0 ** 53, 2.0 ** 54, 1e17, 1e200])
+@pytest.mark.parametrize("n", [200, 4096, 4097, 60000, 70000])
+def test_f64_every_sort_orders_all_code_bits(ctx, n, extent):
+    """FP64 codes use bits 60-62 from an extent of 2^53 on, and leave the top
+    bits of small scenes empty: the untuned sort, the tuner's and every forced
+    one give the oracle's tree."""
+    print("f64 code bits n=%d extent=%g" % (n, extent), flush=True)
+    rng = np.random.default_rng(n)
+    c = rng.random((n, 3)) * extent
+    c[0], c[n // 2], c[-1] = extent, 0.0, extent  # the far corner, out of input order
+    boxes = np.concatenate([c, c], axis=1)
+    plain = lbvh_amd.Context(0)
+    plain.set_autotune(False)
+    for leaf in (0, 1):
+        want, codes, _ = oracle.build_f64(boxes, leaf)
+        assert (extent == 2.0 ** 53) <= bool((codes >> np.uint64(60)).any())
+        assert ctx.build_aabbs_f64(boxes, leaf).tobytes() == want.tobytes()
+        assert plain.build_aabbs_f64(boxes, leaf).tobytes() == want.tobytes()
+        for strategy, digits, tile in [(1, 8, 0), (1, 10, 0), (2, 8, 0), (2, 10, 0), (3, 8, 0),
+                                       (3, 10, 4096)]:
+            got = plain.build_aabbs_f64(boxes, leaf, sort_strategy=strategy,
+                                        sort_digit_bits=digits, sort_tile=tile)
+            assert got.tobytes() == want.tobytes(), (strategy, digits, tile)
+    plain.close()
 
 
 def test_f64_large_matches_oracle(ctx):
