@@ -567,7 +567,7 @@ launch_f64_encode(const double* boxes, uint64_t n, const double* bounds, uint64_
                   uint32_t* counts, uint32_t chunks, uint64_t chunk, hipStream_t s)
 {
   const size_t lds = (size_t(4) << digit_bits) * size_t(passes - first_pass);
-  if (first_pass < 0 || first_pass >= passes || lds > 64 * 1024 ||
+  if (first_pass < 0 || first_pass > passes || lds > 64 * 1024 ||
       (counts && (!chunks || uint64_t(chunks) * chunk < n)))
     return hipErrorInvalidValue;
   // without chunks few workgroups: each flushes up to passes x radix histogram words

@@ -1462,7 +1462,7 @@ launch_encode(int code_bits, const float* cx, const float* cy, const float* cz, 
               int digit_bits, int first_pass, int passes, bool window, uint32_t* counts,
               uint32_t groups, uint64_t chunk, hipStream_t s)
 {
-  if (first_pass < 0 || first_pass >= passes)
+  if (first_pass < 0 || first_pass > passes)
     return hipErrorInvalidValue;
   const uint32_t words = uint32_t(1u << digit_bits) * uint32_t(passes - first_pass);
   if (words > uint32_t(kHistMaxWords))

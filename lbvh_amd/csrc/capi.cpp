@@ -497,21 +497,18 @@ untuned_sort(int key_bits, uint64_t n)
 {
   // the hybrid at 10-bit digits.  From 65,536 keys 4,096-key tiles: the
   // tuner's pick at 1M and 16M 63-bit keys and for batches.  Below, where the
-  // launches are what a sort costs, one global digit and the smaller tile
-  // (more workgroups); up to kHybridTileCap keys no global digit at all.
-  // Device time of a build, us, against reduce-then-scan over every digit:
-  // 4,096 triangles 47 / 95 (30-bit), 49 / 163 (63-bit); 16,384 uniform 70 /
-  // 101, 71 / 175; 65,535 uniform 84 / 117, 86 / 192, clustered (a few full
-  // buckets) 116 / 117, 117 / 191.  Onesweep is faster on the last's 30 bits
-  // (90), but its state belongs to one build: a captured one could not be
-  // replayed.
+  // launches are what a sort costs, no global digit: chunks sorted in LDS and
+  // merged, one chunk up to kHybridTileCap keys.  Device time of a build, us,
+  // against reduce-then-scan over every digit, 30-bit and 63-bit codes: 4,096
+  // triangles 47 / 99 and 49 / 168; 16,384 uniform 61 / 105 and 63 / 182; 60,000
+  // uniform 86 / 120 and 89 / 199, clustered 98 / 120 and 101 / 195, one outlier
+  // beside a cluster 83 / 124 and 104 / 203, two clusters 95 / 120 and 119 /
+  // 201.
   SortConfig h;
   h.digit_bits = 10;
   h.items = n < kTuneMinPrims ? 8 : 16;
   h.strategy = 2;
-  if (n < kTuneMinPrims)
-    h.global_digits = n <= kHybridTileCap ? 0 : 1;
-  else
+  if (n >= kTuneMinPrims)
     h.global_digits = hybrid_global_digits(key_bits, h.digit_bits, n);
   return h.global_digits <= sort_passes(key_bits, h.digit_bits) - 2 ? h : default_sort();
 }
@@ -605,9 +602,9 @@ build_common(lbvh_ctx* c, const float* d_prims, int kind, uint64_t n,
     return st;
   // reduce-then-scan and hybrid sorts: the encode counts the first pass's
   // chunks itself (one encode workgroup per chunk)
-  const bool chunked = cfg.strategy == 1 || cfg.strategy == 2;
-  // ... and one workgroup does it all for the fewest primitives
-  const bool one_wg = cfg.strategy == 2 && cfg.global_digits == 0;
+  const bool chunked = cfg.strategy == 1 || (cfg.strategy == 2 && cfg.global_digits > 0);
+  // ... and sorts in LDS encode themselves (the smallest find the bounds, too)
+  const bool in_lds = cfg.strategy == 2 && cfg.global_digits == 0;
   const uint32_t rts_g = chunked ? rts_groups(n, cfg, nullptr) : 0u;
   const uint32_t small_words = kSmallHist + uint32_t(passes) * radix;
   const uint64_t sw = sort_status_words(n, cfg);
@@ -657,14 +654,11 @@ build_common(lbvh_ctx* c, const float* d_prims, int kind, uint64_t n,
   begin_timed(c, 1);
   record(c, 0);
   hipError_t e = hipSuccess;
-  if (one_wg)
-    e = launch_small_sort(int(opts.code_bits), d_prims, kind, n, b->d_bounds, c->keys_b.p,
-                          with_ids ? static_cast<uint32_t*>(c->ids_b.p) : nullptr, c->stream);
-  else
+  if (!in_lds || n > kHybridTileCap)
     e = launch_centroid_bounds(d_prims, kind, n, cent, cent + n, cent + 2 * n,
                                static_cast<float*>(c->partials.p), small + kSmallTickets,
                                small_words - kSmallTickets, c->stream);
-  if (e == hipSuccess && !one_wg)
+  if (e == hipSuccess && !in_lds)
     e = launch_encode(opts.code_bits, cent, cent + n, cent + 2 * n, n,
                       static_cast<const float*>(c->partials.p), b->d_bounds,
                       c->keys_a.p, ws.hist,
@@ -672,8 +666,14 @@ build_common(lbvh_ctx* c, const float* d_prims, int kind, uint64_t n,
                       cfg.strategy == 2, chunked ? ws.counts : nullptr, rts_g,
                       chunked ? rts_chunk_keys(n, cfg) : 0, c->stream);
   record(c, 1);
-  bool in_b = one_wg;
-  if (e == hipSuccess && !one_wg)
+  bool in_b = false;
+  if (e == hipSuccess && in_lds)
+    e = launch_small_sort(int(opts.code_bits), d_prims, kind, n, cent,
+                          static_cast<const float*>(c->partials.p), b->d_bounds, c->keys_a.p,
+                          c->keys_b.p, with_ids ? static_cast<uint32_t*>(c->ids_a.p) : nullptr,
+                          with_ids ? static_cast<uint32_t*>(c->ids_b.p) : nullptr, &in_b,
+                          c->stream);
+  else if (e == hipSuccess)
     e = launch_sort(key_bits, int(kw), n, c->keys_a.p, c->keys_b.p,
                     with_ids ? static_cast<uint32_t*>(c->ids_a.p) : nullptr,
                     with_ids ? static_cast<uint32_t*>(c->ids_b.p) : nullptr, cfg, ws, epoch,

@@ -74,9 +74,8 @@ queue_f64_build(lbvh_ctx* c, const double* d_boxes, uint64_t n, const lbvh_build
     return fail(c, LBVH_E_INVALID, "unsupported sort digit width / tile");
   const int key_bits = code_key_bits(63);
   const int passes = sort_passes(key_bits, cfg.digit_bits);
-  // the passes whose histogram the encode counts: at least one
-  const int first_pass =
-    cfg.strategy == 2 ? passes - (cfg.global_digits > 0 ? cfg.global_digits : 1) : 0;
+  // the passes whose histogram the encode counts
+  const int first_pass = cfg.strategy == 2 ? passes - cfg.global_digits : 0;
   const uint32_t radix = 1u << cfg.digit_bits;
   const bool with_ids = opts.leaf_order == LBVH_LEAF_PRIMITIVE_ID;
 

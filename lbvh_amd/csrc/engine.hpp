@@ -18,12 +18,15 @@ struct SortConfig
                       //    run of equal top bits sorted by the full key in LDS)
   int groups = 0;     // reduce-then-scan: target number of chunks (0 = about two tiles each, 512-2,048)
   int global_digits = 0; // hybrid: digits sorted by global passes (the top ones); 0:
-                         // at most kHybridTileCap keys, in the LDS of one workgroup
+                         // at most kChunkSortMax keys, in LDS by chunks of
+                         // kHybridTileCap that are then merged
 };
 
 // Hybrid strategy: keys per workgroup of the LDS sort (nominal and maximum).
 constexpr uint32_t kHybridTileKeys = 2048;
 constexpr uint32_t kHybridTileCap = 4096;
+// Most keys of a hybrid without global digits.
+constexpr uint32_t kChunkSortMax = 16 * kHybridTileCap;
 
 // Key bits the sort of a single scene's codes has to order.  63-bit codes hold
 // 20-bit cells, and cell 2^20 for a centre at the far end of an axis of 2^24 or
@@ -90,7 +93,7 @@ hipError_t launch_centroid_bounds(const float* prims, int kind, uint64_t n, floa
 uint32_t centroid_partials_needed(uint64_t n);
 
 // Morton codes (u32 for 30-bit, u64 for 63-bit) and the digit histograms of
-// passes first_pass .. passes - 1, added into hist[p << digit_bits ...] (zero
+// passes first_pass .. passes - 1 (none when they are equal), added into hist[p << digit_bits ...] (zero
 // before).  The centroid bounds are the union of launch_centroid_bounds'
 // partials for the same n; they are also written to `bounds` (6 floats, then
 // the number of low bits that the codes use as a 32-bit word).  Pass p is the
@@ -115,11 +118,14 @@ hipError_t launch_sort(int key_bits, int key_bytes, uint64_t n, void* keys_a, vo
                        uint32_t* ids_a,
                        uint32_t* ids_b, const SortConfig& cfg, const SortWorkspace& ws,
                        uint32_t epoch, bool* result_in_b, hipStream_t s);
-// The sorted codes and ids (ids may be null) of 2 .. kHybridTileCap
-// primitives, with their centroid bounds (6 floats), in one launch: bounds,
-// encode and sort of a build with SortConfig::global_digits 0.
+// The encode and sort of a build with SortConfig::global_digits 0, from its
+// primitives (and their centroid bounds, too: one launch) up to kHybridTileCap
+// of them, from launch_centroid_bounds' centres and partials up to
+// kChunkSortMax.  Writes the bounds (6 floats); ids may be null.
 hipError_t launch_small_sort(int code_bits, const float* prims, int kind, uint64_t n,
-                             float* bounds, void* keys, uint32_t* ids, hipStream_t s);
+                             const float* cent, const float* partials, float* bounds,
+                             void* keys_a, void* keys_b, uint32_t* ids_a, uint32_t* ids_b,
+                             bool* result_in_b, hipStream_t s);
 uint64_t sort_status_words(uint64_t n, const SortConfig& cfg);
 // 32-bit words of ws.counts the sort needs for n keys.
 uint64_t sort_counts_words(uint64_t n, const SortConfig& cfg);

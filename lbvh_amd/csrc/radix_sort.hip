@@ -873,14 +873,17 @@ constexpr uint32_t kCountRankBudget = 64;
 // and then b finish the sort instead.
 //
 // SRC: kTileBuckets, the buckets that start in this workgroup's nominal tile
-// (hi: where their bits start).  Otherwise one workgroup sorts all n <=
+// (hi: where their bits start).  Otherwise a workgroup sorts up to
 // kHybridTileCap keys as one bucket, from the two digits below the highest bit
-// that varies down: kTileKeys, keys kin with ids 0 .. n - 1;
-// kTileTriangles / kTileBoxes, from the primitives themselves -- centres and
-// their bounds (as k_centroid_bounds), codes (as k_encode), sort.  A build of
+// that varies down.  kTileKeys: workgroup g the g-th `chunk` keys kin with ids
+// 0 .. n - 1 (k_merge_chunks joins them); kTileCentres: the same of centres
+// (cx, cy, cz of n each) and the partial bounds of k_centroid_bounds, encoding
+// them (as k_encode).  kTileTriangles / kTileBoxes: all n from the primitives
+// themselves -- centres and their bounds, codes, sort.  A build of
 // so few is bound by its launches: this one takes the place of thirteen, and
 // a build of 4,096 triangles goes from 110 to 50 us of kernels.
-constexpr int kTileBuckets = 0, kTileKeys = 1, kTileTriangles = 2, kTileBoxes = 3;
+constexpr int kTileBuckets = 0, kTileKeys = 1, kTileCentres = 2, kTileTriangles = 3,
+              kTileBoxes = 4;
 
 template<typename KeyT, bool VALS, int SRC>
 __global__ __launch_bounds__(kTileThreads) void
@@ -888,7 +891,8 @@ k_tile_sort(const KeyT* __restrict__ kin, KeyT* __restrict__ kout,
             const uint32_t* __restrict__ vin, uint32_t* __restrict__ vout, uint32_t n,
             DigitAt hi, uint32_t* __restrict__ big,
             uint32_t* __restrict__ big_count, uint32_t big_cap,
-            const float* __restrict__ prims, float* __restrict__ bounds_out)
+            const float* __restrict__ prims, float* __restrict__ bounds_out, uint32_t chunk,
+            const float* __restrict__ partials, uint32_t nparts)
 {
   constexpr uint32_t T = lbvh_eng::kHybridTileKeys;
   constexpr uint32_t CAP = lbvh_eng::kHybridTileCap;
@@ -901,7 +905,7 @@ k_tile_sort(const KeyT* __restrict__ kin, KeyT* __restrict__ kout,
   __shared__ KeyT s_or[kTileWaves];
   __shared__ uint32_t s_first[2];
   __shared__ uint32_t s_work;
-  __shared__ float s_box[SRC >= kTileTriangles ? kTileWaves : 1][6];
+  __shared__ float s_box[SRC >= kTileCentres ? kTileWaves : 1][6];
 
   const int tid = threadIdx.x;
   const int lane = __lane_id();
@@ -909,6 +913,10 @@ k_tile_sort(const KeyT* __restrict__ kin, KeyT* __restrict__ kout,
   uint32_t start = 0, end = 0;
   uint32_t m = n;
   int hi_shift = 0;
+  if constexpr (SRC == kTileKeys || SRC == kTileCentres) {
+    start = blockIdx.x * chunk;
+    m = n - start < chunk ? n - start : chunk;
+  }
   if constexpr (SRC == kTileBuckets) {
     hi_shift = hi.bit();
     const uint64_t t0 = uint64_t(blockIdx.x) * T;
@@ -972,8 +980,8 @@ k_tile_sort(const KeyT* __restrict__ kin, KeyT* __restrict__ kout,
       if (j >= ipw)
         break;
       const uint32_t li = lbase + uint32_t(j) * kWave;
-      key[j] = li < m ? kin[li] : KeyT(0);
-      val[j] = li;
+      key[j] = li < m ? kin[start + li] : KeyT(0);
+      val[j] = start + li;
       aux[j] = 0u;
       if (li < m) {
         k_and &= key[j];
@@ -988,21 +996,36 @@ k_tile_sort(const KeyT* __restrict__ kin, KeyT* __restrict__ kout,
       if (j >= ipw)
         break;
       const uint32_t li = lbase + uint32_t(j) * kWave;
-      b[j] = load_prim_box(prims, SRC == kTileTriangles ? kPrimTriangle : kPrimAabb,
-                           li < n ? li : n - 1);
+      const uint32_t i = start + (li < m ? li : m - 1);
+      if constexpr (SRC == kTileCentres) {
+#pragma unroll
+        for (int k = 0; k < 3; k++)
+          b[j].lo[k] = prims[size_t(k) * n + i];
+      } else {
+        b[j] = load_prim_box(prims, SRC == kTileTriangles ? kPrimTriangle : kPrimAabb, i);
+      }
     }
     float lo[3] = { INFINITY, INFINITY, INFINITY };
     float hi[3] = { -INFINITY, -INFINITY, -INFINITY };
+    if constexpr (SRC == kTileCentres) {
+      for (uint32_t g = tid; g < nparts; g += kTileThreads)
 #pragma unroll
-    for (int j = 0; j < kTileItems; j++) {
-      if (j >= ipw)
-        break;
+        for (int k = 0; k < 3; k++) {
+          lo[k] = std_min(lo[k], partials[6 * g + k]);
+          hi[k] = std_max(hi[k], partials[6 * g + 3 + k]);
+        }
+    } else {
 #pragma unroll
-      for (int k = 0; k < 3; k++) {
-        const float s = b[j].lo[k] + b[j].hi[k];
-        b[j].lo[k] = s * 0.5f; // the centre
-        lo[k] = std_min(lo[k], b[j].lo[k]);
-        hi[k] = std_max(hi[k], b[j].lo[k]);
+      for (int j = 0; j < kTileItems; j++) {
+        if (j >= ipw)
+          break;
+#pragma unroll
+        for (int k = 0; k < 3; k++) {
+          const float s = b[j].lo[k] + b[j].hi[k];
+          b[j].lo[k] = s * 0.5f; // the centre
+          lo[k] = std_min(lo[k], b[j].lo[k]);
+          hi[k] = std_max(hi[k], b[j].lo[k]);
+        }
       }
     }
     wave_reduce_box(lo, hi);
@@ -1025,7 +1048,7 @@ k_tile_sort(const KeyT* __restrict__ kin, KeyT* __restrict__ kout,
         lo[k] = std_min(lo[k], s_box[ww][k]);
         hi[k] = std_max(hi[k], s_box[ww][3 + k]);
       }
-    if (tid == 0)
+    if (tid == 0 && blockIdx.x == 0)
 #pragma unroll
       for (int k = 0; k < 3; k++) {
         bounds_out[k] = lo[k];
@@ -1039,7 +1062,7 @@ k_tile_sort(const KeyT* __restrict__ kin, KeyT* __restrict__ kout,
         break;
       const uint32_t li = lbase + uint32_t(j) * kWave;
       key[j] = morton_code<KeyT>(b[j].lo[0], b[j].lo[1], b[j].lo[2], lo, scale);
-      val[j] = li;
+      val[j] = start + li;
       aux[j] = 0u;
       if (li < m) {
         k_and &= key[j];
@@ -1246,6 +1269,59 @@ k_tile_sort(const KeyT* __restrict__ kin, KeyT* __restrict__ kout,
     if (VALS)
       vout[start + i] = s_vals[i];
   }
+}
+
+// Joins up to kMergeChunks sorted chunks of `chunk` keys kin (a power of two;
+// the last one may be shorter): a key's place is the sum over the chunks of the
+// number of their keys before it (equal keys: of earlier chunks, so ids stay in
+// order).  Its searches step through all chunks together, log2(chunk) + 1
+// dependent loads in all.  Builds of 4,097 to 65,535 primitives take these two
+// launches whatever their codes' distribution.  One global digit before bucket
+// sorts is no faster on an even scene (build of 60,000 triangles, 63-bit codes:
+// 88 us, 89 so), and a bucket that holds most keys is one workgroup's work (an
+// outlier beside a cluster: 691 us, 104 so; every digit by reduce-then-scan:
+// 203).
+constexpr int kMergeChunks = int(lbvh_eng::kChunkSortMax / lbvh_eng::kHybridTileCap);
+constexpr int kMergeBlock = 256;
+
+template<typename KeyT, bool VALS>
+__global__ __launch_bounds__(kMergeBlock) void
+k_merge_chunks(const KeyT* __restrict__ kin, KeyT* __restrict__ kout,
+               const uint32_t* __restrict__ vin, uint32_t* __restrict__ vout, uint32_t n,
+               uint32_t chunk)
+{
+  const uint32_t i = blockIdx.x * kMergeBlock + threadIdx.x;
+  if (i >= n)
+    return;
+  const KeyT key = kin[i];
+  const uint32_t own = blockIdx.x * kMergeBlock / chunk; // a block's keys lie in one chunk
+  const uint32_t chunks = (n + chunk - 1) / chunk;
+  uint32_t below[kMergeChunks];
+#pragma unroll
+  for (int c = 0; c < kMergeChunks; c++)
+    below[c] = 0;
+  for (uint32_t step = chunk; step > 0; step >>= 1) {
+    KeyT probe[kMergeChunks];
+#pragma unroll
+    for (int c = 0; c < kMergeChunks; c++) {
+      const uint32_t at = uint32_t(c) * chunk + below[c] + step - 1;
+      probe[c] = kin[at < n ? at : n - 1];
+    }
+#pragma unroll
+    for (int c = 0; c < kMergeChunks; c++) {
+      const uint32_t to = below[c] + step;
+      const bool before = uint32_t(c) < own ? probe[c] <= key : probe[c] < key;
+      if (to <= chunk && uint32_t(c) * chunk + to <= n && before)
+        below[c] = to;
+    }
+  }
+  uint32_t dst = i - own * chunk;
+#pragma unroll
+  for (int c = 0; c < kMergeChunks; c++)
+    dst += (uint32_t(c) < chunks && uint32_t(c) != own) ? below[c] : 0u;
+  kout[dst] = key;
+  if (VALS)
+    vout[dst] = vin[i];
 }
 
 // Ranges longer than kHybridTileCap: one workgroup per range, stable 8-bit
@@ -1512,11 +1588,40 @@ bucket_sorts(int key_bits, uint64_t n, KeyT* src, KeyT* dst, uint32_t* vsrc, uin
   const uint32_t tiles = uint32_t((n + kHybridTileKeys - 1) / kHybridTileKeys);
   hipLaunchKernelGGL((k_tile_sort<KeyT, VALS, kTileBuckets>), dim3(tiles), dim3(kTileThreads), 0,
                      s, src, dst, vsrc, vdst, uint32_t(n), hi, big, big_count,
-                     uint32_t(big_cap), nullptr, nullptr);
+                     uint32_t(big_cap), nullptr, nullptr, 0u, nullptr, 0u);
   if (n > kHybridTileCap) // else no range is too long for the tile sort
     hipLaunchKernelGGL((k_big_sort<KeyT, VALS>), dim3(kBigBlocks), dim3(kTileThreads), 0, s, src,
                        dst, vsrc, vdst, key_bits, big, big_count, uint32_t(big_cap));
   *in_b = dst_is_b;
+  return hipGetLastError();
+}
+
+// Keys per workgroup of a sort without global digits: all that fit, else 16
+// chunks of the same power of two, at least 1,024.  Builds of 4,097 / 16,384 /
+// 32,768 triangles, 63-bit codes: 79 / 85 / 87 us in chunks of 4,096, 59 / 63 /
+// 69 us so (more chunks, each sorted sooner).
+static uint32_t
+sort_chunk(uint64_t n)
+{
+  if (n <= kHybridTileCap)
+    return kHybridTileCap;
+  uint32_t chunk = 1024;
+  while (uint64_t(chunk) * kMergeChunks < n)
+    chunk <<= 1;
+  return chunk;
+}
+
+// Sorted chunks in b; more than one is merged into a.
+template<typename KeyT, bool VALS>
+static hipError_t
+merge_chunks(uint64_t n, uint32_t chunk, const KeyT* kb, KeyT* ka, const uint32_t* vb,
+             uint32_t* va, bool* in_b, hipStream_t s)
+{
+  *in_b = n <= chunk;
+  if (n > chunk)
+    hipLaunchKernelGGL((k_merge_chunks<KeyT, VALS>),
+                       dim3(uint32_t((n + kMergeBlock - 1) / kMergeBlock)), dim3(kMergeBlock), 0, s,
+                       kb, ka, vb, va, uint32_t(n), chunk);
   return hipGetLastError();
 }
 
@@ -1531,14 +1636,14 @@ run_hybrid(int key_bits, uint64_t n, KeyT* ka, KeyT* kb, uint32_t* va, uint32_t*
   const int gd = cfg.global_digits;
   if (gd < 0 || gd >= passes)
     return hipErrorInvalidValue;
-  if (gd == 0) { // one range, in the LDS of one workgroup
-    if (n > kHybridTileCap)
+  if (gd == 0) {
+    if (n > kChunkSortMax)
       return hipErrorInvalidValue;
-    hipLaunchKernelGGL((k_tile_sort<KeyT, VALS, kTileKeys>), dim3(1), dim3(kTileThreads), 0, s, ka,
-                       kb, nullptr, vb, uint32_t(n), DigitAt{}, nullptr, nullptr, 0u, nullptr,
-                       nullptr);
-    *in_b = true;
-    return hipGetLastError();
+    const uint32_t chunk = sort_chunk(n);
+    hipLaunchKernelGGL((k_tile_sort<KeyT, VALS, kTileKeys>), dim3(uint32_t((n + chunk - 1) / chunk)),
+                       dim3(kTileThreads), 0, s, ka, kb, nullptr, vb, uint32_t(n), DigitAt{},
+                       nullptr, nullptr, 0u, nullptr, nullptr, chunk, nullptr, 0u);
+    return merge_chunks<KeyT, VALS>(n, chunk, kb, ka, vb, va, in_b, s);
   }
   uint32_t chunk_tiles = 1;
   const uint32_t groups = rts_groups(n, cfg, &chunk_tiles);
@@ -1659,39 +1764,46 @@ dispatch(int key_bits, uint64_t n, KeyT* ka, KeyT* kb, uint32_t* va, uint32_t* v
 }
 
 template<typename KeyT, bool VALS>
-static void
-small_sort(const float* prims, int kind, uint64_t n, float* bounds, void* keys, uint32_t* ids,
+static hipError_t
+small_sort(const float* prims, int kind, uint64_t n, const float* cent, const float* partials,
+           float* bounds, void* keys_a, void* keys_b, uint32_t* ids_a, uint32_t* ids_b, bool* in_b,
            hipStream_t s)
 {
-  KeyT* k = static_cast<KeyT*>(keys);
-  if (kind == kPrimTriangle)
+  KeyT* ka = static_cast<KeyT*>(keys_a);
+  KeyT* kb = static_cast<KeyT*>(keys_b);
+  const uint32_t chunk = sort_chunk(n);
+  if (n > chunk)
+    hipLaunchKernelGGL((k_tile_sort<KeyT, VALS, kTileCentres>),
+                       dim3(uint32_t((n + chunk - 1) / chunk)), dim3(kTileThreads), 0, s, nullptr,
+                       kb, nullptr, ids_b, uint32_t(n), DigitAt{}, nullptr, nullptr, 0u, cent,
+                       bounds, chunk, partials, centroid_partials_needed(n));
+  else if (kind == kPrimTriangle)
     hipLaunchKernelGGL((k_tile_sort<KeyT, VALS, kTileTriangles>), dim3(1), dim3(kTileThreads), 0,
-                       s, nullptr, k, nullptr, ids, uint32_t(n), DigitAt{}, nullptr, nullptr, 0u,
-                       prims, bounds);
+                       s, nullptr, kb, nullptr, ids_b, uint32_t(n), DigitAt{}, nullptr, nullptr,
+                       0u, prims, bounds, chunk, nullptr, 0u);
   else
     hipLaunchKernelGGL((k_tile_sort<KeyT, VALS, kTileBoxes>), dim3(1), dim3(kTileThreads), 0, s,
-                       nullptr, k, nullptr, ids, uint32_t(n), DigitAt{}, nullptr, nullptr, 0u,
-                       prims, bounds);
+                       nullptr, kb, nullptr, ids_b, uint32_t(n), DigitAt{}, nullptr, nullptr, 0u,
+                       prims, bounds, chunk, nullptr, 0u);
+  return merge_chunks<KeyT, VALS>(n, chunk, kb, ka, ids_b, ids_a, in_b, s);
 }
 
 hipError_t
-launch_small_sort(int code_bits, const float* prims, int kind, uint64_t n, float* bounds,
-                  void* keys, uint32_t* ids, hipStream_t s)
+launch_small_sort(int code_bits, const float* prims, int kind, uint64_t n, const float* cent,
+                  const float* partials, float* bounds, void* keys_a, void* keys_b,
+                  uint32_t* ids_a, uint32_t* ids_b, bool* in_b, hipStream_t s)
 {
-  if (n < 2 || n > kHybridTileCap || (code_bits != 30 && code_bits != 63))
+  if (n < 2 || n > kChunkSortMax || (code_bits != 30 && code_bits != 63))
     return hipErrorInvalidValue;
-  if (code_bits == 30) {
-    if (ids)
-      small_sort<uint32_t, true>(prims, kind, n, bounds, keys, ids, s);
-    else
-      small_sort<uint32_t, false>(prims, kind, n, bounds, keys, nullptr, s);
-  } else {
-    if (ids)
-      small_sort<uint64_t, true>(prims, kind, n, bounds, keys, ids, s);
-    else
-      small_sort<uint64_t, false>(prims, kind, n, bounds, keys, nullptr, s);
-  }
-  return hipGetLastError();
+  if (code_bits == 30)
+    return ids_a ? small_sort<uint32_t, true>(prims, kind, n, cent, partials, bounds, keys_a,
+                                              keys_b, ids_a, ids_b, in_b, s)
+                 : small_sort<uint32_t, false>(prims, kind, n, cent, partials, bounds, keys_a,
+                                               keys_b, nullptr, nullptr, in_b, s);
+  return ids_a ? small_sort<uint64_t, true>(prims, kind, n, cent, partials, bounds, keys_a, keys_b,
+                                            ids_a, ids_b, in_b, s)
+               : small_sort<uint64_t, false>(prims, kind, n, cent, partials, bounds, keys_a,
+                                             keys_b, nullptr, nullptr, in_b, s);
 }
 
 hipError_t

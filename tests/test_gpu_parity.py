@@ -161,6 +161,33 @@ def test_small_builds_match_oracle(ctx, n, dist):
         bvh.destroy()
 
 
+@pytest.mark.parametrize("kind", ["one-cluster-and-outlier", "duplicates", "two-clusters"])
+@pytest.mark.parametrize("n", [4097, 5120, 8193, 16384, 16385, 32768, 32769, 65535])
+def test_skewed_small_builds_sort_in_chunks(ctx, kind, n):
+    """Builds of 4,097 to 65,535 primitives sort in chunks that are merged by
+    ranks, at the sizes where the chunks change or the last one is short, and
+    not by a global digit, whose fullest bucket would be one workgroup's work;
+    equal codes stay in id order across chunks."""
+    tri = _hybrid_edge_scene(kind, n, 700 + n)
+    for bits, leaf in [(30, 1), (63, 1), (63, 0)]:
+        bvh = ctx.build_triangles(tri, code_bits=bits, leaf_order=leaf, keep_codes=leaf == 1)
+        info = bvh.info()
+        assert (info.sort_strategy, info.sort_global_digits) == (3, 0)
+        on, _, osc, oids = oracle.build(tri, bits, leaf)
+        if leaf == 1:
+            sc, ids, _ = bvh.codes()
+            assert np.array_equal(sc, osc)
+            assert np.array_equal(ids, oids)
+        assert bvh.nodes().tobytes() == on.tobytes()
+        bvh.destroy()
+    p0, p1, p2 = tri[:, 0:3], tri[:, 0:3] - tri[:, 3:6], tri[:, 0:3] + tri[:, 6:9]
+    box = np.concatenate([np.minimum(np.minimum(p0, p1), p2), np.maximum(np.maximum(p0, p1), p2)],
+                         axis=1).astype(np.float64)
+    for leaf in (0, 1):
+        want, _, _ = oracle.build_f64(box, leaf)
+        assert ctx.build_aabbs_f64(box, leaf).tobytes() == want.tobytes()
+
+
 @pytest.mark.parametrize("extent", [0.01, 2.0 ** 24, 2.0 ** 25, 3e7, 1e8, 1e30])
 @pytest.mark.parametrize("n", [200, 4096, 4097, 60000, 70000])
 def test_every_sort_orders_all_code_bits(ctx, n, extent):
