@@ -245,6 +245,16 @@ def _is_device(x):
     return False
 
 
+def _torch_streams(arrays):
+    """torch's current stream on every device that holds a torch tensor of
+    `arrays`."""
+    devices = {x.device for x in arrays if _is_torch(x)}
+    if not devices:
+        return []
+    from torch.cuda import current_stream
+    return [ctypes.c_void_p(current_stream(d).cuda_stream) for d in devices]
+
+
 def _numel(x):
     return int(x.numel())
 
@@ -439,7 +449,6 @@ class Batch:
             if not _is_device(ray_offsets):
                 raise ValueError("device rays need device ray offsets")
             m = _check_dev(rays, "rays", (np.float32,), width=8)
-            self.ctx._after(rays)
             _check_dev(ray_offsets, "ray offsets", (np.uint64, np.int64),
                        count=self.n_scenes + 1)
             if out is None:
@@ -449,6 +458,7 @@ class Batch:
                 uv = DeviceArray((m, 2), np.float32) if with_uv else None
             else:
                 prim, t, uv = _check_dev_out(out, m, with_uv)
+            self.ctx._after(rays, ray_offsets, prim, t, uv)
             self.ctx._check(lib().lbvh_batch_trace_closest_device(
                 self.ctx.handle, self.handle, _dptr(rays), _dptr(ray_offsets), m, mode,
                 _dptr(prim), _dptr(t), _dptr(uv) if uv is not None else None))
@@ -632,13 +642,12 @@ class Context:
             raw = ctypes.c_void_p(int(getattr(stream, "cuda_stream", stream)))
         self._check(lib().lbvh_ctx_set_stream(self.handle, raw))
 
-    def _after(self, x):
-        """Orders the context after the stream that torch is on, when `x` is a
-        torch tensor: what it holds may still be being written there."""
-        if _is_torch(x):
-            from torch.cuda import current_stream
-            self._check(lib().lbvh_ctx_wait_stream(
-                self.handle, ctypes.c_void_p(current_stream(x.device).cuda_stream)))
+    def _after(self, *arrays):
+        """Orders the context after the stream that torch is on, when a call's
+        inputs or outputs (`arrays`; None for one left out) have a torch tensor
+        among them: it may still be being written, or read, there."""
+        for stream in _torch_streams(arrays):
+            self._check(lib().lbvh_ctx_wait_stream(self.handle, stream))
 
     def synchronize(self):
         self._check(lib().lbvh_ctx_synchronize(self.handle))
@@ -720,7 +729,6 @@ class Context:
         opts = _make_opts(63, leaf_order, False, sort_digit_bits, sort_tile, sort_strategy)
         if _is_device(boxes):
             n = _check_dev(boxes, "boxes", (np.float64,), width=6)
-            self._after(boxes)
             if out is None:
                 if _is_torch(boxes):
                     import torch
@@ -731,6 +739,7 @@ class Context:
             nbytes = _dev_nbytes(out)
             if nbytes < 64 * max(n - 1, 0):
                 raise ValueError("out holds fewer than 64 (n - 1) bytes")
+            self._after(boxes, out)
             self._check(lib().lbvh_build_aabbs_f64_device(self.handle, _dptr(boxes), n,
                                                           ctypes.byref(opts), _dptr(out)))
             return out
@@ -755,7 +764,6 @@ class Context:
             m = _check_dev(rays, "rays", (np.float64,), width=8)
             if _dev_nbytes(nodes) < 64 * max(n - 1, 0):
                 raise ValueError("nodes hold fewer than 64 (n - 1) bytes")
-            self._after(rays)
             if out is None:
                 from .hip import DeviceArray
                 prim = DeviceArray(m, np.uint64)
@@ -767,6 +775,7 @@ class Context:
                 _check_dev(t, "t", (np.float64,), at_least=m)
                 if uv is not None:
                     _check_dev(uv, "uv", (np.float64,), at_least=2 * m)
+            self._after(nodes, tri, rays, prim, t, uv)
             self._check(lib().lbvh_trace_closest_f64_device(
                 self.handle, _dptr(nodes), n, _dptr(tri), _dptr(rays), m, mode, _dptr(prim),
                 _dptr(t), _dptr(uv) if uv is not None else None))
@@ -826,7 +835,6 @@ class Context:
         reading)."""
         if _is_device(rays):
             m = _check_dev(rays, "rays", (np.float32,), width=8)
-            self._after(rays)
             if out is None:
                 from .hip import DeviceArray
                 prim = DeviceArray(m, np.uint32)
@@ -834,6 +842,7 @@ class Context:
                 uv = DeviceArray((m, 2), np.float32) if with_uv else None
             else:
                 prim, t, uv = _check_dev_out(out, m, with_uv)
+            self._after(rays, prim, t, uv)
             self._check(lib().lbvh_trace_closest_device(self.handle, bvh.handle, _dptr(rays), m,
                                                         mode, _dptr(prim), _dptr(t),
                                                         _dptr(uv) if uv is not None else None))

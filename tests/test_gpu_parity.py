@@ -584,6 +584,95 @@ def test_torch_inputs_still_being_written_are_waited_for():
     assert "torch order ok" in r.stdout
 
 
+TORCH_ORDER_MIXED = r"""
+import sys, numpy as np
+import torch
+sys.path.insert(0, %r)
+import lbvh_amd, oracle
+from lbvh_amd import workload as W
+from lbvh_amd.hip import DeviceArray
+v, tri = W.scene_uniform(1, 3000, 0.02)
+rays = W.primary_rays(32, 32)
+ctx = lbvh_amd.Context(0)
+big = torch.randn(6144, 6144, device="cuda")
+
+def late(x):
+    "x on the GPU, written only after a few ms of other work"
+    src = torch.from_numpy(np.ascontiguousarray(x).view(np.uint8).reshape(-1)).cuda()
+    d = torch.zeros_like(src)
+    torch.cuda.synchronize()
+    for _ in range(4):
+        y = big @ big
+    d.copy_(src)
+    return d
+
+def outputs(m, prim, t):
+    "written by torch late: the hits have to come after that"
+    o = tuple(torch.zeros(s, dtype=d, device="cuda") for s, d in ((m, prim), (m, t), ((m, 2), t)))
+    torch.cuda.synchronize()
+    for _ in range(4):
+        y = big @ big
+    for x in o:
+        x.fill_(7)
+    return o
+
+# FP64: nodes, then triangles, then outputs still being written, the rest not torch's
+boxes = np.concatenate([c.min(axis=1) if k == 0 else c.max(axis=1) for c in [v.reshape(-1, 3, 3)]
+                        for k in (0, 1)], axis=1).astype(np.float64)
+tri64, rays64 = tri.astype(np.float64), rays.astype(np.float64)
+on, _, _ = oracle.build_f64(boxes, 1)
+op, ot, ouv = oracle.trace_f64(on, tri64, rays64, 0)
+for k in range(4):
+    nodes, t64, out = (DeviceArray.from_host(on.view(np.uint64).reshape(-1)),
+                       DeviceArray.from_host(tri64), None)
+    r64 = DeviceArray.from_host(rays64)
+    if k == 0:
+        nodes = late(on).view(torch.int64)
+    elif k == 1:
+        t64 = late(tri64).view(torch.float64).reshape(-1, 12)
+    elif k == 2:
+        out = outputs(len(rays), torch.int64, torch.float64)
+    else:
+        d_boxes, nodes = DeviceArray.from_host(boxes), outputs(2999 * 8, torch.int64, torch.float64)[0]
+        ctx.build_aabbs_f64(d_boxes, 1, out=nodes)
+    prim, t, uv = ctx.trace_f64(nodes, t64, r64, out=out)
+    ctx.synchronize()
+    host = lambda x: x.cpu().numpy() if isinstance(x, torch.Tensor) else x.numpy()
+    assert np.array_equal(host(prim).view(np.uint64), op), k
+    assert np.array_equal(host(t).view(np.uint64), ot.view(np.uint64)), k
+    torch.cuda.synchronize()
+# a batch: ray offsets, then outputs
+off = np.array([0, 1000, 3000], np.uint64)
+roff = np.array([0, 500, 1024], np.uint64)
+batch = ctx.build_batch(DeviceArray.from_host(tri), off, leaf_order=1)
+want = batch.trace(rays, roff)
+for k in range(2):
+    d_rays, d_off, out = DeviceArray.from_host(rays), DeviceArray.from_host(roff), None
+    if k == 0:
+        d_off = late(roff).view(torch.int64)
+    else:
+        out = outputs(len(rays), torch.int32, torch.float32)
+    prim, t, uv = batch.trace(d_rays, d_off, out=out)
+    ctx.synchronize()
+    assert np.array_equal(host(prim).view(np.uint32), want[0]), k
+    assert np.array_equal(host(t).view(np.uint32), want[1].view(np.uint32)), k
+    torch.cuda.synchronize()
+print("torch mixed order ok")
+"""
+
+
+def test_any_torch_argument_orders_the_call():
+    """Inputs and outputs alike: a call starts after torch's current stream
+    when any one of its arrays is a torch tensor and the others are not."""
+    import subprocess
+    import sys
+    from conftest import ROOT
+    r = subprocess.run([sys.executable, "-c", TORCH_ORDER_MIXED % ROOT], capture_output=True,
+                       text=True, timeout=180)
+    assert r.returncode == 0, r.stdout + r.stderr
+    assert "torch mixed order ok" in r.stdout
+
+
 def test_cpp_dropin_conformance(tmp_path):
     """The C++ drop-in header (include/lbvh_mi355x.hpp) used with the
     reference's call shapes: builder over triangles and over a user primitive
