@@ -488,6 +488,13 @@ void lbvh_server_destroy(lbvh_server* server);
  * new scene's id for a new scene). */
 lbvh_status lbvh_server_submit(lbvh_server* server, const lbvh_request* req,
                                uint64_t* ticket, uint64_t* scene);
+/* As lbvh_server_submit, for a device request whose arrays another stream of
+ * the server's device (a hipStream_t; NULL: the default stream) may still be
+ * writing or reading: the request's work starts after the work queued on
+ * `stream` so far.  Does not block the host.  While the stream is being
+ * captured into a graph the order is the caller's. */
+lbvh_status lbvh_server_submit_after(lbvh_server* server, const lbvh_request* req, void* stream,
+                                     uint64_t* ticket, uint64_t* scene);
 /* Waits for a request and collects it: its status is returned. */
 lbvh_status lbvh_server_wait(lbvh_server* server, uint64_t ticket,
                              lbvh_request_info* info);

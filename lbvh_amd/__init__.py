@@ -174,6 +174,8 @@ SIGNATURES = {
     "lbvh_server_destroy": (None, [VP]),
     "lbvh_server_submit": (ctypes.c_int, [VP, ctypes.POINTER(Request), ctypes.POINTER(U64),
                                           ctypes.POINTER(U64)]),
+    "lbvh_server_submit_after": (ctypes.c_int, [VP, ctypes.POINTER(Request), VP,
+                                                ctypes.POINTER(U64), ctypes.POINTER(U64)]),
     "lbvh_server_wait": (ctypes.c_int, [VP, U64, ctypes.POINTER(RequestInfo)]),
     "lbvh_server_poll": (ctypes.c_int, [VP, U64, ctypes.POINTER(RequestInfo)]),
     "lbvh_server_release_scene": (ctypes.c_int, [VP, U64]),
@@ -519,6 +521,7 @@ class Server:
         req = Request()
         req.scene = scene
         keep = []
+        after = []
         if _is_device(rays):
             m = _check_dev(rays, "rays", (np.float32,), width=8)
             if tri is not None:
@@ -539,6 +542,7 @@ class Server:
                 req.tri48 = _dptr(tri).value
                 req.n_tri = _numel(tri) // 12
             keep = [rays, tri]
+            after = _torch_streams((rays, tri, prim, t, uv))
         else:
             r = np.ascontiguousarray(rays, dtype=np.float32).reshape(-1, 8)
             m = r.shape[0]
@@ -557,8 +561,12 @@ class Server:
             keep.append(r)
         req.n_rays = m
         ticket, sid = U64(), U64()
-        st = lib().lbvh_server_submit(self.handle, ctypes.byref(req), ctypes.byref(ticket),
-                                      ctypes.byref(sid))
+        if after:  # tensors on the server's device: its current stream is the one
+            st = lib().lbvh_server_submit_after(self.handle, ctypes.byref(req), after[0],
+                                                ctypes.byref(ticket), ctypes.byref(sid))
+        else:
+            st = lib().lbvh_server_submit(self.handle, ctypes.byref(req), ctypes.byref(ticket),
+                                          ctypes.byref(sid))
         if st != 0:
             raise LbvhError(st, "lbvh_server_submit")
         self._live[ticket.value] = (keep, prim, t, uv)

@@ -162,6 +162,17 @@ capturing(hipStream_t s)
 
 } // namespace
 
+hipError_t
+stream_pending(hipStream_t s)
+{
+  if (capturing(s))
+    return hipSuccess;
+  const hipError_t e = hipStreamQuery(s);
+  if (e != hipSuccess)
+    (void)hipGetLastError();
+  return e;
+}
+
 uint64_t
 pool_cached(int device)
 {
@@ -842,12 +853,11 @@ lbvh_ctx_wait_stream(lbvh_ctx* c, void* stream)
   lbvh_status st = set_device(c);
   if (st != LBVH_OK)
     return st;
-  if (capturing(s) || capturing(c->stream))
+  if (capturing(c->stream))
     return LBVH_OK;
-  hipError_t e = hipStreamQuery(s); // idle, as for inputs that are ready: nothing to wait for
+  const hipError_t e = stream_pending(s); // idle, as for inputs that are ready: nothing to wait for
   if (e == hipSuccess)
     return LBVH_OK;
-  (void)hipGetLastError();
   if (e != hipErrorNotReady)
     return hip_fail(c, e, "hipStreamQuery");
   if (!c->wait_event)

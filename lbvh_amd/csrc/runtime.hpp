@@ -151,6 +151,10 @@ void pool_release(int device);
 // hipMalloc; what the pool keeps is given back and the call repeated if it fails.
 hipError_t dev_malloc(int device, void** p, uint64_t bytes);
 lbvh_status set_device(lbvh_ctx* c);
+// Whether work queued on the stream may still run (hipErrorNotReady) or not
+// (hipSuccess; also while it is being captured: its order is then the
+// caller's); another error is a failed query.
+hipError_t stream_pending(hipStream_t s);
 // Finds this device's copy of the allocation-free build's scratch array (the
 // device must be current; once per device).
 lbvh_status noalloc_init(lbvh_ctx* c);

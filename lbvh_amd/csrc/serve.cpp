@@ -151,9 +151,20 @@ struct Req
   uint64_t footprint = 0; // device bytes reserved while active
   Buf d_rays, d_out, h_in, h_out;
   hipEvent_t ev_ready = nullptr;
+  hipEvent_t ev_after = nullptr; // the caller's stream's work that it waits for
   int launch = -1; // traversal launch it joined
   uint32_t coalesced = 0;
   double t_submit = 0, t_admit = 0, t_ready = 0, t_done = 0;
+
+  void destroy_events()
+  {
+    for (hipEvent_t* e : { &ev_ready, &ev_after }) {
+      if (*e)
+        (void)hipEventDestroy(*e);
+      *e = nullptr;
+    }
+  }
+  ~Req() { destroy_events(); }
 };
 
 struct Launch
@@ -406,6 +417,9 @@ start(lbvh_server* s, Req* q, Scene* sc)
     return bad(LBVH_E_INVALID, "the scene's build failed");
   const bool dev = on_device(q);
   const float* tri_src = q->r.tri48;
+  // its traversal is launched when the lane's work has finished, so that waits too
+  if (q->ev_after && hipStreamWaitEvent(st, q->ev_after, 0) != hipSuccess)
+    return bad(LBVH_E_HIP, "waiting for the caller's stream failed");
   if (!dev) {
     const uint64_t in_bytes = nr * 32 + ntri * 48;
     if (in_bytes) {
@@ -614,9 +628,7 @@ finish(lbvh_server* s, Req* q)
   s->mem_used += s->lane_ws; // lane workspace grows once and stays
   s->lane_ws = 0;
   q->footprint = 0;
-  if (q->ev_ready)
-    (void)hipEventDestroy(q->ev_ready);
-  q->ev_ready = nullptr;
+  q->destroy_events();
   q->st = St::Done;
   q->t_done = us_since(s);
   if (q->status == LBVH_OK)
@@ -824,8 +836,12 @@ lbvh_server_destroy(lbvh_server* s)
   delete s;
 }
 
-lbvh_status
-lbvh_server_submit(lbvh_server* s, const lbvh_request* r, uint64_t* ticket, uint64_t* scene_out)
+} // extern "C"
+
+// after: the stream whose work so far the request waits for, or nullptr for none.
+static lbvh_status
+submit(lbvh_server* s, const lbvh_request* r, const hipStream_t* after, uint64_t* ticket,
+       uint64_t* scene_out)
 {
   if (!s || !r || !ticket)
     return LBVH_E_INVALID;
@@ -848,9 +864,18 @@ lbvh_server_submit(lbvh_server* s, const lbvh_request* r, uint64_t* ticket, uint
     delete q;
     return LBVH_E_HIP;
   }
+  if (after) {
+    const hipError_t e = stream_pending(*after);
+    if (e != hipSuccess &&
+        (e != hipErrorNotReady ||
+         hipEventCreateWithFlags(&q->ev_after, hipEventDisableTiming) != hipSuccess ||
+         hipEventRecord(q->ev_after, *after) != hipSuccess)) {
+      delete q;
+      return LBVH_E_HIP;
+    }
+  }
   std::lock_guard<std::mutex> g(s->mu);
   if (s->stop) {
-    (void)hipEventDestroy(q->ev_ready);
     delete q;
     return LBVH_E_BUSY;
   }
@@ -862,7 +887,6 @@ lbvh_server_submit(lbvh_server* s, const lbvh_request* r, uint64_t* ticket, uint
     if (!made) {
       if (sc)
         destroy_scene(sc);
-      (void)hipEventDestroy(q->ev_ready);
       delete q;
       return LBVH_E_OOM;
     }
@@ -876,12 +900,10 @@ lbvh_server_submit(lbvh_server* s, const lbvh_request* r, uint64_t* ticket, uint
   } else {
     auto it = s->scenes.find(r->scene);
     if (it == s->scenes.end()) {
-      (void)hipEventDestroy(q->ev_ready);
       delete q;
       return LBVH_E_INVALID;
     }
     if ((r->tri48 && r->n_tri != it->second->n) || it->second->failed) {
-      (void)hipEventDestroy(q->ev_ready);
       delete q;
       return LBVH_E_INVALID;
     }
@@ -899,6 +921,22 @@ lbvh_server_submit(lbvh_server* s, const lbvh_request* r, uint64_t* ticket, uint
     *scene_out = q->scene;
   s->cv_work.notify_all();
   return LBVH_OK;
+}
+
+extern "C" {
+
+lbvh_status
+lbvh_server_submit(lbvh_server* s, const lbvh_request* r, uint64_t* ticket, uint64_t* scene_out)
+{
+  return submit(s, r, nullptr, ticket, scene_out);
+}
+
+lbvh_status
+lbvh_server_submit_after(lbvh_server* s, const lbvh_request* r, void* stream, uint64_t* ticket,
+                         uint64_t* scene_out)
+{
+  const hipStream_t after = static_cast<hipStream_t>(stream);
+  return submit(s, r, &after, ticket, scene_out);
 }
 
 static void

@@ -253,3 +253,63 @@ def test_server_host_refit_of_device_scene_leaves_borrowed_buffer(ctx):
     assert np.array_equal(uv.view(np.uint32), e1[2].view(np.uint32))
     assert d_tri0.numpy().tobytes() == tri0.tobytes(), "the borrowed device buffer was written"
     srv.close()
+
+
+TORCH_REQUESTS = r"""
+import sys, numpy as np
+import torch
+sys.path.insert(0, %r)
+import lbvh_amd
+from lbvh_amd import workload as W
+tri = [W.make_triangles(W.cluster_vertices(600 + k, n)) for k, n in enumerate((3000, 50000))]
+moved = W.make_triangles(W.perturb(9, W.cluster_vertices(601, 50000), 2e-4))
+rays = W.primary_rays(64, 48)
+ctx = lbvh_amd.Context(0)
+trees = [ctx.build_triangles(x, code_bits=63, leaf_order=1) for x in tri]
+want = [ctx.trace(b, rays) for b in trees]
+ctx.refit_triangles(trees[1], moved)
+want.append(ctx.trace(trees[1], rays))
+big = torch.randn(6144, 6144, device="cuda")
+src = [torch.from_numpy(x).cuda() for x in tri + [moved, rays]]
+srv = lbvh_amd.Server(0)
+for stream in (torch.cuda.default_stream(), torch.cuda.Stream()):
+    d = [torch.zeros_like(x) for x in src]
+    out = [(torch.zeros(len(rays), dtype=torch.int32, device="cuda"),
+            torch.zeros(len(rays), device="cuda"), torch.zeros(len(rays), 2, device="cuda"))
+           for _ in want]
+    torch.cuda.synchronize()
+    with torch.cuda.stream(stream):
+        tickets, ids = [], []
+        for k in range(3):  # two scenes, a refit of the second
+            for _ in range(4):
+                y = big @ big  # a few ms before the arrays are written
+            d[k].copy_(src[k])
+            if k == 0:
+                d[3].copy_(src[3])
+            for x in out[k]:
+                x.fill_(7)
+            ticket, sid = srv.submit(d[3], ids[1] if k == 2 else 0, d[k], out=out[k])
+            tickets.append(ticket)
+            ids.append(sid)
+    for k, ticket in enumerate(tickets):
+        p, t, uv, _ = srv.wait(ticket)
+        assert np.array_equal(p.cpu().numpy().view(np.uint32), want[k][0]), k
+        assert np.array_equal(t.cpu().numpy().view(np.uint32), want[k][1].view(np.uint32)), k
+        assert np.array_equal(uv.cpu().numpy().view(np.uint32), want[k][2].view(np.uint32)), k
+    torch.cuda.synchronize()
+srv.close()
+print("torch requests ok")
+"""
+
+
+def test_server_requests_wait_for_torch():
+    """Device requests whose torch tensors, inputs and outputs, are still being
+    written on torch's current stream: a new scene, a second one and its refit
+    answer as the plain path does."""
+    import subprocess
+    import sys
+    from conftest import ROOT
+    r = subprocess.run([sys.executable, "-c", TORCH_REQUESTS % ROOT], capture_output=True,
+                       text=True, timeout=180)
+    assert r.returncode == 0, r.stdout + r.stderr
+    assert "torch requests ok" in r.stdout
