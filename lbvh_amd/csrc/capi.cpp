@@ -443,7 +443,7 @@ alloc_bvh(lbvh_ctx* c, lbvh_bvh* b, bool keep_codes)
     *r.p = at;
     at += (r.bytes + 255) & ~uint64_t(255);
   }
-  b->bytes += total;
+  b->bytes += b->block_held; // a block from the pool may be larger than asked for
   return LBVH_OK;
 }
 
@@ -646,9 +646,6 @@ build_common(lbvh_ctx* c, const float* d_prims, int kind, uint64_t n,
     free_bvh(b);
     return st;
   }
-  if (owns)
-    b->bytes += n * (kind == 0 ? 48 : 24);
-
   uint32_t* small = static_cast<uint32_t*>(c->small.p);
   float* cent = static_cast<float*>(c->cent.p);
   SortWorkspace ws;
@@ -1025,6 +1022,7 @@ build_host(lbvh_ctx* c, const float* host, int kind, uint64_t n, const lbvh_buil
     return st;
   }
   (*out)->prims_held = held;
+  (*out)->bytes += held;
   st = sync_and_check(c);
   if (st != LBVH_OK) {
     free_bvh(*out);
@@ -1115,7 +1113,7 @@ lbvh_refit_triangles(lbvh_ctx* c, lbvh_bvh* b, const float* tri)
       return fail(c, LBVH_E_OOM, "device allocation for primitives failed");
     b->d_prims = d;
     b->owns_prims = true;
-    b->bytes += b->n * 48;
+    b->bytes += b->prims_held;
   }
   HIP_TRY(c, hipMemcpyAsync(b->d_prims, tri, b->n * 48, hipMemcpyHostToDevice, c->stream));
   if ((st = queue_refit(c, b)) != LBVH_OK)

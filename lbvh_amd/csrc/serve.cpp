@@ -476,6 +476,14 @@ start(lbvh_server* s, Req* q, Scene* sc)
     sc->bytes = (sc->owns_tri ? ntri * 48 : 0) + sc->bvh->bytes;
     std::lock_guard<std::mutex> g(s->mu);
     s->lane_ws += ws1 - ws0;
+    // a kept block that is larger than the estimate: the request holds the rest
+    // of it, too, from now on (those bytes have just left the pool)
+    const uint64_t est = tree_bytes_estimate(ntri, s->opts.leaf_order);
+    if (sc->bvh->bytes > est) {
+      q->footprint += sc->bvh->bytes - est;
+      s->mem_used += sc->bvh->bytes - est;
+      s->mem_peak = std::max(s->mem_peak, s->mem_used);
+    }
   } else {
     if (sc->has_tree_ev)
       (void)hipStreamWaitEvent(st, sc->ev_tree, 0);

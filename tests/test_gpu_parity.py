@@ -773,6 +773,20 @@ def test_tree_memory_reused_across_threads_and_contexts(leaf):
     assert not bad, bad
 
 
+def test_reported_bytes_are_those_held():
+    """device_bytes counts the whole block that a tree took from a freed one,
+    and its host-built triangles'."""
+    c = lbvh_amd.Context(0)
+    held = []
+    for n in (61234, 60987, 30000):  # no other test's block lies between the first two
+        bvh = c.build_triangles(W.make_triangles(W.uniform_vertices(n, n, 0.01)))
+        held.append(bvh.info().device_bytes)
+        bvh.destroy()
+    assert held[1] == held[0] >= 61234 * (48 + 48)
+    assert 30000 * (48 + 48) <= held[2] < held[0] // 2 + 65536
+    c.close()
+
+
 def test_phase_timing_reports_four_phases(ctx):
     v, tri = W.scene_uniform(1, 65536, 0.01)
     ctx.set_timing(True)

@@ -179,6 +179,30 @@ def test_server_memory_cap_evicts_idle_scenes(ctx):
     srv.close()
 
 
+def test_server_charges_the_memory_that_reused_blocks_hold():
+    """A new scene may take an evicted one's larger block: the server charges
+    the bytes that the scene holds, so trees of slightly falling sizes stay
+    under the cap."""
+    def need(n):  # triangles, tree, workspace share, ray and hit buffers of 64 rays
+        return 48 * n + 52 * n + 4096 + 44 * n + (1 << 20) + 2 * 4096
+    rays = _rays(1, 64)
+    probe = lbvh_amd.Server(0, lanes=1, reserve_prims=65536)
+    base = probe.stats()["memory_used_bytes"]
+    probe.close()
+    srv = lbvh_amd.Server(0, lanes=1, reserve_prims=65536,
+                          memory_cap_bytes=base + need(61234) + 3_800_000)
+    used = []
+    for n in (61234, 60987):  # both do not fit; the first's block and the second request do
+        srv.wait(srv.submit(rays, 0, _scene(n, n))[0])
+        st = srv.stats()
+        used.append(st["memory_used_bytes"] - base - 48 * n)
+    assert st["evictions"] == 1
+    assert used[0] >= 52 * 61234 - 256
+    assert used[1] == used[0], "the second scene holds the first one's block"
+    assert st["memory_peak_bytes"] <= st["memory_cap_bytes"]
+    srv.close()
+
+
 def test_server_rejects_bad_requests():
     srv = lbvh_amd.Server(0)
     with pytest.raises(lbvh_amd.LbvhError):
