@@ -90,6 +90,7 @@ struct TreePool
   {
     void* p;
     uint64_t bytes;
+    const void* owner;
   } kept[kPoolMaxBlocks];
   size_t count = 0;
   uint64_t bytes = 0;
@@ -174,43 +175,61 @@ stream_pending(hipStream_t s)
 }
 
 uint64_t
-pool_cached(int device)
+pool_cached(int device, const void* owner)
 {
   if (!pooled(device))
     return 0;
   std::lock_guard<std::mutex> g(g_pool_mutex);
-  return g_pools[device].bytes;
+  const TreePool& t = g_pools[device];
+  uint64_t bytes = 0;
+  for (size_t k = 0; k < t.count; k++)
+    bytes += t.kept[k].owner == owner ? t.kept[k].bytes : 0;
+  return bytes;
 }
 
 void
-pool_release(int device)
+pool_release(int device, const void* owner)
 {
-  if (pooled(device))
-    pool_trim(device, 0, 0);
+  if (!pooled(device))
+    return;
+  for (;;) {
+    void* p = nullptr;
+    {
+      std::lock_guard<std::mutex> g(g_pool_mutex);
+      TreePool& t = g_pools[device];
+      for (size_t k = 0; k < t.count && !p; k++)
+        if (t.kept[k].owner == owner)
+          p = t.take(k).p;
+    }
+    if (!p)
+      return;
+    (void)hipFree(p); // without the lock: it waits for the device
+  }
 }
 
 hipError_t
 dev_malloc(int device, void** p, uint64_t bytes)
 {
   hipError_t e = hipMalloc(p, bytes);
-  if (e != hipSuccess && pool_cached(device) > 0) {
+  if (e != hipSuccess && pooled(device)) {
     (void)hipGetLastError();
-    pool_release(device);
+    pool_trim(device, 0, 0); // every owner's
     e = hipMalloc(p, bytes);
   }
   return e;
 }
 
 void*
-pool_alloc(int device, uint64_t bytes, hipStream_t stream, uint64_t* held)
+pool_alloc(int device, const void* owner, uint64_t bytes, hipStream_t stream, uint64_t* held)
 {
-  if (pooled(device) && pool_cached(device) >= bytes && !capturing(stream)) {
+  if (pooled(device) && pool_cached(device, owner) >= bytes && !capturing(stream)) {
     // the smallest kept block that fits without wasting more than a quarter
     std::lock_guard<std::mutex> g(g_pool_mutex);
     TreePool& t = g_pools[device];
     size_t best = t.count;
     for (size_t k = 0; k < t.count; k++)
-      if (t.kept[k].bytes >= bytes && t.kept[k].bytes - bytes <= bytes / 4 + (1u << 16) &&
+      if (t.kept[k].owner == owner && t.kept[k].bytes >= bytes &&
+          t.kept[k].bytes - bytes <= bytes / 4 + (1u << 16) &&
           (best == t.count || t.kept[k].bytes < t.kept[best].bytes))
         best = k;
     if (best < t.count) {
@@ -229,7 +248,7 @@ pool_alloc(int device, uint64_t bytes, hipStream_t stream, uint64_t* held)
 }
 
 void
-pool_free(int device, void* p, uint64_t held)
+pool_free(int device, const void* owner, void* p, uint64_t held)
 {
   if (!p)
     return;
@@ -240,7 +259,7 @@ pool_free(int device, void* p, uint64_t held)
       std::lock_guard<std::mutex> g(g_pool_mutex);
       TreePool& t = g_pools[device];
       if (t.contexts > 0 && t.count < kPoolMaxBlocks && t.bytes + held <= kPoolMaxBytes) {
-        t.kept[t.count++] = TreePool::Block{ p, held };
+        t.kept[t.count++] = TreePool::Block{ p, held, owner };
         t.bytes += held;
         return;
       }
@@ -433,7 +452,7 @@ alloc_bvh(lbvh_ctx* c, lbvh_bvh* b, bool keep_codes)
   for (auto& r : req)
     if (r.bytes)
       total += (r.bytes + 255) & ~uint64_t(255);
-  b->block = pool_alloc(c->device, total, c->stream, &b->block_held);
+  b->block = pool_alloc(c->device, c->pool_owner, total, c->stream, &b->block_held);
   if (!b->block)
     return fail(c, LBVH_E_OOM, "device allocation for the tree failed");
   char* at = static_cast<char*>(b->block);
@@ -455,9 +474,9 @@ free_bvh(lbvh_bvh* b)
   int cur = 0;
   (void)hipGetDevice(&cur);
   (void)hipSetDevice(b->device);
-  pool_free(b->device, b->block, b->block_held); // every tree buffer
+  pool_free(b->device, b->pool_owner, b->block, b->block_held); // every tree buffer
   if (b->owns_prims)
-    pool_free(b->device, b->d_prims, b->prims_held);
+    pool_free(b->device, b->pool_owner, b->d_prims, b->prims_held);
   (void)hipSetDevice(cur);
   delete b;
 }
@@ -634,6 +653,7 @@ build_common(lbvh_ctx* c, const float* d_prims, int kind, uint64_t n,
   if (!b)
     return fail(c, LBVH_E_OOM, "host allocation failed");
   b->device = c->device;
+  b->pool_owner = c->pool_owner;
   b->n = n;
   b->code_bits = opts.code_bits;
   b->leaf_order = opts.leaf_order;
@@ -1007,18 +1027,18 @@ build_host(lbvh_ctx* c, const float* host, int kind, uint64_t n, const lbvh_buil
     return st;
   const uint64_t bytes = n * (kind == 0 ? 48 : 24);
   uint64_t held = 0;
-  float* d = static_cast<float*>(pool_alloc(c->device, bytes, c->stream, &held));
+  float* d = static_cast<float*>(pool_alloc(c->device, c->pool_owner, bytes, c->stream, &held));
   if (!d)
     return fail(c, LBVH_E_OOM, "device allocation for primitives failed");
   hipError_t e = hipMemcpyAsync(d, host, bytes, hipMemcpyHostToDevice, c->stream);
   if (e != hipSuccess) {
-    pool_free(c->device, d, held);
+    pool_free(c->device, c->pool_owner, d, held);
     return hip_fail(c, e, "hipMemcpyAsync");
   }
   st = build_common(c, d, kind, n, opts, true, out);
   if (st != LBVH_OK) {
     (void)hipStreamSynchronize(c->stream);
-    pool_free(c->device, d, held);
+    pool_free(c->device, c->pool_owner, d, held);
     return st;
   }
   (*out)->prims_held = held;
@@ -1107,8 +1127,8 @@ lbvh_refit_triangles(lbvh_ctx* c, lbvh_bvh* b, const float* tri)
   if (st != LBVH_OK)
     return st;
   if (!b->owns_prims) {
-    float* d =
-      static_cast<float*>(pool_alloc(c->device, b->n * 48, c->stream, &b->prims_held));
+    float* d = static_cast<float*>(
+      pool_alloc(c->device, b->pool_owner, b->n * 48, c->stream, &b->prims_held));
     if (!d)
       return fail(c, LBVH_E_OOM, "device allocation for primitives failed");
     b->d_prims = d;

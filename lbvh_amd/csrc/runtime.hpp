@@ -62,6 +62,7 @@ struct lbvh_ctx
   hipStream_t own_stream = nullptr;
   hipStream_t stream = nullptr;
   hipEvent_t wait_event = nullptr; // lbvh_ctx_wait_stream
+  const void* pool_owner = nullptr; // whose kept tree memory it uses: a server's lanes the server's
   int timing = 0; // 0 off, 1 per phase, 2 per call
   std::vector<lbvh_rt::EventSet> sets; // pool; sets[0..used) belong to timed calls
   size_t used = 0;
@@ -104,6 +105,7 @@ struct lbvh_bvh
   uint32_t* d_other_end = nullptr; // other end of each internal node's leaf range
   void* block = nullptr;           // the one allocation holding every buffer above
   uint64_t block_held = 0, prims_held = 0; // pool bytes of block and of owned primitives
+  const void* pool_owner = nullptr;        // of the context that made it
   uint64_t bytes = 0;
   lbvh_eng::SortConfig sort;       // the sort configuration the build used
   uint64_t id = 0;                 // unique per tree in the process (refit caches)
@@ -139,15 +141,20 @@ void dev_free(void* p);
 // first; all of it when the device's last context goes, or when an
 // allocation of the engine fails.  pool_free waits for the device first, as
 // hipFree does, so a kept block has no user left on any stream; a block
-// carries no contents from one tree to the next.  Safe from any thread.
+// carries no contents from one tree to the next.  A block is kept for its owner
+// (a server, or all other contexts of the device: nullptr), so that a server
+// counts and frees under its memory cap what its own trees left, no one else's.
+// Safe from any thread.
 constexpr uint64_t kPoolMaxBytes = uint64_t(4) << 30;
 constexpr size_t kPoolMaxBlocks = 64;
 // stream: the caller's; while it is being captured the pool is left alone.
 // *held: the block's bytes, for pool_free.
-void* pool_alloc(int device, uint64_t bytes, hipStream_t stream, uint64_t* held);
-void pool_free(int device, void* p, uint64_t held);
-uint64_t pool_cached(int device);
-void pool_release(int device);
+void* pool_alloc(int device, const void* owner, uint64_t bytes, hipStream_t stream,
+                 uint64_t* held);
+void pool_free(int device, const void* owner, void* p, uint64_t held);
+// The bytes kept for an owner, and giving them back.
+uint64_t pool_cached(int device, const void* owner);
+void pool_release(int device, const void* owner);
 // hipMalloc; what the pool keeps is given back and the call repeated if it fails.
 hipError_t dev_malloc(int device, void** p, uint64_t bytes);
 lbvh_status set_device(lbvh_ctx* c);

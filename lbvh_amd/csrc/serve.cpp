@@ -285,13 +285,13 @@ destroy_scene(Scene* sc)
 bool
 make_room(lbvh_server* s, uint64_t need)
 {
-  const uint64_t trees = pool_cached(s->device);
+  const uint64_t trees = pool_cached(s->device, s); // what this server's trees left
   if (s->mem_used + s->dev_pool.cached + trees + need <= s->mem_cap)
     return true;
   // cached pool buffers go first, those kept of freed trees among them
   if (s->dev_pool.cached || trees) {
     s->dev_pool.release_all();
-    pool_release(s->device);
+    pool_release(s->device, s);
     if (s->mem_used + need <= s->mem_cap)
       return true;
   }
@@ -315,8 +315,8 @@ make_room(lbvh_server* s, uint64_t need)
     s->stats.evictions++;
   }
   // the evicted trees' memory stays kept for the next trees only under the cap
-  if (s->mem_used + pool_cached(s->device) + need > s->mem_cap)
-    pool_release(s->device);
+  if (s->mem_used + pool_cached(s->device, s) + need > s->mem_cap)
+    pool_release(s->device, s);
   return s->mem_used + need <= s->mem_cap;
 }
 
@@ -775,6 +775,7 @@ lbvh_server_create(int device, const lbvh_server_opts* opts, lbvh_server** out)
     }
     // a request's latency must not include tuning runs
     lbvh_ctx_set_autotune(c, 0);
+    c->pool_owner = s;
     s->lanes.push_back(c);
     if (o.reserve_prims >= 2) {
       // the power of two a build of reserve_prims would grow the lane to
@@ -835,6 +836,7 @@ lbvh_server_destroy(lbvh_server* s)
     destroy_scene(kv.second);
   for (auto& kv : s->reqs)
     delete kv.second;
+  pool_release(s->device, s);
   s->dev_pool.release_all();
   s->host_pool.release_all();
   for (auto* l : s->lanes)

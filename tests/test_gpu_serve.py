@@ -203,6 +203,25 @@ def test_server_charges_the_memory_that_reused_blocks_hold():
     srv.close()
 
 
+def test_server_leaves_what_other_contexts_keep(ctx):
+    """Memory that a plain context keeps of its freed trees is neither counted
+    under a server's cap nor given back by the server."""
+    rays = _rays(1, 64)
+    a = ctx.build_triangles(_scene(1, 701234), code_bits=63, leaf_order=1)
+    held = a.info().device_bytes  # more than the server's cap
+    a.destroy()
+    srv = lbvh_amd.Server(0, lanes=1, memory_cap_bytes=48 << 20)
+    for k in range(4):
+        srv.wait(srv.submit(rays, 0, _scene(k, 20000))[0])
+    st = srv.stats()
+    assert st["memory_cap_bytes"] < held
+    assert st["evictions"] == 0 and st["resident_scenes"] == 4
+    b = ctx.build_triangles(_scene(1, 701000), code_bits=63, leaf_order=1)
+    assert b.info().device_bytes == held, "the context's kept memory was given back"
+    b.destroy()
+    srv.close()
+
+
 def test_server_rejects_bad_requests():
     srv = lbvh_amd.Server(0)
     with pytest.raises(lbvh_amd.LbvhError):
