@@ -139,8 +139,10 @@ void dev_free(void* p);
 // than the build (hipFree of a 16M-primitive tree: 20 ms).  At most
 // kPoolMaxBytes and kPoolMaxBlocks are kept per device, the oldest given back
 // first; all of it when the device's last context goes, or when an
-// allocation of the engine fails.  pool_free waits for the device first, as
-// hipFree does, so a kept block has no user left on any stream; a block
+// allocation of the engine fails; a block of more than kPoolMaxBytes / 2 (a
+// tree of about 41M primitives) is never kept.  pool_free waits for the device
+// first, as hipFree does, so a kept block has no user left on any stream (and
+// like hipFree it may be called while streams are being captured); a block
 // carries no contents from one tree to the next.  A block is kept for its owner
 // (a server, or all other contexts of the device: nullptr), so that a server
 // counts and frees under its memory cap what its own trees left, no one else's.

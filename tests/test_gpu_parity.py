@@ -773,6 +773,52 @@ def test_tree_memory_reused_across_threads_and_contexts(leaf):
     assert not bad, bad
 
 
+@pytest.mark.parametrize("mode", [0, 1, 2], ids=["global", "thread-local", "relaxed"])
+@pytest.mark.parametrize("other_thread", [False, True], ids=["same-thread", "other-thread"])
+def test_captures_survive_frees_and_stream_waits(ctx, mode, other_thread):
+    """Destroying a tree and ordering a context after a stream leave a graph
+    capture valid, in any capture mode and from any thread."""
+    import ctypes
+    import threading
+    from lbvh_amd.hip import DeviceArray, check, hip
+    P = ctypes.c_void_p
+    L = hip()
+    trees = [ctx.build_triangles(W.scene_uniform(1, n, 0.01)[1]) for n in (3000, 70001)]
+    a, b = (DeviceArray.from_host(np.full(4096, v, np.uint32)) for v in (1, 2))
+    cap, idle, graph, run = P(), P(), P(), P()
+    for s in (cap, idle):
+        check(L.hipStreamCreateWithFlags(ctypes.byref(s), 1), "stream")
+
+    def copy():
+        return L.hipMemcpyAsync(P(b.ptr), P(a.ptr), ctypes.c_size_t(16384), 3, cap)
+
+    def disturb():
+        for t in trees:
+            t.destroy()
+        ctx._check(lbvh_amd.lib().lbvh_ctx_wait_stream(ctx.handle, idle))
+
+    print("capture mode=%d other_thread=%d" % (mode, other_thread), flush=True)
+    check(L.hipStreamBeginCapture(cap, mode), "begin")
+    rc = [copy()]
+    if other_thread:
+        t = threading.Thread(target=disturb)
+        t.start()
+        t.join()
+    else:
+        disturb()
+    rc.append(copy())
+    rc.append(L.hipStreamEndCapture(cap, ctypes.byref(graph)))
+    assert rc == [0, 0, 0]
+    check(L.hipGraphInstantiate(ctypes.byref(run), graph, None, None, ctypes.c_size_t(0)), "graph")
+    check(L.hipGraphLaunch(run, cap), "launch")
+    check(L.hipStreamSynchronize(cap), "sync")
+    assert (b.numpy() == 1).all()
+    check(L.hipGraphExecDestroy(run), "destroy")
+    check(L.hipGraphDestroy(graph), "destroy")
+    for s in (cap, idle):
+        check(L.hipStreamDestroy(s), "destroy")
+
+
 def test_reported_bytes_are_those_held():
     """device_bytes counts the whole block that a tree took from a freed one,
     and its host-built triangles'."""
