@@ -235,7 +235,12 @@ lbvh_status lbvh_bvh_download_nodes(lbvh_ctx* ctx, const lbvh_bvh* bvh,
 lbvh_status lbvh_bvh_download_codes(lbvh_ctx* ctx, const lbvh_bvh* bvh,
                                     void* codes, uint32_t* ids,
                                     float* bounds6);
+/* Waits for the device, as hipFree does.  Up to 4 GiB of freed trees' memory is
+ * kept per device for the next trees, until its last context goes. */
 void lbvh_bvh_destroy(lbvh_bvh* bvh);
+/* Gives back what is kept of freed trees on a device, for other allocators of
+ * the process.  Safe from any thread. */
+lbvh_status lbvh_trim_memory(int device);
 
 /* -- builder<double> --------------------------------------------------------
  * Replaces lbvh::builder<double>::operator()(primitives, count, converter)

@@ -154,6 +154,7 @@ SIGNATURES = {
     "lbvh_bvh_download_nodes": (ctypes.c_int, [VP, VP, VP, U64]),
     "lbvh_bvh_download_codes": (ctypes.c_int, [VP, VP, VP, VP, VP]),
     "lbvh_bvh_destroy": (None, [VP]),
+    "lbvh_trim_memory": (ctypes.c_int, [ctypes.c_int]),
     "lbvh_trace_closest": (ctypes.c_int, [VP, VP, VP, U64, ctypes.c_int, VP, VP, VP]),
     "lbvh_trace_closest_device": (ctypes.c_int, [VP, VP, VP, U64, ctypes.c_int, VP, VP, VP]),
     "lbvh_build_batch": (ctypes.c_int, [VP, VP, VP, ctypes.c_uint32, ctypes.POINTER(BuildOpts),
@@ -245,6 +246,14 @@ def _is_device(x):
             raise ValueError("device arrays must be contiguous")
         return True
     return False
+
+
+def trim_memory(device=0):
+    """Gives back the device memory that the engine keeps of freed trees (up to
+    4 GiB) for the next ones."""
+    st = lib().lbvh_trim_memory(device)
+    if st != 0:
+        raise LbvhError(st, "lbvh_trim_memory")
 
 
 def _torch_streams(arrays):

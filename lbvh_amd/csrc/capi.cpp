@@ -851,6 +851,22 @@ lbvh_ctx_create(int device, lbvh_ctx** out)
   return LBVH_OK;
 }
 
+lbvh_status
+lbvh_trim_memory(int device)
+{
+  int count = 0;
+  if (hipGetDeviceCount(&count) != hipSuccess || count <= 0) {
+    (void)hipGetLastError();
+    return LBVH_E_NODEVICE;
+  }
+  if (device < 0 || device >= count)
+    return LBVH_E_INVALID;
+  RelaxedCapture relaxed;
+  if (pooled(device))
+    pool_trim(device, 0, 0);
+  return LBVH_OK;
+}
+
 void
 lbvh_ctx_destroy(lbvh_ctx* c)
 {

@@ -773,6 +773,22 @@ def test_tree_memory_reused_across_threads_and_contexts(leaf):
     assert not bad, bad
 
 
+def test_trim_gives_kept_memory_back(ctx):
+    """A freed tree's memory stays with the engine until it is trimmed."""
+    from lbvh_amd import hip
+    lbvh_amd.trim_memory()
+    before = hip.mem_info()[0]
+    tree = ctx.build_triangles(W.make_triangles(W.uniform_vertices(1, 1500000, 0.01)))
+    held = tree.info().device_bytes
+    tree.destroy()
+    kept = hip.mem_info()[0]
+    lbvh_amd.trim_memory()
+    assert hip.mem_info()[0] - kept >= held
+    assert kept <= before - held
+    with pytest.raises(lbvh_amd.LbvhError):
+        lbvh_amd.trim_memory(-1)
+
+
 @pytest.mark.parametrize("mode", [0, 1, 2], ids=["global", "thread-local", "relaxed"])
 @pytest.mark.parametrize("other_thread", [False, True], ids=["same-thread", "other-thread"])
 def test_captures_survive_frees_and_stream_waits(ctx, mode, other_thread):
