@@ -92,7 +92,8 @@ typedef struct lbvh_bvh_info
   uint32_t sort_digit_bits; /* the sort configuration the build used */
   uint32_t sort_tile;
   uint32_t sort_strategy;   /* 1 onesweep, 2 reduce-then-scan, 3 hybrid */
-  uint32_t sort_global_digits; /* hybrid: top digits sorted by global passes */
+  uint32_t sort_global_digits; /* hybrid: top digits sorted by global passes (0: in
+                                  LDS chunks, builds below 65,536 primitives) */
 } lbvh_bvh_info;
 
 /* One configuration timed by the context's autotuner: the sort of a build

@@ -880,8 +880,9 @@ constexpr uint32_t kCountRankBudget = 64;
 // (cx, cy, cz of n each) and the partial bounds of k_centroid_bounds, encoding
 // them (as k_encode).  kTileTriangles / kTileBoxes: all n from the primitives
 // themselves -- centres and their bounds, codes, sort.  A build of
-// so few is bound by its launches: this one takes the place of thirteen, and
-// a build of 4,096 triangles goes from 110 to 50 us of kernels.
+// so few is bound by its launches: this one takes the place of thirteen (30-bit
+// codes by reduce-then-scan), and a build of 4,096 triangles goes from 110 to
+// 50 us of kernels.
 constexpr int kTileBuckets = 0, kTileKeys = 1, kTileCentres = 2, kTileTriangles = 3,
               kTileBoxes = 4;
 

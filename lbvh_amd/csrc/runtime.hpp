@@ -178,7 +178,7 @@ lbvh_status sync_and_check(lbvh_ctx* c);
 SortConfig default_sort();
 // The sort a single build uses without tuning (tuner off, or before a
 // bucket is tuned): the hybrid, with fewer global digits for fewer keys (none
-// for what one workgroup sorts).
+// below kTuneMinPrims).
 SortConfig untuned_sort(int key_bits, uint64_t n);
 // Grows a context's workspace to what a build of n primitives with this
 // code width and sort configuration needs.

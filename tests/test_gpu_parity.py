@@ -131,7 +131,7 @@ def test_build_matches_oracle_ragged(ctx, n, bits, leaf):
 @pytest.mark.parametrize("dist", ["uniform", "clustered", "equal", "two"])
 def test_small_builds_match_oracle(ctx, n, dist):
     """Builds below 65,536 primitives sort in one workgroup (up to 4,096) or
-    with one global digit: wave and block remainders, runs of a few dense
+    in chunks that are merged: wave and block remainders, runs of a few dense
     spots, one code for everything, two far groups; triangles and boxes, both
     code widths and leaf orders."""
     rng = np.random.default_rng(n)
